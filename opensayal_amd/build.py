@@ -31,8 +31,9 @@ SOURCES = [
     "fluid_host.cpp",
     "batch_host.cpp",
     "kernels_step.hip",
-    "kernels_project.hip",
-    "kernels_batch.hip",
+    # one object per storage type, so that they build at once
+    *[f"kernels_batch.hip:{t}" for t in range(3)],
+    *[f"kernels_project.hip:{t}" for t in range(3)],
     "kernels_view.hip",
     "noalloc.hip",
     "arith_check.hip",
@@ -66,12 +67,14 @@ def _up_to_date(src: Path, out: Path) -> bool:
 
 
 def _compile(src: str, incremental: bool = False) -> Path:
-    out = OBJ / (Path(src).stem + ".o")
+    src, _, storage = src.partition(":")
+    only = [f"-DOSY_ONLY_STORAGE={storage}"] if storage else []
+    out = OBJ / (Path(src).stem + storage + ".o")
     path = CSRC / src
     if incremental and _up_to_date(path, out):
         return out
     if src.endswith(".hip"):
-        cmd = [HIPCC, *COMMON, *DEVICE, "-x", "hip", "-c", str(path), "-o", str(out)]
+        cmd = [HIPCC, *COMMON, *DEVICE, *only, "-x", "hip", "-c", str(path), "-o", str(out)]
     else:
         cmd = [HIPCC, *COMMON, "-c", str(path), "-o", str(out)]
     res = subprocess.run(cmd, capture_output=True, text=True)

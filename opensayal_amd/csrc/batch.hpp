@@ -29,7 +29,6 @@ enum BatchStageKind : int {
 // Tile of the forces and advection stages in a batch: 64 x 64 cells, one
 // row group per wavefront.
 constexpr int kBatchAdvTX = 64, kBatchAdvTY = 64;
-constexpr int kBatchThreads = 64 * kRegWaves;  // 512
 
 // Per simulation: parameters, buffers, and the buffer parity rule.  At launch
 // number e after the last rebuild, u and v sit in buffer uv0 ^ (e & flip_uv
@@ -55,7 +54,7 @@ struct BatchStage {
   int smoke;   // BK_FORCES: smoke part
   int dep;     // stage that must be complete first, -1 for none
   int dep_tiles;
-  int ntx;     // tiles per row of this stage's tiling
+  int ntx, nty;  // tiles per row and column of this stage's tiling
   int tile_dep;  // 1: wait only for the item's own list of predecessor tiles
 };
 

@@ -122,11 +122,14 @@ int rebuild(osy_batch* b) {
   // that fill the GPU alone step on their own graphs instead
   for (size_t m = 0; m < b->members.size(); m++) {
     osy_fluid* fl = b->members[m];
-    if (b->per_grid_cells > 0 && (int64_t)fl->W * fl->H >= b->per_grid_cells) {
+    const bool pressure = fl->cfg.enable_pressure != 0;
+    // (so do the rare members whose pressure sums need a division, which
+    // the persistent kernel leaves out: d_t = 0 or |d_t| >= 2)
+    if ((b->per_grid_cells > 0 && (int64_t)fl->W * fl->H >= b->per_grid_cells) ||
+        (pressure && fl->params(fl->cfg.d_t, nullptr).pdt_recip == 0.0)) {
       b->solo.push_back(fl);
       continue;
     }
-    const bool pressure = fl->cfg.enable_pressure != 0;
     auto it = std::find_if(b->groups.begin(), b->groups.end(), [&](const osy_batch::Group& g) {
       return g.storage == fl->storage && g.pressure == pressure;
     });
@@ -196,6 +199,7 @@ int rebuild(osy_batch* b) {
         st.dep = prev[si];
         st.dep_tiles = prev_tiles[si];
         st.ntx = p.ntx;
+        st.nty = p.ntiles / p.ntx;
         // a projection launch after a projection or forces stage waits only
         // for the predecessor tiles within 2k of its owned tile: those wrote
         // what its region reads, or read what its tile writes (the pressure

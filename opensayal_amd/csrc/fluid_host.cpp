@@ -88,8 +88,7 @@ BlockLayout block_layout(int W, int H, int storage) {
   L.flg = align_up(cells, 256);
   L.red = align_up(sizeof(float) * (2 * kReduceBlocks + 2), 256);
   L.dred = align_up(sizeof(double) * (2 * kReduceBlocks + 2), 256);
-  // resident projection: flag words, finished count, error word
-  L.rsd = align_up(sizeof(unsigned) * (kResidentMaxTiles + 2), 256);
+  L.rsd = 256;  // resident projection: error word
   return L;
 }
 
@@ -137,6 +136,8 @@ int create_impl(const osy_config* cfg, osy_fluid** out) {
   const size_t fld = L.fld, f32 = L.f32, ref = L.ref, flg = L.flg, red = L.red, dred = L.dred;
   int khz = 0;
   e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, fl->device);
+  if (e == hipSuccess)
+    e = hipDeviceGetAttribute(&fl->cus, hipDeviceAttributeMultiprocessorCount, fl->device);
   if (e != hipSuccess) {
     delete fl;
     return set_error(OSY_E_HIP, std::string("device attribute: ") + hipGetErrorString(e));
@@ -164,8 +165,7 @@ int create_impl(const osy_config* cfg, osy_fluid** out) {
   fl->f.scratch = (float*)b; b += red;
   fl->f.dscratch = (double*)b; b += dred;
   fl->f.prange = fl->f.scratch + 2 * kReduceBlocks;
-  fl->f.rflags = (unsigned*)b;
-  fl->f.error = (int*)(fl->f.rflags + kResidentMaxTiles + 1);
+  fl->f.error = (int*)b;
   b += L.rsd;
 
   e = init_projection_kernels();
@@ -240,6 +240,18 @@ int enqueue_graph_steps(osy_fluid* fl, int32_t steps, float d_t, hipStream_t s) 
   return OSY_OK;
 }
 
+// Makes `t` the handle's projection shape (its graphs are gone and its
+// stream is idle).  The rings of another shape lie elsewhere, so the
+// resident projection starts from a clean exchange buffer.
+int adopt_tuning(osy_fluid* fl, const ProjTuning& t) {
+  if (t.kernel == PROJ_RESIDENT) {
+    if (int st = fluid_clean_exchange(fl, t)) return st;
+    OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+  }
+  fl->tuning = t;
+  return OSY_OK;
+}
+
 int field_elem_ok(int field) { return field >= OSY_FIELD_VEL_X && field <= OSY_FIELD_TOTAL_S; }
 
 }  // namespace
@@ -257,10 +269,32 @@ namespace osy {
 bool tuning_fits(const osy_fluid* fl, const ProjTuning& t) {
   if (!t.valid(fl->cfg.enable_pressure != 0)) return false;
   if (t.kernel != PROJ_RESIDENT) return true;
-  const int tiles = t.tiles(fl->W, fl->H);
-  int slots = 0;
-  if (resident_capacity(t.reg_rows(), &slots) != hipSuccess) return false;
-  return tiles <= kResidentMaxTiles && tiles <= slots;
+  return t.tiles(fl->W, fl->H) <= resident_slots(t.reg_rows(), fl->cus);
+}
+
+int fluid_clean_exchange(osy_fluid* fl, const ProjTuning& shape) {
+  ProjTuning t;
+  if (!shape.resident_plan(fl->W, fl->H, fl->cus, &t)) return OSY_OK;
+  const size_t bytes =
+      256 + 3 * 8 * t.exchange_words(fl->W, fl->H, (size_t)fl->elem);
+  if (fl->exchange_bytes < bytes) {
+    OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+    if (fl->exchange) OSY_HIP_CHECK(hipFree(fl->exchange));
+    fl->exchange = nullptr;
+    fl->exchange_bytes = 0;
+    hipError_t e = hipMalloc(&fl->exchange, bytes);
+    if (e != hipSuccess) {
+      fl->exchange = nullptr;
+      return set_error(OSY_E_NOMEM, "halo exchange of " + std::to_string(bytes) +
+                                        " bytes: " + hipGetErrorString(e));
+    }
+    fl->exchange_bytes = bytes;
+    fl->f.rstate = (unsigned*)fl->exchange;
+    fl->f.exchange = (char*)fl->exchange + 256;
+  }
+  OSY_HIP_CHECK(hipMemsetAsync(fl->exchange, 0, 256, fl->stream));
+  OSY_HIP_CHECK(hipMemsetAsync(fl->f.exchange, 0xFF, fl->exchange_bytes - 256, fl->stream));
+  return OSY_OK;
 }
 
 int fluid_check_error(osy_fluid* fl) {
@@ -271,6 +305,10 @@ int fluid_check_error(osy_fluid* fl) {
   if (err) {
     const int zero = 0;
     OSY_HIP_CHECK(hipMemcpy(fl->f.error, &zero, sizeof(int), hipMemcpyHostToDevice));
+    // rings may be left half read
+    if (fl->tuning.kernel == PROJ_RESIDENT)
+      if (int st = fluid_clean_exchange(fl, fl->tuning)) return st;
+    OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
     return set_error(OSY_E_STATE,
                      "projection: a neighbour wait of the resident kernel timed out; the "
                      "fields are invalid");
@@ -506,14 +544,12 @@ int osy_fluid_set_tuning(osy_fluid* fl, const osy_tuning* t) {
     pt.kernel = PROJ_COLOUR;
   } else if (pt.kernel == PROJ_RESIDENT && pt.valid(fl->cfg.enable_pressure != 0) &&
              !tuning_fits(fl, pt)) {
-    int slots = 0;
-    const hipError_t e = resident_capacity(pt.reg_rows(), &slots);
     return set_error(OSY_E_INVALID,
                      "resident projection: " + std::to_string(pt.tiles(fl->W, fl->H)) +
                          " tiles do not all fit on the device at once (" +
-                         std::to_string(slots) + " workgroup slots at " +
-                         std::to_string(pt.reg_rows()) + " rows per wavefront; " +
-                         hipGetErrorString(e) + ")");
+                         std::to_string(resident_slots(pt.reg_rows(), fl->cus)) +
+                         " workgroup slots at " + std::to_string(pt.reg_rows()) +
+                         " rows per wavefront)");
   } else if (!pt.valid(fl->cfg.enable_pressure != 0)) {
     return set_error(OSY_E_INVALID,
                      "tiled projection needs 1 <= k <= 64, an even tile width >= 2, a tile "
@@ -530,8 +566,7 @@ int osy_fluid_set_tuning(osy_fluid* fl, const osy_tuning* t) {
         OSY_HIP_CHECK(hipGraphExecDestroy(g.exec));
         g.exec = nullptr;
       }
-  fl->tuning = pt;
-  return OSY_OK;
+  return adopt_tuning(fl, pt);
 }
 
 int osy_fluid_set_wait_limit(osy_fluid* fl, int64_t microseconds) {
@@ -570,9 +605,9 @@ TuneKey tune_key(const osy_fluid* fl) {
 }
 
 // Every launch shape the autotuner times: the colour-phase kernel, the
-// register-resident kernels (several launches, and one resident launch when
-// the tiles fit) at 4, 8, 10, 12 and 16 rows per wavefront and 1..12 sweeps
-// per launch or stage, and a few LDS-tiled shapes.
+// register-resident kernels at regions of 32, 64, 80, 96 and 128 rows and
+// 1..12 sweeps per launch or stage (several launches, and one resident launch
+// at 32 and 96 rows when the tiles fit), and a few LDS-tiled shapes.
 std::vector<ProjTuning> tuning_candidates(bool pressure) {
   std::vector<ProjTuning> out;
   ProjTuning c;
@@ -586,6 +621,9 @@ std::vector<ProjTuning> tuning_candidates(bool pressure) {
         r.k = k;
         r.tw = 128 - 4 * k;
         r.th = kRegWaves * rows - 4 * k;
+        // (64 to 128 rows run the same resident kernel; with pressure sums
+        // only up to 64 are valid)
+        if (kern == PROJ_RESIDENT && rows != 4 && rows != (pressure ? 8 : 12)) continue;
         if (r.valid(pressure)) out.push_back(r);
       }
     }
@@ -672,6 +710,8 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
     for (const ProjTuning& cand : tuning_candidates(pressure)) {
       if (e != hipSuccess) break;
       if (!tuning_fits(fl, cand)) continue;
+      if (cand.kernel == PROJ_RESIDENT)
+        if (fluid_clean_exchange(fl, cand) != OSY_OK) continue;  // no memory for it
       float t_min = 1e30f;
       for (int rep = 0; rep < 3 && e == hipSuccess; rep++) {  // rep 0 warms up
         e = restore(fl->stream);
@@ -707,7 +747,8 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
     if (e != hipSuccess) return set_error(OSY_E_HIP, std::string("autotune: ") + hipGetErrorString(e));
     int st = drop_graphs(fl);
     if (st != OSY_OK) return st;
-    fl->tuning = best;
+    st = adopt_tuning(fl, best);
+    if (st != OSY_OK) return st;
     std::lock_guard<std::mutex> lock(g_tune_mu);
     g_tune_cache[tune_key(fl)] = best;
   }
@@ -730,8 +771,8 @@ int osy_fluid_autotune_cached(osy_fluid* fl) {
   }
   OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
   int st = drop_graphs(fl);
+  if (st == OSY_OK) st = adopt_tuning(fl, t);
   if (st != OSY_OK) return st;
-  fl->tuning = t;
   return 1;
 }
 

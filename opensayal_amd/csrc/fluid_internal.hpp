@@ -34,8 +34,11 @@ struct osy_fluid {
   float* staging = nullptr;  // W*H*4 bytes, reference-order copies
   void* trace_buf = nullptr;  // path-line output, grown on demand
   size_t trace_cap = 0;
+  void* exchange = nullptr;   // resident projection's halo exchange, made when
+  size_t exchange_bytes = 0;  // that shape is first chosen (fluid_clean_exchange)
   ProjTuning tuning;  // projection kernel shape, chosen at create
   long long spin_ticks = 0;  // bound of a resident projection's neighbour wait
+  int cus = 0;               // CUs of the device
   int wall_khz = 100000;     // the device's wall-clock rate
   bool resident_pending = false;  // a resident projection ran since the last
                                   // read of the error word
@@ -52,6 +55,7 @@ struct osy_fluid {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
     if (block) (void)hipFree(block);
     if (trace_buf) (void)hipFree(trace_buf);
+    if (exchange) (void)hipFree(exchange);
     if (stream) (void)hipStreamDestroy(stream);
   }
 
@@ -101,6 +105,7 @@ struct osy_fluid {
     sp.visc_den = 1.0f + 4.0f * sp.visc_a;
     sp.pdt_recip = (d_t != 0.0f && std::fabs(d_t) < 2.0f) ? 1.0 / (double)d_t : 0.0;
     sp.spin_ticks = spin_ticks;
+    sp.cus = cus;
     return sp;
   }
 };
@@ -118,6 +123,10 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t);
 // osy_fluid_autotune without the batch-membership check: the batch
 // autotuner tunes the projection of members that step on their own graphs.
 int fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms);
+
+// Makes the handle's halo exchange buffer large enough for projection shape
+// t and fills it with empty words on the handle's stream.
+int fluid_clean_exchange(osy_fluid* fl, const ProjTuning& t);
 
 // Reads and clears the device error word (a resident projection whose
 // neighbour wait timed out) when a resident projection ran since the last

@@ -49,6 +49,7 @@ struct StepParams {
   double pdt_recip;
   // bound of one neighbour wait of the resident projection (wall-clock ticks)
   long long spin_ticks;
+  int cus;  // CUs of the device
 };
 
 // Device buffers of one simulation; T is the storage type of u, v, smoke.
@@ -62,8 +63,8 @@ struct FieldPtrs {
   float* scratch;   // reductions: partial results
   float* prange;    // [min, max] of pressure
   double* dscratch; // divergence reduction partials
-  unsigned* rflags; // resident projection: stages each tile has published,
-                    // then the count of finished workgroups (kResidentMaxTiles + 1)
+  void* exchange;   // resident projection: halo exchange slots (null until needed)
+  unsigned* rstate; // resident projection: finished workgroups, slot of ring 0
   int* error;       // set by a resident projection whose neighbour wait timed out
 };
 
@@ -75,16 +76,15 @@ enum ProjectionKernel : int {
   PROJ_RESIDENT = 3,  // register-resident tiles kept for all n sweeps, one launch
 };
 
-// Tiles a resident projection may have (its flag words); a shape also needs
-// every tile's workgroup resident on the GPU at once.
-constexpr int kResidentMaxTiles = 4096;
-
-// Register-resident kernel: 8 wavefronts stacked vertically, each holding
-// 128 cells x kRegRows rows in VGPRs; the region is 128 x 8*kRegRows cells.
+// Register-resident kernels: a region of 128 x 8*rows cells held in VGPRs,
+// by 8 wavefronts of `rows` rows each up to 10 rows (two workgroups per CU),
+// by 16 of rows / 2 above (one): four wavefronts per SIMD either way, and
+// more at 4 rows.
 constexpr int kRegWaves = 8;
 inline bool reg_rows_supported(int rows) {
   return rows == 4 || rows == 8 || rows == 10 || rows == 12 || rows == 16;
 }
+inline int reg_waves(int rows) { return rows > 10 ? 2 * kRegWaves : kRegWaves; }
 
 // Workgroup of the tiled kernel: 8 wavefronts of 64 lanes.
 constexpr int kTileWaves = 8;
@@ -114,7 +114,7 @@ struct ProjTuning {
     const size_t flag_bytes = (size_t)(region_h() + 1) * (region_w() + 1);
     return cells * 4 * (pressure ? 3 : 2) + cells + flag_bytes;
   }
-  // PROJ_REGS: rows each wavefront holds
+  // PROJ_REGS, PROJ_RESIDENT: region rows / 8
   int reg_rows() const { return (th + 4 * k) / kRegWaves; }
   bool valid(bool pressure) const {
     if (kernel == PROJ_COLOUR) return true;
@@ -134,12 +134,45 @@ struct ProjTuning {
     if (kernel == PROJ_RESIDENT) return sweeps > 0 ? 1 : 0;
     return kernel == PROJ_COLOUR ? 2 * sweeps : (sweeps + k - 1) / k;
   }
-  // register kernels: tiles over a W x H grid
-  int tiles(int W, int H) const { return ((W + tw - 1) / tw) * ((H + th - 1) / th); }
+  // register kernels: tiles over a W x H grid (the first and last of a row
+  // or column own 2k cells more, RegPlace)
+  int tiles_x(int W) const { return W <= 4 * k + tw ? 1 : (W - 4 * k + tw - 1) / tw; }
+  int tiles_y(int H) const { return H <= 4 * k + th ? 1 : (H - 4 * k + th - 1) / th; }
+  int tiles(int W, int H) const { return tiles_x(W) * tiles_y(H); }
+  // What a resident projection of this shape runs on a device of `cus` CUs.
+  // Every tile's workgroup must be on the GPU at once, and the fewer, larger
+  // workgroups a CU holds, the less it computes and exchanges in its halos:
+  // regions of 64 rows and more run as one of 96 (16 wavefronts of 6 rows, a
+  // CU's registers; 50 sweeps of 1920 x 1080 at k = 5 take 120 us, in
+  // regions of 64 rows, two per CU, 233 us).  False when those do not fit
+  // either: then each stage is a launch of this shape's register kernel,
+  // the same tiles and results.
+  bool resident_plan(int W, int H, int cus, ProjTuning* run) const {
+    *run = *this;
+    if (reg_rows() > 4) run->th = kRegWaves * 12 - 4 * k;
+    return run->th >= 2 * k && run->tiles(W, H) <= (reg_rows() == 4 ? 3 : 1) * cus;
+  }
+  // resident kernel: 8-byte words of one of its three exchange slots (every
+  // tile's region, two words per cell pair in binary32, one in 16 bits)
+  size_t exchange_words(int W, int H, size_t elem) const {
+    return (size_t)tiles(W, H) * region_h() * 64 * (elem / 2);
+  }
 };
 
 // Number of float slots `scratch` must hold, and doubles for `dscratch`.
 constexpr int kReduceBlocks = 512;
+
+// Tiles that a resident shape may be asked to have: as many as workgroups of
+// its register kernel fit the device, from the launch bounds (which the
+// compiler meets): 8 wavefronts within 80 VGPRs at 4 rows (6 per SIMD: 3
+// workgroups per CU) and 128 at 8 and 10 rows (4: 2 workgroups); 16
+// wavefronts above (1).  LDS (12 KiB per 8 wavefronts) and the wavefront
+// slots allow more.  (The runtime's occupancy query was not used: it has
+// returned 0 for a kernel that fits, depending on what ran before.)
+inline int resident_slots(int rows, int cus) { return (rows == 4 ? 3 : rows <= 10 ? 2 : 1) * cus; }
+
+// Lets the projection kernels use all of the LDS on the current device.
+hipError_t init_projection_kernels();
 
 // Cell flags, then the projection gate bytes derived from them.
 void launch_build_flags(const MaskParams& m, uint8_t* flags, uint8_t* gates, hipStream_t s);

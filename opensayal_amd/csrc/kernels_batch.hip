@@ -23,8 +23,9 @@ namespace {
 
 static_assert(kBatchAdvTX == kAdvTX, "advection tile width");
 
+template <int NW>
 union BatchShared {
-  RegShared reg;
+  RegShared<NW> reg;
   AdvShared<kBatchAdvTY> adv;
 };
 
@@ -80,9 +81,9 @@ __device__ inline bool wait_tiles(const unsigned long long* tdone, const unsigne
   return true;
 }
 
-template <typename T, bool PRESSURE, int R>
+template <typename T, bool PRESSURE, int R, int NW>
 __device__ __attribute__((always_inline)) inline void run_item(const BatchStage& st, const BatchSim& sim, int tile,
-                                unsigned epoch_bit, int tw, int th, int k, BatchShared& sh) {
+                                unsigned epoch_bit, int tw, int th, int k, BatchShared<NW>& sh) {
   const StepParams& sp = sim.sp;
   const int uv = sim.uv0 ^ (int)(epoch_bit & (unsigned)sim.flip_uv);
   const int sm = sim.sm0 ^ (int)(epoch_bit & (unsigned)sim.flip_sm);
@@ -94,28 +95,30 @@ __device__ __attribute__((always_inline)) inline void run_item(const BatchStage&
     a.th = th;
     a.k = k;
     a.ntx = st.ntx;
+    a.nty = st.nty;
+    a.inset = 2 * k;
     a.sweeps = st.sweeps;
     a.forces = st.forces;
     const int in = uv ^ (st.q & 1);
-    project_regs_tile<T, PRESSURE, R, true>(sp, sim.gates, (const T*)sim.u[in], (const T*)sim.v[in],
-                                      (T*)sim.u[in ^ 1], (T*)sim.v[in ^ 1], sim.p, a, tile,
-                                      sh.reg);
+    project_regs_tile<T, PRESSURE ? PM_RECIP : PM_NONE, R, NW>(sp, sim.gates, (const T*)sim.u[in],
+                                                 (const T*)sim.v[in], (T*)sim.u[in ^ 1],
+                                                 (T*)sim.v[in ^ 1], sim.p, a, tile, sh.reg);
     return;
   }
   const int bx = tile % st.ntx, by = tile / st.ntx;
   if (kind == BK_FORCES) {
-    forces_tile<T, kBatchAdvTY, kRegWaves>(sp, st.forces, st.smoke, (T*)sim.u[uv], (T*)sim.v[uv],
+    forces_tile<T, kBatchAdvTY, NW>(sp, st.forces, st.smoke, (T*)sim.u[uv], (T*)sim.v[uv],
                                            (T*)sim.smoke[sm], sim.p, bx, by);
     return;
   }
   if (kind == BK_ADV_UV) {
     const int in = uv ^ (st.q & 1);
     if (sp.cs == 1)
-      advect_velocity_tile<T, true, kBatchAdvTY, kRegWaves>(
+      advect_velocity_tile<T, true, kBatchAdvTY, NW>(
           sp, g, (const T*)sim.u[in], (const T*)sim.v[in], (T*)sim.u[in ^ 1], (T*)sim.v[in ^ 1],
           bx, by, sh.adv);
     else
-      advect_velocity_tile<T, false, kBatchAdvTY, kRegWaves>(
+      advect_velocity_tile<T, false, kBatchAdvTY, NW>(
           sp, g, (const T*)sim.u[in], (const T*)sim.v[in], (T*)sim.u[in ^ 1], (T*)sim.v[in ^ 1],
           bx, by, sh.adv);
     return;
@@ -123,11 +126,11 @@ __device__ __attribute__((always_inline)) inline void run_item(const BatchStage&
   // BK_ADV_SMOKE: the velocities after this step's advection
   const int cur = uv ^ ((st.q + 1) & 1);
   if (sp.cs == 1)
-    advect_smoke_tile<T, true, kBatchAdvTY, kRegWaves>(
+    advect_smoke_tile<T, true, kBatchAdvTY, NW>(
         sp, g, (const T*)sim.u[cur], (const T*)sim.v[cur], (const T*)sim.smoke[sm],
         (T*)sim.smoke[sm ^ 1], bx, by, sh.adv);
   else
-    advect_smoke_tile<T, false, kBatchAdvTY, kRegWaves>(
+    advect_smoke_tile<T, false, kBatchAdvTY, NW>(
         sp, g, (const T*)sim.u[cur], (const T*)sim.v[cur], (const T*)sim.smoke[sm],
         (T*)sim.smoke[sm ^ 1], bx, by, sh.adv);
 }
@@ -137,11 +140,12 @@ __device__ __attribute__((always_inline)) inline void run_item(const BatchStage&
 // completion count of the current one.  (Two thread-0 regions adjacent across
 // the loop's back-edge let the compiler merge them and move a barrier into a
 // loop that thread 0 leaves, which deadlocks the other threads.)
-// OCC2: registers capped for two workgroups per CU (at the price of some
-// spilling for R = 8); the batch autotuner decides whether that pays.
-template <typename T, bool PRESSURE, int R, bool OCC2>
-__global__ void __launch_bounds__(kBatchThreads, OCC2 ? 4 : 1) k_batch_step(BatchArgs A) {
-  __shared__ BatchShared sh;
+// A region of 8 wavefronts of 8 rows (rows 8) or 16 of 6 (rows 12).  OCC2:
+// registers capped at 128, for sixteen wavefronts per CU (two workgroups of
+// eight, or one of sixteen); the batch autotuner decides whether that pays.
+template <typename T, bool PRESSURE, int R, int NW, bool OCC2>
+__global__ void __launch_bounds__(64 * NW, OCC2 ? 4 : 1) k_batch_step(BatchArgs A) {
+  __shared__ BatchShared<NW> sh;
   __shared__ unsigned long long s_claim;
   __shared__ int s_ok;
   const unsigned long long per = (unsigned long long)A.nitems + (unsigned long long)A.grid;
@@ -178,7 +182,7 @@ __global__ void __launch_bounds__(kBatchThreads, OCC2 ? 4 : 1) k_batch_step(Batc
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_ok)) {
       const int simi = __builtin_amdgcn_readfirstlane(st.sim);
-      run_item<T, PRESSURE, R>(st, A.sims[simi], tile, (unsigned)(epoch & 1ULL), A.tw, A.th, A.k,
+      run_item<T, PRESSURE, R, NW>(st, A.sims[simi], tile, (unsigned)(epoch & 1ULL), A.tw, A.th, A.k,
                                sh);
     }
     // every wavefront's stores have reached the L2 before the barrier; thread
@@ -204,23 +208,38 @@ __global__ void __launch_bounds__(kBatchThreads, OCC2 ? 4 : 1) k_batch_step(Batc
 }
 
 template <typename T, bool PRESSURE>
-const void* batch_kernel(int rows, int occupancy) {
-  if (rows == 12) return (const void*)k_batch_step<T, PRESSURE, 12, true>;
-  return occupancy == 2 ? (const void*)k_batch_step<T, PRESSURE, 8, true>
-                        : (const void*)k_batch_step<T, PRESSURE, 8, false>;
+const void* kernel_of(int rows, int occupancy) {
+  if (rows == 12) return (const void*)k_batch_step<T, PRESSURE, 6, 16, true>;
+  return occupancy == 2 ? (const void*)k_batch_step<T, PRESSURE, 8, 8, true>
+                        : (const void*)k_batch_step<T, PRESSURE, 8, 8, false>;
 }
+
+}  // namespace
+
+template <typename T>
+const void* batch_kernel(bool pressure, int rows, int occupancy) {
+  return pressure ? kernel_of<T, true>(rows, occupancy) : kernel_of<T, false>(rows, occupancy);
+}
+
+// one storage type per object (OSY_ONLY_STORAGE), so that they build at once
+#if !defined(OSY_ONLY_STORAGE) || OSY_ONLY_STORAGE == 0
+template const void* batch_kernel<float>(bool, int, int);
+#endif
+#if !defined(OSY_ONLY_STORAGE) || OSY_ONLY_STORAGE == 1
+template const void* batch_kernel<__half>(bool, int, int);
+#endif
+#if !defined(OSY_ONLY_STORAGE) || OSY_ONLY_STORAGE == 2
+template const void* batch_kernel<__hip_bfloat16>(bool, int, int);
+#endif
+
+#if !defined(OSY_ONLY_STORAGE) || OSY_ONLY_STORAGE == 0
+namespace {
 
 const void* batch_kernel_for(int storage, bool pressure, int rows, int occupancy) {
   switch (storage) {
-    case OSY_STORAGE_F16:
-      return pressure ? batch_kernel<__half, true>(rows, occupancy)
-                      : batch_kernel<__half, false>(rows, occupancy);
-    case OSY_STORAGE_BF16:
-      return pressure ? batch_kernel<__hip_bfloat16, true>(rows, occupancy)
-                      : batch_kernel<__hip_bfloat16, false>(rows, occupancy);
-    default:
-      return pressure ? batch_kernel<float, true>(rows, occupancy)
-                      : batch_kernel<float, false>(rows, occupancy);
+    case OSY_STORAGE_F16: return batch_kernel<__half>(pressure, rows, occupancy);
+    case OSY_STORAGE_BF16: return batch_kernel<__hip_bfloat16>(pressure, rows, occupancy);
+    default: return batch_kernel<float>(pressure, rows, occupancy);
   }
 }
 
@@ -232,7 +251,7 @@ hipError_t batch_grid_size(int storage, bool pressure, int rows, int occupancy, 
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e == hipSuccess)
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, batch_kernel_for(storage, pressure, rows, occupancy), kBatchThreads, 0);
+        &per_cu, batch_kernel_for(storage, pressure, rows, occupancy), 64 * reg_waves(rows), 0);
   if (e != hipSuccess) return e;
   *grid = (per_cu < 1 ? 1 : per_cu) * (cus < 1 ? 1 : cus);
   return hipSuccess;
@@ -242,7 +261,9 @@ void enqueue_batch_step(int storage, bool pressure, int rows, int occupancy, con
                         hipStream_t s) {
   const void* fn = batch_kernel_for(storage, pressure, rows, occupancy);
   void* args[] = {(void*)&a};
-  (void)hipLaunchKernel(fn, dim3(a.grid), dim3(kBatchThreads), args, 0, s);
+  (void)hipLaunchKernel(fn, dim3(a.grid), dim3(64 * reg_waves(rows)), args, 0, s);
 }
+
+#endif
 
 }  // namespace osy

@@ -245,18 +245,19 @@ __global__ void __launch_bounds__(kTileThreads)
   }
 }
 
-// 8 and 10 rows per wavefront are held within 128 VGPRs, so two workgroups
-// share a CU (8 rows with pressure sums spill a few values outside the
-// sweep loop, which beats one workgroup per CU); 4 rows within 80, so three
-// share one (the others take what the compiler allocates).
-template <typename T, bool PRESSURE, int R>
-__global__ void __launch_bounds__(64 * kRegWaves, (R == 8 || R == 10) ? 4 : (R == 4 ? 6 : 1))
+// Eight wavefronts hold 4, 8 or 10 rows each, sixteen hold taller regions
+// (reg_waves): so a CU always has four wavefronts per SIMD to hide latency
+// with (six at 4 rows), within 128 VGPRs (80 at 4 rows).
+template <int R, int NW> constexpr int reg_waves_per_simd() { return R == 4 && NW == 8 ? 6 : 4; }
+
+template <typename T, int PM, int R, int NW>
+__global__ void __launch_bounds__(64 * NW, (reg_waves_per_simd<R, NW>()))
     k_project_regs(StepParams sp, const uint8_t* __restrict__ gates, const T* __restrict__ u_in,
                    const T* __restrict__ v_in, T* __restrict__ u_out, T* __restrict__ v_out,
                    float* __restrict__ p, RegArgs a) {
-  __shared__ RegShared sh;
-  project_regs_tile<T, PRESSURE, R, false>(sp, gates, u_in, v_in, u_out, v_out, p, a,
-                                    xcd_tile(blockIdx.x, gridDim.x), sh);
+  __shared__ RegShared<NW> sh;
+  project_regs_tile<T, PM, R, NW>(sp, gates, u_in, v_in, u_out, v_out, p, a,
+                                        xcd_tile(blockIdx.x, gridDim.x), sh);
 }
 
 template <typename T, bool PRESSURE>
@@ -289,184 +290,175 @@ void launch_tiled(const StepParams& sp, const GridView& g, const FieldPtrs& f, i
 // registers from the first sweep to the last.  The sweeps run in stages of
 // k (the last stage takes the rest); after a stage the owned cells are
 // exact and the halo is stale, so the workgroup stores the ring of owned
-// cells its neighbours read as halo (those within 2k of the tile's edge),
-// publishes the stage on its flag, waits for the adjacent tiles' flags and
-// reloads only its halo from their rings.  Stage s reads buffer s & 1 and
-// writes buffer (s + 1) & 1, so a ring is overwritten (two stages later)
-// only after every neighbour has finished the stage that read it, which it
-// did before publishing the stage this tile waited for.  The last stage
-// stores the whole tile (and the pressure sums) into buffer nstages & 1.
-// The last workgroup to finish clears the flags for the next launch.
+// cells its neighbours read as halo in the exchange buffer and takes its own
+// halo from theirs (projection_device.hpp, "halo exchange").  The fields
+// are read once, at the start, from buffer u_in, v_in and written once, at
+// the end, to u_out, v_out.
 //
 // Every tile's workgroup must be resident at once (the host checks the
-// tile count against resident_capacity); a wait is bounded by spin_ticks,
+// tile count, ProjTuning::resident_plan); a wait is bounded by spin_ticks,
 // after which the error word is set and the launch drains without waiting.
+constexpr int kWaitVm = 0x0F70;  // s_waitcnt vmcnt(0)
+
 struct ResidentArgs {
   int nstages;      // ceil(n / k)
   int last_sweeps;  // sweeps of the last stage
-  int nty;          // tile rows
-  unsigned* flags;  // [tiles]: stages published; [tiles]: finished workgroups
+  XWord* slots;     // kXSlots slots of slot_words words
+  long slot_words;
+  unsigned* state;  // finished workgroups; slot of "ring 0"
   int* error;
   long long spin_ticks;
 };
 
-// Wavefront 0: wait until the adjacent tiles (up to 8, one per lane) have
-// published `stage`.  False on timeout, or at once when another wait of the
-// launch has timed out.  The rings are read with agent-coherent loads
-// issued after this wait (behind the workgroup barrier that follows it), so
-// no cache needs invalidating.
-__device__ inline bool wait_neighbours(const ResidentArgs& ra, int ntx, int tile, unsigned stage) {
-  const int lane = (int)(threadIdx.x & 63);
-  const int tx = tile % ntx, ty = tile / ntx;
-  const int nx = tx + lane % 3 - 1, ny = ty + lane / 3 - 1;
-  const bool poll = lane < 9 && lane != 4 && (unsigned)nx < (unsigned)ntx &&
-                    (unsigned)ny < (unsigned)ra.nty;
-  const unsigned* f = ra.flags + (poll ? ny * ntx + nx : 0);
-  const long long t0 = wall_clock64();
-  for (;;) {
-    const bool ready =
-        !poll || __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= stage;
-    if (__all(ready)) break;
-    if (__hip_atomic_load(ra.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return false;
-    if (wall_clock64() - t0 > ra.spin_ticks) return false;
-    __builtin_amdgcn_s_sleep(1);
-  }
-  return true;
-}
-
-template <typename T, bool PRESSURE, int R>
-__global__ void __launch_bounds__(64 * kRegWaves, (R == 8 || R == 10) ? 4 : (R == 4 ? 6 : 1))
-    k_project_resident(StepParams sp, const uint8_t* __restrict__ gates, T* u0, T* v0, T* u1,
-                       T* v1, float* __restrict__ p, RegArgs a, ResidentArgs ra) {
-  __shared__ RegShared sh;
-  __shared__ int s_last;
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const RegPlace pl = reg_place<R>(a, tile);
-  RegTile<R> t;
-  reg_load<T, PRESSURE, R>(t, sp, gates, u0, v0, p, a, pl);
+// All stages of a wavefront of kind KIND, and the store of its rows.
+template <typename T, int PM, int R, int NW, int KIND>
+__device__ __attribute__((always_inline)) inline void resident_kind(
+    RegTile<R>& t, const StepParams& sp, const uint8_t* __restrict__ gates, T* __restrict__ u_out,
+    T* __restrict__ v_out, float* __restrict__ p, const RegArgs& a, const ResidentArgs& ra,
+    const RegPlace& pl, const XPlace& x, int base, RegShared<NW>& sh) {
+  if constexpr (KIND == WK_ANY) reg_masks<R>(t);
   for (int s = 0; s < ra.nstages; s++) {
-    const bool odd = (s & 1) != 0;
     if (s > 0) {
-      if (threadIdx.x < 64) {
-        const bool ok = wait_neighbours(ra, a.ntx, tile, (unsigned)s);
-        if (!ok && threadIdx.x == 0)
-          __hip_atomic_store(ra.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      // the barrier orders every wavefront's halo loads after the wait
-      __syncthreads();
-      reg_reload_halo<T, R>(t, odd ? u1 : u0, odd ? v1 : v0, sp, a, pl);
+      XWord* ring = ra.slots + (long)((base + s) % kXSlots) * ra.slot_words;
+      ring_store<T, R, NW, false>(t, ring, x, pl);
+      ring_load<T, R, NW>(t, ring, x, pl, ra.error, ra.spin_ticks);
     }
-    const bool last = s + 1 == ra.nstages;
-    // one barrier per colour phase (measured 0.4% faster than two here)
-    reg_sweeps<T, PRESSURE, R, true>(t, sh, sp, pl, a.th, last ? ra.last_sweeps : a.k);
-    T* uo = odd ? u0 : u1;
-    T* vo = odd ? v0 : v1;
-    if (!last) {
-      reg_store<T, PRESSURE, R, true>(t, uo, vo, p, sp, a, pl);
-      // every wavefront's ring stores (agent-coherent) have completed before
-      // the barrier, so they are visible GPU-wide before the flag is
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      if (threadIdx.x == 0)
-        __hip_atomic_store(ra.flags + tile, (unsigned)(s + 1), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-      reg_store<T, PRESSURE, R, false>(t, uo, vo, p, sp, a, pl);
-    }
+    // the barrier in reg_begin: every wavefront has read its part of ring s
+    const RowExchange rx = reg_begin<R, NW>(t, sh, pl.w, reg_lane());
+    // no load is outstanding here; saying so keeps the compiler from waiting
+    // for one, and so for the clearing stores below, in the sweeps
+    __builtin_amdgcn_s_waitcnt(kWaitVm);
+    if (s > 0)
+      ring_store<T, R, NW, true>(t, ra.slots + (long)((base + s - 1) % kXSlots) * ra.slot_words,
+                                 x, pl);
+    reg_sweeps<T, PM, R, NW, KIND>(t, sh, rx, sp, pl,
+                                         s + 1 == ra.nstages ? ra.last_sweeps : a.k);
+    // this wavefront's clearing stores have completed before it publishes
+    __builtin_amdgcn_s_waitcnt(kWaitVm);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
   }
-  // every other workgroup has finished waiting when the last one counts
-  // itself in, so that one may clear the flags
-  const int ntiles = a.ntx * ra.nty;
-  if (threadIdx.x == 0)
-    s_last = __hip_atomic_fetch_add(ra.flags + ntiles, 1u, __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(ntiles - 1);
-  __syncthreads();
-  if (s_last) {
-    for (int i = (int)threadIdx.x; i <= ntiles; i += (int)blockDim.x)
-      __hip_atomic_store(ra.flags + i, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  reg_store<T, PM, R>(t, gates, u_out, v_out, p, sp, a, pl);
+}
+
+template <typename T, int PM, int R, int NW>
+__global__ void __launch_bounds__(64 * NW, (reg_waves_per_simd<R, NW>()))
+    k_project_resident(StepParams sp, const uint8_t* __restrict__ gates,
+                       const T* __restrict__ u_in, const T* __restrict__ v_in,
+                       T* __restrict__ u_out, T* __restrict__ v_out, float* __restrict__ p,
+                       RegArgs a, ResidentArgs ra) {
+  __shared__ RegShared<NW> sh;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const RegPlace pl = reg_place<R, NW>(a, tile, sp.W, sp.H);
+  const XPlace x = x_place<T, R, NW>(a, pl, tile);
+  const int base = __builtin_amdgcn_readfirstlane((int)ra.state[1]);
+  RegTile<R> t;
+  reg_load<T, PM, R>(t, sp, gates, u_in, v_in, p, a, pl);
+  if (t.kind == WK_OPEN)
+    resident_kind<T, PM, R, NW, WK_OPEN>(t, sp, gates, u_out, v_out, p, a, ra, pl, x, base,
+                                               sh);
+  else if (t.kind == WK_WALL)
+    resident_kind<T, PM, R, NW, WK_WALL>(t, sp, gates, u_out, v_out, p, a, ra, pl, x, base,
+                                               sh);
+  else if (t.kind == WK_DRAIN)
+    resident_kind<T, PM, R, NW, WK_DRAIN>(t, sp, gates, u_out, v_out, p, a, ra, pl, x, base,
+                                                sh);
+  else if (t.kind == WK_DRAIN0)
+    resident_kind<T, PM, R, NW, WK_DRAIN0>(t, sp, gates, u_out, v_out, p, a, ra, pl, x, base,
+                                                 sh);
+  else
+    resident_kind<T, PM, R, NW, WK_ANY>(t, sp, gates, u_out, v_out, p, a, ra, pl, x, base,
+                                              sh);
+  // the last workgroup to finish moves "ring 0" to the ring left uncleared
+  if (threadIdx.x == 0 && __hip_atomic_fetch_add(ra.state, 1u, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+    __hip_atomic_store(ra.state, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(ra.state + 1, (unsigned)((base + ra.nstages - 1) % kXSlots),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
-template <typename T, bool PRESSURE, int R>
-const void* resident_kernel_r() {
-  return (const void*)k_project_resident<T, PRESSURE, R>;
-}
-
-template <typename T, bool PRESSURE>
+// The shapes' kernels, by region rows / 8 (resident ones:
+// ProjTuning::resident_plan).
+template <typename T, int PM>
 const void* resident_kernel(int rows) {
-  switch (rows) {
-    case 4: return resident_kernel_r<T, PRESSURE, 4>();
-    case 8: return resident_kernel_r<T, PRESSURE, 8>();
-    case 10: return resident_kernel_r<T, PRESSURE, 10>();
-    case 12: return resident_kernel_r<T, PRESSURE, 12>();
-    default: return resident_kernel_r<T, PRESSURE, 16>();
+  return rows == 4 ? (const void*)k_project_resident<T, PM, 4, 8>
+                   : (const void*)k_project_resident<T, PM, 6, 16>;  // 12
+}
+
+template <typename T, int PM>
+const void* regs_kernel(int rows) {
+  if (rows == 4) return (const void*)k_project_regs<T, PM, 4, 8>;
+  if (rows == 8) return (const void*)k_project_regs<T, PM, 8, 8>;
+  switch (PM == PM_NONE ? rows : 0) {
+    case 10: return (const void*)k_project_regs<T, PM_NONE, 10, 8>;
+    case 12: return (const void*)k_project_regs<T, PM_NONE, 6, 16>;
+    case 16: return (const void*)k_project_regs<T, PM_NONE, 8, 16>;
+    default: return nullptr;
   }
 }
 
-template <typename T, bool PRESSURE>
-void launch_resident(const StepParams& sp, const FieldPtrs& f, int* cur, const ProjTuning& t,
-                     long long spin_ticks, hipStream_t s) {
-  if (sp.n <= 0) return;
+RegArgs reg_args(const StepParams& sp, const ProjTuning& t) {
   RegArgs a;
   a.tw = t.tw;
   a.th = t.th;
   a.k = t.k;
-  a.ntx = (sp.W + a.tw - 1) / a.tw;
+  a.ntx = t.tiles_x(sp.W);
+  a.nty = t.tiles_y(sp.H);
+  a.inset = 0;
   a.sweeps = t.k;
   a.forces = sp.forces_in_projection ? 1 : 0;
+  return a;
+}
+
+template <typename T, int PM>
+void launch_resident(const StepParams& sp, const FieldPtrs& f, int* cur, const ProjTuning& t,
+                     hipStream_t s) {
+  if (sp.n <= 0) return;
+  RegArgs a = reg_args(sp, t);
   ResidentArgs ra;
   ra.nstages = (sp.n + t.k - 1) / t.k;
   ra.last_sweeps = sp.n - (ra.nstages - 1) * t.k;
-  ra.nty = (sp.H + a.th - 1) / a.th;
-  ra.flags = f.rflags;
+  ra.slots = (XWord*)f.exchange;
+  ra.slot_words = t.exchange_words(sp.W, sp.H, sizeof(T));
+  ra.state = f.rstate;
   ra.error = f.error;
-  ra.spin_ticks = spin_ticks;
+  ra.spin_ticks = sp.spin_ticks;
   const int in = *cur, other = 1 - in;
-  T* u0 = (T*)f.u[in];
-  T* v0 = (T*)f.v[in];
+  const T* u0 = (const T*)f.u[in];
+  const T* v0 = (const T*)f.v[in];
   T* u1 = (T*)f.u[other];
   T* v1 = (T*)f.v[other];
   void* args[] = {(void*)&sp, (void*)&f.gates, (void*)&u0, (void*)&v0, (void*)&u1,
                   (void*)&v1, (void*)&f.p, (void*)&a, (void*)&ra};
-  (void)hipLaunchKernel(resident_kernel<T, PRESSURE>(t.reg_rows()), dim3(a.ntx * ra.nty),
-                        dim3(64 * kRegWaves), args, 0, s);
-  if (ra.nstages & 1) *cur = other;
+  (void)hipLaunchKernel(resident_kernel<T, PM>(t.reg_rows()), dim3(a.ntx * a.nty),
+                        dim3(64 * reg_waves(t.reg_rows())), args, 0, s);
+  *cur = other;
 }
 
-template <typename T, bool PRESSURE, int R>
-void launch_regs_r(const StepParams& sp, const GridView& g, const FieldPtrs& f, int* cur,
-                   const ProjTuning& t, hipStream_t s) {
-  RegArgs a;
-  a.tw = t.tw;
-  a.th = t.th;
-  a.k = t.k;
-  a.ntx = (sp.W + a.tw - 1) / a.tw;
-  const int nty = (sp.H + a.th - 1) / a.th;
+template <typename T, int PM>
+void launch_regs(const StepParams& sp, const FieldPtrs& f, int* cur, const ProjTuning& t,
+                 hipStream_t s) {
+  RegArgs a = reg_args(sp, t);
   for (int done = 0; done < sp.n; done += t.k) {
     a.sweeps = (sp.n - done < t.k) ? sp.n - done : t.k;
-    a.forces = (done == 0 && sp.forces_in_projection) ? 1 : 0;
+    if (done > 0) a.forces = 0;
     const int nxt = 1 - *cur;
-    hipLaunchKernelGGL((k_project_regs<T, PRESSURE, R>), dim3(a.ntx * nty), dim3(64 * kRegWaves),
-                       0, s, sp, f.gates, (const T*)f.u[*cur], (const T*)f.v[*cur], (T*)f.u[nxt],
-                       (T*)f.v[nxt], f.p, a);
+    const T* u0 = (const T*)f.u[*cur];
+    const T* v0 = (const T*)f.v[*cur];
+    T* u1 = (T*)f.u[nxt];
+    T* v1 = (T*)f.v[nxt];
+    void* args[] = {(void*)&sp, (void*)&f.gates, (void*)&u0, (void*)&v0,
+                    (void*)&u1, (void*)&v1,      (void*)&f.p, (void*)&a};
+    (void)hipLaunchKernel(regs_kernel<T, PM>(t.reg_rows()), dim3(a.ntx * a.nty),
+                          dim3(64 * reg_waves(t.reg_rows())), args, 0, s);
     *cur = nxt;
   }
 }
 
-template <typename T, bool PRESSURE>
-void launch_regs(const StepParams& sp, const GridView& g, const FieldPtrs& f, int* cur,
-                 const ProjTuning& t, hipStream_t s) {
-  switch (t.reg_rows()) {
-    case 4: launch_regs_r<T, PRESSURE, 4>(sp, g, f, cur, t, s); break;
-    case 8: launch_regs_r<T, PRESSURE, 8>(sp, g, f, cur, t, s); break;
-    case 10: launch_regs_r<T, PRESSURE, 10>(sp, g, f, cur, t, s); break;
-    case 12: launch_regs_r<T, PRESSURE, 12>(sp, g, f, cur, t, s); break;
-    default: launch_regs_r<T, PRESSURE, 16>(sp, g, f, cur, t, s); break;
-  }
-}
+}  // namespace
 
 template <typename T>
-hipError_t allow_large_lds() {
+hipError_t init_projection() {
   const int bytes = (int)kLdsLimit;
   hipError_t e = hipFuncSetAttribute((const void*)k_project_tiled<T, false>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
@@ -476,46 +468,27 @@ hipError_t allow_large_lds() {
   return e;
 }
 
-
-}  // namespace
-
-hipError_t init_projection_kernels() {
-  hipError_t e = allow_large_lds<float>();
-  if (e == hipSuccess) e = allow_large_lds<__half>();
-  if (e == hipSuccess) e = allow_large_lds<__hip_bfloat16>();
-  return e;
-}
-
-// Workgroups of kRegWaves wavefronts a CU holds at once, from the register
-// kernels' launch bounds (which the compiler meets): at most 80 VGPRs at 4
-// rows (6 wavefronts per SIMD: 3 workgroups), 128 at 8 and 10 rows (4: 2
-// workgroups), up to 256 otherwise (1).  LDS (12 KiB per workgroup) and the
-// wavefront slots allow more.  (The runtime's occupancy query was not used:
-// it has returned 0 for a kernel that fits, depending on what ran before.)
-hipError_t resident_capacity(int rows, int* slots) {
-  int dev = 0, cus = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const int per_cu = rows == 4 ? 3 : (rows == 8 || rows == 10) ? 2 : 1;
-  *slots = e == hipSuccess ? per_cu * cus : 0;
-  return e;
-}
-
 template <typename T>
 void enqueue_projection(const StepParams& sp, const GridView& g, const FieldPtrs& f, int* cur,
                         const ProjTuning& t, hipStream_t s) {
-  if (t.kernel == PROJ_RESIDENT && t.valid(sp.pressure_on)) {
-    if (sp.pressure_on)
-      launch_resident<T, true>(sp, f, cur, t, sp.spin_ticks, s);
-    else
-      launch_resident<T, false>(sp, f, cur, t, sp.spin_ticks, s);
-    return;
-  }
-  if (t.kernel == PROJ_REGS && t.valid(sp.pressure_on)) {
-    if (sp.pressure_on)
-      launch_regs<T, true>(sp, g, f, cur, t, s);
-    else
-      launch_regs<T, false>(sp, g, f, cur, t, s);
+  if ((t.kernel == PROJ_RESIDENT || t.kernel == PROJ_REGS) && t.valid(sp.pressure_on)) {
+    // (pressure sums that need a division, d_t = 0 or |d_t| >= 2, always run
+    // a launch per stage)
+    ProjTuning run;
+    const bool resident = t.kernel == PROJ_RESIDENT && f.exchange &&
+                          t.resident_plan(sp.W, sp.H, sp.cus, &run);
+    if (!sp.pressure_on) {
+      resident ? launch_resident<T, PM_NONE>(sp, f, cur, run, s)
+               : launch_regs<T, PM_NONE>(sp, f, cur, t, s);
+    } else if (sp.pdt_recip == 0.0) {
+      launch_regs<T, PM_DIVIDE>(sp, f, cur, t, s);
+    } else if (sp.density == 1.0f && sp.cs == 1) {
+      resident ? launch_resident<T, PM_UNIT>(sp, f, cur, run, s)
+               : launch_regs<T, PM_UNIT>(sp, f, cur, t, s);
+    } else {
+      resident ? launch_resident<T, PM_RECIP>(sp, f, cur, run, s)
+               : launch_regs<T, PM_RECIP>(sp, f, cur, t, s);
+    }
     return;
   }
   if (t.kernel == PROJ_TILED && t.valid(sp.pressure_on)) {
@@ -534,12 +507,19 @@ void enqueue_projection(const StepParams& sp, const GridView& g, const FieldPtrs
   }
 }
 
-template void enqueue_projection<float>(const StepParams&, const GridView&, const FieldPtrs&, int*,
-                                        const ProjTuning&, hipStream_t);
-template void enqueue_projection<__half>(const StepParams&, const GridView&, const FieldPtrs&,
-                                         int*, const ProjTuning&, hipStream_t);
-template void enqueue_projection<__hip_bfloat16>(const StepParams&, const GridView&,
-                                                 const FieldPtrs&, int*, const ProjTuning&,
-                                                 hipStream_t);
+#define OSY_PROJECTION(T)                                                                  \
+  template hipError_t init_projection<T>();                                                \
+  template void enqueue_projection<T>(const StepParams&, const GridView&, const FieldPtrs&, \
+                                      int*, const ProjTuning&, hipStream_t);
+// one storage type per object (OSY_ONLY_STORAGE), so that they build at once
+#if !defined(OSY_ONLY_STORAGE) || OSY_ONLY_STORAGE == 0
+OSY_PROJECTION(float)
+#endif
+#if !defined(OSY_ONLY_STORAGE) || OSY_ONLY_STORAGE == 1
+OSY_PROJECTION(__half)
+#endif
+#if !defined(OSY_ONLY_STORAGE) || OSY_ONLY_STORAGE == 2
+OSY_PROJECTION(__hip_bfloat16)
+#endif
 
 }  // namespace osy

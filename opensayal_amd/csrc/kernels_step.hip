@@ -452,6 +452,13 @@ void layout_t(int field, bool to_ref, const StepParams& sp, const FieldPtrs& f, 
 
 }  // namespace
 
+hipError_t init_projection_kernels() {
+  hipError_t e = init_projection<float>();
+  if (e == hipSuccess) e = init_projection<__half>();
+  if (e == hipSuccess) e = init_projection<__hip_bfloat16>();
+  return e;
+}
+
 void launch_build_flags(const MaskParams& m, uint8_t* flags, uint8_t* gates, hipStream_t s) {
   hipLaunchKernelGGL(k_build_flags, cell_grid(m.P, m.H), dim3(kBX, kBY), 0, s, m, flags);
   hipLaunchKernelGGL(k_build_gates, cell_grid(m.P, m.H), dim3(kBX, kBY), 0, s, m, flags, gates);

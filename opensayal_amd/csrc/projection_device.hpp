@@ -37,23 +37,6 @@ __device__ inline float relaxed_quotient(float div, uint32_t g, float o) {
   return o * q;
 }
 
-// 2^-log2(s) of a cell with gate byte g (for s = 1, 2, 4).
-__device__ inline float gate_scale(uint32_t g) {
-  return __uint_as_float(0x3F800000u - (((g >> G_L2_SHIFT) & 3u) << 23));
-}
-
-// The same quotient for the register-resident kernel, from the cell's
-// gate_scale y: `slow` (wavefront uniform) says whether any lane of this
-// row may need the division; only such rows divide, every lane, and select.
-__device__ inline float row_quotient(float div, float y, uint32_t g, float o, bool slow) {
-  float q = div * y;
-  if (slow) {
-    const float qs = div / (float)__builtin_popcount(g & 15u);
-    q = (g & G_SLOW) ? qs : q;
-  }
-  return o * q;
-}
-
 // x + gate(d): d when the gate bit is set, else -0 (x + -0 == x for every x,
 // signed zeros and NaN included), so the face keeps its bits when closed.
 __device__ inline float gated_add(float x, float d, uint32_t g, int bit) {
@@ -99,62 +82,18 @@ __device__ inline void store_pair(T* __restrict__ a, long k, bool in0, bool in1,
   }
 }
 
-// Accesses of the resident projection's halo exchange, coherent across the
-// GPU without cache maintenance: relaxed agent-scope atomics, which the
-// compiler issues as loads and stores that bypass the caches that are not
-// coherent between CUs and XCDs (a CU's L1, an XCD's L2).  The bits of a
-// pair travel as one 2-element word.
-template <typename T>
-__device__ inline void coherent_load_pair(const T* a, long k, float& x0, float& x1) {
-  using W = typename std::conditional<sizeof(T) == 4, unsigned long long, unsigned>::type;
-  const W w = __hip_atomic_load(reinterpret_cast<const W*>(a + k), __ATOMIC_RELAXED,
-                                __HIP_MEMORY_SCOPE_AGENT);
-  typename PairOf<T>::type pr;
-  __builtin_memcpy(&pr, &w, sizeof(W));
-  x0 = Store<T>::ld(pr.x);
-  x1 = Store<T>::ld(pr.y);
-}
-
-template <typename T>
-__device__ inline void coherent_store_one(T* a, long k, float x) {
-  using W = typename std::conditional<sizeof(T) == 4, unsigned, unsigned short>::type;
-  const T e = Store<T>::st(x);
-  W w;
-  __builtin_memcpy(&w, &e, sizeof(W));
-  __hip_atomic_store(reinterpret_cast<W*>(a + k), w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-template <typename T>
-__device__ inline void coherent_store_pair(T* a, long k, bool in0, bool in1, float x0,
-                                           float x1) {
-  if (in0 && in1) {  // k is even and rows start on 64-element boundaries
-    using W = typename std::conditional<sizeof(T) == 4, unsigned long long, unsigned>::type;
-    typename PairOf<T>::type pr;
-    pr.x = Store<T>::st(x0);
-    pr.y = Store<T>::st(x1);
-    W w;
-    __builtin_memcpy(&w, &pr, sizeof(W));
-    __hip_atomic_store(reinterpret_cast<W*>(a + k), w, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  } else {
-    if (in0) coherent_store_one(a, k, x0);
-    if (in1) coherent_store_one(a, k + 1, x1);
-  }
-}
-
-// ---- register-resident kernel ------------------------------------------------
+// ---- register-resident kernels -----------------------------------------------
 //
-// Eight wavefronts stacked vertically; wavefront w holds region rows
+// NW wavefronts stacked vertically; wavefront w holds region rows
 // [w*R, w*R + R), lane l holds cells 2l and 2l+1 of each of them: u, v and
-// the gate byte of both cells, all in VGPRs for the whole launch.  The
-// region is 128 x 8R cells and the owned tile (128 - 4k) x (8R - 4k).
+// the face masks of both cells, all in VGPRs for the whole launch.  The
+// region is 128 x NW*R cells.
 //
 // In a colour phase each row has one active cell per lane (parity b).  For
 // b = 0 every face the cell touches is in the lane's own registers.  For
 // b = 1 the right face u(2l+2) belongs to lane l+1: it is read and updated
 // through DPP lane shifts.  The top face of a wavefront's last row belongs
-// to the wavefront above: its value is published through LDS before the
-// phase and the update sent back after it (two barriers per phase).
+// to the wavefront above and is exchanged through LDS (reg_phase).
 
 __device__ inline float lane_from_right(float x) {  // lane l gets lane l+1's x (0 for lane 63)
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, true));
@@ -162,18 +101,20 @@ __device__ inline float lane_from_right(float x) {  // lane l gets lane l+1's x 
 __device__ inline float lane_from_left(float x) {  // lane l gets lane l-1's x (0 for lane 0)
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
 }
-
-// gate of d: d when the bit is set, else -0 (which an addition leaves out
-// bit for bit)
-__device__ inline float gate_neg(float d, uint32_t g, int bit) {
-  const uint32_t m = (uint32_t)((int32_t)(g << (31 - bit)) >> 31);
-  return __uint_as_float((__float_as_uint(d) & m) | (~m & 0x80000000u));
+__device__ inline uint32_t lane_from_right_u(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x130, 0xf, 0xf, true);
+}
+__device__ inline uint32_t lane_from_left_u(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x138, 0xf, 0xf, true);
 }
 
-// gate of d: d when the bit is set, else +0
-__device__ inline float gate_pos(float d, uint32_t g, int bit) {
-  const uint32_t m = (uint32_t)((int32_t)(g << (31 - bit)) >> 31);
-  return __uint_as_float(__float_as_uint(d) & m);
+// A copy of x in a register of its own.  The values of a pair are loaded and
+// stored as one 8-byte register; left to itself the compiler keeps them in
+// such pairs through the sweeps, which it cannot colour without spilling.
+__device__ inline float own_register(float x) {
+  float y;
+  asm("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
+  return y;
 }
 
 // Gate byte of a cell from its flag f, the right neighbour's flag fr and
@@ -194,13 +135,48 @@ __device__ inline uint32_t gate_byte(uint32_t f, uint32_t fr, uint32_t ft) {
 }
 
 struct RegArgs {
-  int tw, th, k;  // owned tile and sweeps per launch (halo 2k)
-  int ntx;        // tiles per grid row
+  int tw, th, k;  // tile pitch and sweeps per launch or stage (halo 2k)
+  int ntx, nty;   // tiles per grid row and column
+  int inset;      // 0, or 2k: how far the first region reaches out of the grid
   int sweeps;     // sweeps this launch (<= k)
   int forces;     // apply the velocity forces on load, pressure sums from 0
 };
 
-__device__ inline bool lc_in_tile(int lc, int K, int tw) { return lc >= 2 * K && lc < 2 * K + tw; }
+// Where a workgroup's tile lies.  Region (tx, ty) starts at grid cell
+// (tx*tw, ty*th) - inset, all even, and is 128 x NW*R cells.  With inset 0 a
+// tile owns the cells of its region at least 2k from the region's edges, and
+// also those up to an edge that is the grid's own: nothing outside the grid
+// reaches them, so the first and last tiles need no halo there, and
+// (W - 4k) / tw tiles, rounded up, cover a row of W cells (one when
+// W <= 128).  The batch's tiles keep the halo all round (inset 2k, W / tw
+// tiles, rounded up).  Wavefront-uniform.
+struct RegPlace {
+  int K, gx0, gy0, w, rbase;
+  int c0, c1, r0, r1;  // owned columns [c0, c1) and rows [r0, r1) of the region
+  int rows;            // region rows inside the grid (inset 0)
+  bool left, right, below, above;  // a neighbouring tile on that side
+};
+
+template <int R, int NW>
+__device__ inline RegPlace reg_place(const RegArgs& a, int tile, int W, int H) {
+  RegPlace pl;
+  pl.K = a.k;
+  const int tx = tile % a.ntx, ty = tile / a.ntx;
+  pl.gx0 = tx * a.tw - a.inset;
+  pl.gy0 = ty * a.th - a.inset;
+  pl.w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  pl.rbase = pl.w * R;
+  pl.left = tx > 0;
+  pl.right = tx + 1 < a.ntx;
+  pl.below = ty > 0;
+  pl.above = ty + 1 < a.nty;
+  pl.c0 = pl.left ? 2 * a.k : a.inset;
+  pl.c1 = pl.right ? 2 * a.k + a.tw : W - pl.gx0;
+  pl.r0 = pl.below ? 2 * a.k : a.inset;
+  pl.r1 = pl.above ? 2 * a.k + a.th : H - pl.gy0;
+  pl.rows = min(NW * R, H - pl.gy0);
+  return pl;
+}
 
 // The divisor of update_pressure_at: d_t, and recip = 1.0 / (double)d_t
 // (the double nearest 1/d_t) when 0 < |d_t| < 2, else 0.
@@ -223,291 +199,316 @@ __device__ inline float pressure_term(float d, float density, float csf,
   return pd.recip != 0.0 ? (float)((double)x * pd.recip) : x / pd.d_t;
 }
 
-// Register state of one lane of the register-resident kernel.
+// How a kernel adds the pressure sums: not at all; through the double
+// reciprocal with density = cell_size = 1, whose products are the identity;
+// through it in general; by division.
+enum PressureMode : int { PM_NONE = 0, PM_UNIT = 1, PM_RECIP = 2, PM_DIVIDE = 3 };
+
+struct SweepParams {
+  float o, density, csf;
+  PressureDivisor pd;
+  int drain;  // region column of the grid's last column (W - 1); past the
+              // region (128 or more) in all but the last tiles of a row
+};
+
+template <int PM>
+__device__ inline float pressure_add(float p, float d, const SweepParams& q) {
+  if constexpr (PM == PM_UNIT) return p + (float)((double)d * q.pd.recip);
+  if constexpr (PM == PM_RECIP) return p + (float)((double)((d * q.density) * q.csf) * q.pd.recip);
+  if constexpr (PM == PM_DIVIDE) return p + ((d * q.density) * q.csf) / q.pd.d_t;
+  return p;
+}
+
+// Register state of one lane.  The face masks (wavefronts of kind WK_ANY
+// only, reg_masks) are one word per face, all
+// ones where the projection may move the face, else 0: mu0, mu1 the left
+// faces of cells 2l and 2l+1 (mu1 is also the right face of cell 2l, the
+// next lane's mu0 that of cell 2l+1), mv0, mv1 their bottom faces (row r+1's
+// are the top faces of row r), mt0, mt1 the top faces of row R-1.  A closed
+// face then costs one bit operation in each update: x + d becomes
+// x + (d or -0) and x - d becomes x - (d or +0), both of which leave every
+// x's bits when closed.
+//
+// The last column of an open grid (the drain) is fluid but not projected:
+// its left face moves with the cell to its left only, so the drain column's
+// own d is forced to -0 (SweepParams::drain), which leaves that face as it
+// is; its other faces are closed.
 template <int R>
 struct RegTile {
   float u0[R], u1[R], v0[R], v1[R];  // faces of cells 2l and 2l+1, rows 0..R-1
   float s0[R], s1[R];                // pressure sums (pressure runs only)
   uint32_t gw[R];                    // gate bytes: cell 2l in bits 0-7, 2l+1 in 8-15
-  uint32_t m0[R], m1[R];             // face masks of cells 2l and 2l+1 (reg_face_masks)
-  uint32_t slow;                     // wavefront-uniform: bit 2 rho + c set when some
-                                     // lane's cell c of row rho needs the general
-                                     // quotient (row_quotient, mask_quotient)
+  uint32_t mu0[R], mu1[R], mv0[R], mv1[R];
+  uint32_t mt0, mt1;
+  uint32_t cls[R];  // quotient_class of cell 2l, and of cell 2l+1 in the high half
+  // wavefront-uniform
+  bool enclosed;   // some projected cell has no open face (pressure runs)
+  int kind;        // WaveKind, and the lanes of a wall or the drain
+  unsigned long long lanes;
 };
 
-// Whether a tile keeps each cell's four face gates as byte masks (one VGPR
-// per cell, byte k 0xFF when face bit k is set, else 0) rather than as bits
-// of the gate byte: a gated face update is then one AND that selects and
-// sign-extends the mask byte in its operand, and one add.  Pressure runs
-// keep the gate byte, whose projected bit gates the sum.
-template <int R, bool PRESSURE> constexpr bool reg_face_masks() { return !PRESSURE; }
+// What the cells of a wavefront's rows are.
+enum WaveKind : int {
+  WK_OPEN = 0,   // all open: no face mask, quotient div * 0.25
+  WK_WALL = 1,   // open but for a wall, the same in every row: in some lanes
+                 // the even cell is solid and the odd cell's left face closed
+  WK_DRAIN = 2,  // open but for the drain column, an odd one, and the cells
+                 // right of it (outside the grid)
+  WK_DRAIN0 = 3,  // the same with an even drain column
+  WK_ANY = 4,     // anything else: face masks, any quotient
+};
 
-// The face masks of gate byte g: bit k of g (k = 0..3) spread to bit 8k by
-// one multiply (the 16 partial products land on distinct bits), then to
-// the whole byte.
-__device__ inline uint32_t face_masks(uint32_t g) {
-  return (((g & 15u) * 0x00204081u) & 0x01010101u) * 0xFFu;
+// Every kind is straight-line code: a tile waits for its slowest neighbour,
+// so the tiles at walls and obstacles set the pace of all, and a branch per
+// row, which leaves nothing to overlap a row's latency with, made those 1.5
+// times as slow.  A cell that moves nothing takes d = -0 where d is added
+// and +0 where it is subtracted, which leaves every face's bits.
+__device__ inline bool in_lanes(unsigned long long m) {
+  return __builtin_amdgcn_inverse_ballot_w64(m);
 }
 
-// d where face K of the masks m is open, else +0.
-template <int K>
-__device__ inline float mask_face(float d, uint32_t m) {
-  const uint32_t mk = (uint32_t)(int32_t)(int8_t)(uint8_t)(m >> (8 * K));
-  return __uint_as_float(__float_as_uint(d) & mk);
+// div / s with y = 1 / s rounded: third_quotient's correction, which for
+// s = 1, 2, 4 adds the (exact) remainder of a quotient that is already
+// rounded, so nothing.  With s = y = 0 it gives div * 0.
+__device__ inline float any_quotient(float div, float y, float s) {
+  const float q0 = div * y;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, s, div), y, q0);
+  return (q0 == 0.0f || __builtin_isinf(q0)) ? q0 : q1;
 }
 
-// div / s for a cell with face masks m (popcount(m) = 8s).  A cell with
-// s = 0 moves no face, so its quotient is never used, and almost every
-// other cell has s = 4: a row whose lanes all have s = 0 or 4 takes
-// div * 0.25.  The rest (`mixed`, wavefront uniform) take div * 2^-log2(s)
-// for s = 1, 2, 4 (log2(s) = 8s >> 4), exact, and third_quotient for s = 3
-// (the IEEE quotient div / 3 for every binary32 div).
-__device__ inline float mask_quotient(float div, uint32_t m, bool mixed) {
-  float q = div * 0.25f;
-  if (mixed) {
-    const uint32_t c8 = (uint32_t)__builtin_popcount(m);
-    const float qp = __builtin_amdgcn_ldexpf(div, -(int)(c8 >> 4));
-    q = c8 == 24u ? third_quotient(div) : qp;
+// The number s of a cell's open faces in the low byte and 12 / s (0 for
+// s = 0) in the next: y = (12 / s) * RN(1 / 12) is 1 / s rounded for every s.
+// (A table in a constant: with diverging branches here the compiler spilled a
+// register at their join before it had widened the lane mask again.)
+__device__ inline uint32_t quotient_class(int s) {
+  return (uint32_t)s | ((0x346C0u >> (4 * s)) & 15u) << 8;
+}
+
+// The quotient of the active cell of row rho, parity B.  A projected cell
+// without open faces adds div / 0 to its pressure (`enclosed`: the wavefront
+// has such cells), which is div * infinity.
+template <int R, int B, int PM, int KIND>
+__device__ __attribute__((always_inline)) inline float kind_quotient(const RegTile<R>& t,
+                                                                     const int rho, float div,
+                                                                     int lane, int drain) {
+  if constexpr (KIND == WK_WALL && B == 1) {
+    const bool w = in_lanes(t.lanes);
+    return any_quotient(div, w ? 1.0f / 3.0f : 0.25f, w ? 3.0f : 4.0f);
   }
-  return q;
+  if constexpr (KIND == WK_ANY) {
+    const uint32_t c = t.cls[rho] >> (16 * B);
+    const float s = (float)(c & 255u), y = (float)((c >> 8) & 255u) * (1.0f / 12.0f);
+    float q = any_quotient(div, y, s);
+    if constexpr (PM != PM_NONE) {
+      if (t.enclosed) q = (c & 255u) == 0 ? div * __builtin_inff() : q;
+    }
+    return 2 * lane + B == drain ? -0.0f : q;
+  }
+  return div * 0.25f;
 }
 
-// Whether some lane's face masks m need mask_quotient's general branch.
-__device__ inline bool mask_mixed(uint32_t m) {
-  const uint32_t c8 = (uint32_t)__builtin_popcount(m);
-  return __any(c8 != 0u && c8 != 32u);
+// The changes of the active cell's faces: `l`, `b` are added to its left and
+// bottom face, `r`, `t` subtracted from its right and top face.  For an odd
+// cell the right face's is taken by the next lane, which masks it.
+template <int B, int KIND>
+__device__ __attribute__((always_inline)) inline void face_changes(float d, uint32_t ml,
+                                                                   uint32_t mr, uint32_t mb,
+                                                                   uint32_t mt,
+                                                                   unsigned long long lanes,
+                                                                   float& l, float& r, float& b,
+                                                                   float& t) {
+  l = r = b = t = d;
+  if constexpr (KIND == WK_WALL) {
+    if constexpr (B == 0) {
+      l = b = in_lanes(lanes) ? -0.0f : d;
+      r = t = in_lanes(lanes) ? 0.0f : d;
+    } else {
+      l = in_lanes(lanes) ? -0.0f : d;
+    }
+  } else if constexpr (KIND == WK_DRAIN0 || (KIND == WK_DRAIN && B == 1)) {
+    l = b = in_lanes(lanes) ? -0.0f : d;
+    r = t = in_lanes(lanes) ? 0.0f : d;
+  } else if constexpr (KIND == WK_ANY) {
+    l = __uint_as_float((__float_as_uint(d) & ml) | (~ml & 0x80000000u));
+    b = __uint_as_float((__float_as_uint(d) & mb) | (~mb & 0x80000000u));
+    if constexpr (B == 0) r = __uint_as_float(__float_as_uint(d) & mr);
+    t = __uint_as_float(__float_as_uint(d) & mt);
+  }
 }
 
 // apply_projection_at for the active cell of row rho (parity B) of every
 // lane.  Cells near the region edge compute with stale neighbours; their
 // wrong values move one cell per phase and never reach the tile within a
-// launch, so no lane or row is masked.
-template <typename T, int R, int B, bool PRESSURE>
+// launch, so no lane or row is masked.  Cells that are not projected gather
+// a meaningless pressure sum, which reg_store leaves out.
+template <typename T, int R, int B, int PM, int KIND>
 __device__ __attribute__((always_inline)) inline void reg_row(RegTile<R>& t, const int rho,
                                                               float vt0, float vt1, float& dtop,
-                                                              float o, float density, float csf,
-                                                              const PressureDivisor& pd) {
+                                                              const SweepParams& sq, int lane) {
   const int up = rho + 1 < R ? rho + 1 : rho;  // row above (when inside the strip)
-  if constexpr (reg_face_masks<R, PRESSURE>()) {
-    // x + gate(d) as x - mask(-d) and x - gate(d) as x - mask(d): an open
-    // face gets x + d (x - (-d) is x + d in IEEE arithmetic), a closed one
-    // x - (+0), which is x for every x
-    if constexpr (B == 0) {
-      const uint32_t m = t.m0[rho];
-      const float uu = t.u0[rho], ur = t.u1[rho], vv = t.v0[rho];
-      const float vt = (rho + 1 < R) ? t.v0[up] : vt0;
-      const float div = ((ur - uu) + vt) - vv;
-      const float q = mask_quotient(div, m, (t.slow >> (2 * rho)) & 1u);
-      const float d = o * q, nd = -d;
-      float nu0 = uu - mask_face<0>(nd, m), nu1 = ur - mask_face<1>(d, m);
-      rnd2<T>(nu0, nu1);
-      t.u0[rho] = nu0;
-      t.u1[rho] = nu1;
-      if (rho + 1 < R) {
-        float nv = vv - mask_face<2>(nd, m), nt = vt - mask_face<3>(d, m);
-        rnd2<T>(nv, nt);
-        t.v0[rho] = nv;
-        t.v0[up] = nt;
-      } else {
-        t.v0[rho] = rnd<T>(vv - mask_face<2>(nd, m));
-        dtop = mask_face<3>(d, m);
-      }
-    } else {
-      const uint32_t m = t.m1[rho];
-      const float uu = t.u1[rho], ur = lane_from_right(t.u0[rho]), vv = t.v1[rho];
-      const float vt = (rho + 1 < R) ? t.v1[up] : vt1;
-      const float div = ((ur - uu) + vt) - vv;
-      const float q = mask_quotient(div, m, (t.slow >> (2 * rho + 1)) & 1u);
-      const float d = o * q, nd = -d;
-      float nu1 = uu - mask_face<0>(nd, m), nu0 = t.u0[rho] - lane_from_left(mask_face<1>(d, m));
-      rnd2<T>(nu1, nu0);
-      t.u1[rho] = nu1;
-      t.u0[rho] = nu0;
-      if (rho + 1 < R) {
-        float nv = vv - mask_face<2>(nd, m), nt = vt - mask_face<3>(d, m);
-        rnd2<T>(nv, nt);
-        t.v1[rho] = nv;
-        t.v1[up] = nt;
-      } else {
-        t.v1[rho] = rnd<T>(vv - mask_face<2>(nd, m));
-        dtop = mask_face<3>(d, m);
-      }
-    }
-  } else if constexpr (B == 0) {
-    // active cell 2l: faces u0, u1, v0[rho], v0[rho+1] (all in this lane)
-    const uint32_t g = t.gw[rho];
+  const bool inside = rho + 1 < R;
+  float cl, cr, cb, ct;
+  if constexpr (B == 0) {
+    const uint32_t mtop = inside ? t.mv0[up] : t.mt0;
     const float uu = t.u0[rho], ur = t.u1[rho], vv = t.v0[rho];
-    const float vt = (rho + 1 < R) ? t.v0[up] : vt0;
+    const float vt = inside ? t.v0[up] : vt0;
     const float div = ((ur - uu) + vt) - vv;
-    const float d = row_quotient(div, gate_scale(g), g, o, (t.slow >> (2 * rho)) & 1u);
-    if constexpr (PRESSURE) {
-      // a cell that is not projected adds -0, which leaves its sum's bits
-      t.s0[rho] = t.s0[rho] + gate_neg(pressure_term(d, density, csf, pd), g, 4);
-    }
-    float nu0 = gated_add(uu, d, g, 0), nu1 = gated_sub(ur, d, g, 1);
+    const float q = kind_quotient<R, 0, PM, KIND>(t, rho, div, lane, sq.drain);
+    const float d = sq.o * q;
+    if constexpr (PM != PM_NONE) t.s0[rho] = pressure_add<PM>(t.s0[rho], d, sq);
+    face_changes<0, KIND>(d, t.mu0[rho], t.mu1[rho], t.mv0[rho], mtop, t.lanes, cl, cr, cb, ct);
+    float nu0 = uu + cl, nu1 = ur - cr;
     rnd2<T>(nu0, nu1);
     t.u0[rho] = nu0;
     t.u1[rho] = nu1;
-    if (rho + 1 < R) {
-      float nv = gated_add(vv, d, g, 2), nt = gated_sub(vt, d, g, 3);
+    if (inside) {
+      float nv = vv + cb, nt = vt - ct;
       rnd2<T>(nv, nt);
       t.v0[rho] = nv;
       t.v0[up] = nt;
     } else {
-      t.v0[rho] = rnd<T>(gated_add(vv, d, g, 2));
-      dtop = gate_pos(d, g, 3);
+      t.v0[rho] = rnd<T>(vv + cb);
+      dtop = ct;
     }
   } else {
-    // active cell 2l+1: faces u1, u0 of lane l+1, v1[rho], v1[rho+1]
-    const uint32_t g = t.gw[rho] >> 8;
+    const uint32_t mtop = inside ? t.mv1[up] : t.mt1;
     const float uu = t.u1[rho], ur = lane_from_right(t.u0[rho]), vv = t.v1[rho];
-    const float vt = (rho + 1 < R) ? t.v1[up] : vt1;
+    const float vt = inside ? t.v1[up] : vt1;
     const float div = ((ur - uu) + vt) - vv;
-    const float d = row_quotient(div, gate_scale(g), g, o, (t.slow >> (2 * rho + 1)) & 1u);
-    if constexpr (PRESSURE) {
-      t.s1[rho] = t.s1[rho] + gate_neg(pressure_term(d, density, csf, pd), g, 4);
-    }
-    float nu1 = gated_add(uu, d, g, 0), nu0 = t.u0[rho] - lane_from_left(gate_pos(d, g, 1));
+    const float q = kind_quotient<R, 1, PM, KIND>(t, rho, div, lane, sq.drain);
+    const float d = sq.o * q;
+    if constexpr (PM != PM_NONE) t.s1[rho] = pressure_add<PM>(t.s1[rho], d, sq);
+    face_changes<1, KIND>(d, t.mu1[rho], 0, t.mv1[rho], mtop, t.lanes, cl, cr, cb, ct);
+    cr = lane_from_left(cr);
+    if constexpr (KIND == WK_ANY) cr = __uint_as_float(__float_as_uint(cr) & t.mu0[rho]);
+    float nu1 = uu + cl, nu0 = t.u0[rho] - cr;
     rnd2<T>(nu1, nu0);
     t.u1[rho] = nu1;
     t.u0[rho] = nu0;
-    if (rho + 1 < R) {
-      float nv = gated_add(vv, d, g, 2), nt = gated_sub(vt, d, g, 3);
+    if (inside) {
+      float nv = vv + cb, nt = vt - ct;
       rnd2<T>(nv, nt);
       t.v1[rho] = nv;
       t.v1[up] = nt;
     } else {
-      t.v1[rho] = rnd<T>(gated_add(vv, d, g, 2));
-      dtop = gate_pos(d, g, 3);
+      t.v1[rho] = rnd<T>(vv + cb);
+      dtop = ct;
     }
   }
 }
 
-// LDS the register-resident tile exchanges rows through, two slots of each
-// (with one barrier per phase consecutive phases use different slots).
+// LDS the wavefronts exchange rows through, two slots of each (consecutive
+// phases use different slots).
+template <int NW>
 struct RegShared {
-  float2 vrow[2][kRegWaves][64];  // row 0 (v0, v1) of each wavefront
-  float dsend[2][kRegWaves][64];  // top-row update for the wavefront above
+  float2 vrow[2][NW][64];  // row 0 (v0, v1) of each wavefront
+  float dsend[2][NW][64];  // top-row update for the wavefront above
 };
 
-// Rows RHO..R-1 of one phase, unrolled at compile time.
-template <typename T, int R, int PB, bool PRESSURE, int RHO>
+// What a wavefront has read of its neighbours' rows after a phase and not
+// yet used: the update from below of its row 0, row 0 of the wavefront above,
+// and its own update of that row.
+struct RowExchange {
+  float dd;
+  float2 x;
+  float dtop;
+};
+
+// The update from below reaches row 0.  PB is the parity of row 0's active
+// cell in the coming phase, the one whose face the wavefront below moved.
+template <typename T, int R, int PB>
+__device__ __attribute__((always_inline)) inline void reg_settle(RegTile<R>& t,
+                                                                 const RowExchange& x) {
+  if constexpr (PB == 1)
+    t.v1[0] = rnd<T>(t.v1[0] - x.dd);
+  else
+    t.v0[0] = rnd<T>(t.v0[0] - x.dd);
+}
+
+// Rows RHO..LAST of one phase, unrolled at compile time.
+template <typename T, int R, int PB, int PM, int KIND, int RHO, int LAST>
 __device__ __attribute__((always_inline)) inline void reg_rows_from(RegTile<R>& t, float vt0,
                                                                     float vt1, float& dtop,
-                                                                    float o, float density,
-                                                                    float csf, const PressureDivisor& pd) {
-  if constexpr (RHO < R) {
-    reg_row<T, R, ((PB + RHO) & 1), PRESSURE>(t, RHO, vt0, vt1, dtop, o, density, csf, pd);
-    reg_rows_from<T, R, PB, PRESSURE, RHO + 1>(t, vt0, vt1, dtop, o, density, csf, pd);
+                                                                    const SweepParams& sq,
+                                                                    int lane) {
+  if constexpr (RHO <= LAST) {
+    reg_row<T, R, ((PB + RHO) & 1), PM, KIND>(t, RHO, vt0, vt1, dtop, sq, lane);
+    reg_rows_from<T, R, PB, PM, KIND, RHO + 1, LAST>(t, vt0, vt1, dtop, sq, lane);
   }
+}
+
+// The rows of a phase: those inside the strip first, then the first and the
+// last, which need what the exchange of the previous phase brings, so its
+// latency is hidden.  (Active cells of adjacent rows share no face, so the
+// order of the rows does not matter.)
+template <typename T, int R, int PB, int PM, int KIND>
+__device__ __attribute__((always_inline)) inline void reg_rows(RegTile<R>& t, const RowExchange& x,
+                                                               float& dtop, const SweepParams& sq,
+                                                               int lane) {
+  reg_rows_from<T, R, PB, PM, KIND, 1, R - 2>(t, 0.0f, 0.0f, dtop, sq, lane);
+  reg_settle<T, R, PB>(t, x);
+  reg_row<T, R, PB, PM, KIND>(t, 0, 0.0f, 0.0f, dtop, sq, lane);
+  // row 0 of the wavefront above as that wavefront has it once it settles
+  constexpr bool odd = ((PB + R) & 1) != 0;
+  const float vt0 = odd ? x.x.x : rnd<T>(x.x.x - x.dtop);
+  const float vt1 = odd ? rnd<T>(x.x.y - x.dtop) : x.x.y;
+  reg_row<T, R, ((PB + R - 1) & 1), PM, KIND>(t, R - 1, vt0, vt1, dtop, sq, lane);
 }
 
 // One colour phase.  PB is the parity of the active cell in row 0 of this
-// wavefront (compile time: phases come in pairs with PB and 1 - PB).  A
-// wavefront none of whose rows can still reach the tile skips the phase;
-// the others run it as straight-line code over registers.
+// wavefront (compile time: phases come in pairs with PB and 1 - PB); with
+// ACTIVE false the wavefront's rows stay as they are.
 //
-// (vt0, vt1) is row 0 of the wavefront above as it stands when the phase
-// starts: the top faces of this wavefront's last row.  The last row moves
-// those faces by dtop, which the wavefront above applies to its row 0.
-// Two ways to exchange both through LDS:
-//  * two barriers (ONE_SYNC false): each wavefront publishes its row 0 and
-//    reads (vt0, vt1) after the first; sends dtop and applies the one from
-//    below after the second.
-//  * one barrier (ONE_SYNC true): each wavefront publishes its row 0 after
-//    computing (this phase's own updates, before the one from below) beside
-//    dtop; after the barrier it applies the update from below to its row 0,
-//    and the wavefront below applies the same update, with the same
-//    rounding, to the copy it reads, which is then the row as the wavefront
-//    above holds it.  The slots alternate between phases (slot b), so none
-//    is rewritten before every reader of its previous contents has passed
-//    the next barrier.  The caller publishes and reads the rows as loaded
-//    before the first phase.
-// The two give the same bits.  The persistent batch kernel measured faster
-// with one barrier; the per-grid kernel measured no faster at 8 rows and
-// slower at 4 (its extra live registers cost a wavefront per SIMD).
-template <typename T, int R, int PB, bool PRESSURE, bool ONE_SYNC>
-__device__ __attribute__((always_inline)) inline void reg_phase(RegTile<R>& t, RegShared& sh,
-                                                                float& vt0, float& vt1, int lane,
-                                                                int w, int rbase, int s,
-                                                                int nphase, int K, int th,
-                                                                float o, float density,
-                                                                float csf, const PressureDivisor& pd) {
-  const int e = nphase - 1 - s;
-  const int lo = 2 * K - 1 - e;
-  const int rhi = 2 * K + th + e;
-  const int rlo = lo - rbase, rhi_rel = rhi - rbase;  // box rows of this wavefront
-  const int b = ONE_SYNC ? (s + 1) & 1 : 0;
-  if constexpr (!ONE_SYNC) {
-    if (w > 0) sh.vrow[0][w][lane] = make_float2(t.v0[0], t.v1[0]);
-    __syncthreads();
-    vt0 = vt1 = 0.0f;  // not carried from the previous phase
-    if (w < kRegWaves - 1) {
-      const float2 x = sh.vrow[0][w + 1][lane];
-      vt0 = x.x;
-      vt1 = x.y;
-    }
-  }
+// The top faces of a wavefront's last row are row 0's of the wavefront
+// above.  One barrier per phase: each wavefront publishes its row 0 after
+// computing (this phase's own updates, before the one from below) beside
+// dtop, the update its last row makes to the row above; after the barrier it
+// reads both its neighbours'.  In the next phase it applies the update from
+// below to its row 0, and the wavefront below applies the same update, with
+// the same rounding, to the copy it has read, which is then the row as the
+// wavefront above holds it.  The slots alternate between phases, so none is
+// rewritten before every reader of its previous contents has passed the next
+// barrier.  reg_begin publishes and reads the rows as loaded.
+template <typename T, int R, int NW, int PB, int SLOT, int PM, int KIND, bool ACTIVE>
+__device__ __attribute__((always_inline)) inline void reg_phase(RegTile<R>& t, RegShared<NW>& sh,
+                                                                RowExchange& x, int lane, int w,
+                                                                const SweepParams& sq) {
   float dtop = 0.0f;
-  if (rlo < R && rhi_rel > 0) {  // wavefront-uniform: some row is in the box
-    // the gate words do not change during the launch; hiding that from the
-    // compiler keeps it from hoisting the 8 face masks per row out of the
-    // phase loop into registers
-#pragma unroll
-    for (int rho = 0; rho < R; rho++) {
-      if constexpr (reg_face_masks<R, PRESSURE>()) {
-        asm volatile("" : "+v"(t.m0[rho]));
-        asm volatile("" : "+v"(t.m1[rho]));
-      } else {
-        asm volatile("" : "+v"(t.gw[rho]));
-      }
-    }
-    reg_rows_from<T, R, PB, PRESSURE, 0>(t, vt0, vt1, dtop, o, density, csf, pd);
-  }
-  if constexpr (ONE_SYNC) {
-    if (w > 0) sh.vrow[b][w][lane] = make_float2(t.v0[0], t.v1[0]);
-  }
-  if (w < kRegWaves - 1) sh.dsend[b][w][lane] = dtop;
+  if constexpr (ACTIVE)
+    reg_rows<T, R, PB, PM, KIND>(t, x, dtop, sq, lane);
+  else
+    reg_settle<T, R, PB>(t, x);
+  if (w > 0) sh.vrow[SLOT][w][lane] = make_float2(t.v0[0], t.v1[0]);
+  if (w < NW - 1) sh.dsend[SLOT][w][lane] = dtop;
   __syncthreads();
-  if (w > 0) {
-    // the wavefront below moved the top faces of its last row: they are
-    // this wavefront's row-0 v of parity 1 - PB
-    const float dd = sh.dsend[b][w - 1][lane];
-    if constexpr (PB == 0)
-      t.v1[0] = rnd<T>(t.v1[0] - dd);
-    else
-      t.v0[0] = rnd<T>(t.v0[0] - dd);
-  }
-  if constexpr (ONE_SYNC) {
-    if (w < kRegWaves - 1) {
-      const float2 x = sh.vrow[b][w + 1][lane];
-      if constexpr (PB == 0) {
-        vt0 = x.x;
-        vt1 = rnd<T>(x.y - dtop);
-      } else {
-        vt0 = rnd<T>(x.x - dtop);
-        vt1 = x.y;
-      }
-    }
-  }
+  x.dd = w > 0 ? sh.dsend[SLOT][w - 1][lane] : 0.0f;
+  x.x = w < NW - 1 ? sh.vrow[SLOT][w + 1][lane] : make_float2(0.0f, 0.0f);
+  x.dtop = dtop;
 }
 
-// Where a workgroup's tile lies: K (halo 2K), the region origin (gx0 is
-// even) and this wavefront's first region row.  Wavefront-uniform.
-struct RegPlace {
-  int K, gx0, gy0, w, rbase;
-};
-
-template <int R>
-__device__ inline RegPlace reg_place(const RegArgs& a, int tile) {
-  RegPlace pl;
-  pl.K = a.k;
-  const int tx = tile % a.ntx, ty = tile / a.ntx;
-  pl.gx0 = tx * a.tw - 2 * a.k;
-  pl.gy0 = ty * a.th - 2 * a.k;
-  pl.w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  pl.rbase = pl.w * R;
-  return pl;
+// `pairs` pairs of phases.  A loop of its own for each kind keeps the rows in
+// the same registers throughout (a choice inside the loop made the compiler
+// copy them at every phase).
+template <typename T, int R, int NW, int PB, int PM, int KIND, bool ACTIVE>
+__device__ __attribute__((always_inline)) inline void reg_pairs(RegTile<R>& t, RegShared<NW>& sh,
+                                                                RowExchange& x, int lane, int w,
+                                                                int pairs,
+                                                                const SweepParams& sq) {
+  for (int i = 0; i < pairs; i++) {
+    if constexpr (ACTIVE && KIND == WK_ANY) {
+      // the masks do not change during the launch; hiding that from the
+      // compiler keeps it from hoisting what it derives from them out of the
+      // phase loop into registers
+#pragma unroll
+      for (int rho = 0; rho < R; rho++) {
+        asm volatile("" : "+v"(t.mu0[rho]), "+v"(t.mu1[rho]));
+        asm volatile("" : "+v"(t.mv0[rho]), "+v"(t.mv1[rho]), "+v"(t.cls[rho]));
+      }
+      asm volatile("" : "+v"(t.mt0), "+v"(t.mt1));
+    }
+    reg_phase<T, R, NW, PB, 1, PM, KIND, ACTIVE>(t, sh, x, lane, w, sq);
+    reg_phase<T, R, NW, 1 - PB, 0, PM, KIND, ACTIVE>(t, sh, x, lane, w, sq);
+  }
 }
 
 // This lane's index, re-read from the thread index so that it is not kept
@@ -523,7 +524,7 @@ __device__ inline int reg_lane() {
 // into the row (so a pair stays inside its row of P cells) and the row
 // clamped into the grid, with no branch, so a wavefront waits for HBM once
 // rather than once per row.  Cells outside the grid are then set to 0.
-template <typename T, bool PRESSURE, int R>
+template <typename T, int PM, int R>
 __device__ __attribute__((always_inline)) inline void reg_load(RegTile<R>& t, const StepParams& sp,
                                                                const uint8_t* __restrict__ gates,
                                                                const T* __restrict__ u_in,
@@ -535,108 +536,193 @@ __device__ __attribute__((always_inline)) inline void reg_load(RegTile<R>& t, co
   const int W = sp.W, H = sp.H, P = sp.P;
   const int gi = pl.gx0 + 2 * lane;
   const bool col0 = (unsigned)gi < (unsigned)W, col1 = (unsigned)(gi + 1) < (unsigned)W;
-  t.slow = 0;
-  const int gic = min(max(gi, 0), P - 2);
+  // a scalar row pointer and one column offset for every access
+  const unsigned gic = (unsigned)min(max(gi, 0), P - 2);
   uint32_t graw[R];
 #pragma unroll
   for (int rho = 0; rho < R; rho++) {
-    const long k = (long)min(max(pl.gy0 + pl.rbase + rho, 0), H - 1) * P + gic;
-    load_pair(u_in, k, true, true, t.u0[rho], t.u1[rho]);
-    load_pair(v_in, k, true, true, t.v0[rho], t.v1[rho]);
-    graw[rho] = *reinterpret_cast<const uint16_t*>(gates + k);
-    if constexpr (PRESSURE) {
-      const float2 pp = *reinterpret_cast<const float2*>(p + k);
-      t.s0[rho] = pp.x;
-      t.s1[rho] = pp.y;
+    const long row = (long)min(max(pl.gy0 + pl.rbase + rho, 0), H - 1) * P;
+    load_pair(u_in + row, gic, true, true, t.u0[rho], t.u1[rho]);
+    load_pair(v_in + row, gic, true, true, t.v0[rho], t.v1[rho]);
+    graw[rho] = *reinterpret_cast<const uint16_t*>(gates + row + gic);
+    if constexpr (PM != PM_NONE) {
+      // the sums of the owned cells only; they start at 0 with the forces
+      const int r = pl.rbase + rho;
+      t.s0[rho] = t.s1[rho] = 0.0f;
+      if (!a.forces && r >= pl.r0 && r < pl.r1) {
+        const float2 pp = *reinterpret_cast<const float2*>(p + row + gic);
+        t.s0[rho] = pp.x;
+        t.s1[rho] = pp.y;
+      }
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // a wavefront inside the grid whose cells are all open needs no more
+  const bool inside = pl.gx0 >= 0 && pl.gx0 + 128 <= W && pl.gy0 + pl.rbase >= 0 &&
+                      pl.gy0 + pl.rbase + R <= H;
+  uint32_t open = 0x0F0Fu;
+#pragma unroll
+  for (int rho = 0; rho < R; rho++) open &= graw[rho];
+  t.enclosed = false;
+  t.lanes = 0;
+  if (inside && __all(open == 0x0F0Fu)) {
+    t.kind = WK_OPEN;
+  } else {
+    // cells outside the grid hold 0 and closed faces
+    bool same = true;
+    unsigned long long even = 0, odd = 0, wall1 = ~0ULL, none0 = ~0ULL, none1 = ~0ULL;
+#pragma unroll
+    for (int rho = 0; rho < R; rho++) {
+      const bool row_in = (unsigned)(pl.gy0 + pl.rbase + rho) < (unsigned)H;
+      const bool in0 = row_in && col0, in1 = row_in && col1;
+      t.u0[rho] = in0 ? t.u0[rho] : 0.0f;
+      t.v0[rho] = in0 ? t.v0[rho] : 0.0f;
+      t.u1[rho] = in1 ? t.u1[rho] : 0.0f;
+      t.v1[rho] = in1 ? t.v1[rho] : 0.0f;
+      // the gate bytes of cells 2l and 2l+1 (static, built with the flags)
+      const uint32_t g0 = in0 ? (graw[rho] & 0xFFu) : 0u, g1 = in1 ? (graw[rho] >> 8) : 0u;
+      t.gw[rho] = g0 | g1 << 8;
+      const int n0 = __builtin_popcount(g0 & 15u), n1 = __builtin_popcount(g1 & 15u);
+      if constexpr (PM != PM_NONE)
+        t.enclosed |= __any(((g0 & G_UPD) && n0 == 0) || ((g1 & G_UPD) && n1 == 0));
+      const unsigned long long open0 = __ballot(n0 == 4), open1 = __ballot(n1 == 4);
+      if (rho == 0) {
+        even = open0;
+        odd = open1;
+      }
+      wall1 &= __ballot(n1 == 3 && !(g1 & G_L));
+      same = same && even == open0 && odd == open1 && (__ballot(n0 != 0) & ~open0) == 0;
+      none0 &= __ballot(n0 == 0);
+      none1 &= __ballot(n1 == 0);
+    }
+    // lanes from the drain column's on
+    const int drain = W - 1 - pl.gx0;
+    const unsigned long long past = drain < 128 ? ~0ULL << (drain >> 1) : 0ULL;
+    // (an enclosed cell has to show in the pressure)
+    same = same && !t.enclosed;
+    t.kind = WK_ANY;
+    if (same && (even & odd) == ~0ULL) {
+      t.kind = WK_OPEN;
+    } else if (same && even == odd && wall1 == ~odd && drain >= 128) {
+      t.kind = WK_WALL;
+      t.lanes = ~odd;
+    } else if (same && odd == ~past && none1 == past) {
+      t.lanes = past;
+      if ((drain & 1) && even == ~(past << 1))
+        t.kind = WK_DRAIN;
+      else if (!(drain & 1) && even == ~past && none0 == past)
+        t.kind = WK_DRAIN0;
     }
   }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int rho = 0; rho < R; rho++) {
-    const int gj = pl.gy0 + pl.rbase + rho;
-    const bool row_in = (unsigned)gj < (unsigned)H;
-    const bool in0 = row_in && col0, in1 = row_in && col1;
-    t.u0[rho] = in0 ? t.u0[rho] : 0.0f;
-    t.v0[rho] = in0 ? t.v0[rho] : 0.0f;
-    t.u1[rho] = in1 ? t.u1[rho] : 0.0f;
-    t.v1[rho] = in1 ? t.v1[rho] : 0.0f;
+    t.u0[rho] = own_register(t.u0[rho]);
+    t.v0[rho] = own_register(t.v0[rho]);
+    t.u1[rho] = own_register(t.u1[rho]);
+    t.v1[rho] = own_register(t.v1[rho]);
     if (a.forces) {  // the forces' results as stored (rounded to T)
-      if (in0) {
+      const int gj = pl.gy0 + pl.rbase + rho;
+      const bool row_in = (unsigned)gj < (unsigned)H;
+      if (row_in && col0) {
         force_uv(sp, gi, gj, t.u0[rho], t.v0[rho]);
         t.u0[rho] = rnd<T>(t.u0[rho]);
         t.v0[rho] = rnd<T>(t.v0[rho]);
       }
-      if (in1) {
+      if (row_in && col1) {
         force_uv(sp, gi + 1, gj, t.u1[rho], t.v1[rho]);
         t.u1[rho] = rnd<T>(t.u1[rho]);
         t.v1[rho] = rnd<T>(t.v1[rho]);
       }
     }
-    if constexpr (PRESSURE) {  // the forces zero the pressure
-      t.s0[rho] = (in0 && !a.forces) ? t.s0[rho] : 0.0f;
-      t.s1[rho] = (in1 && !a.forces) ? t.s1[rho] : 0.0f;
+    if constexpr (PM != PM_NONE) {
+      t.s0[rho] = own_register(t.s0[rho]);
+      t.s1[rho] = own_register(t.s1[rho]);
     } else {
       t.s0[rho] = t.s1[rho] = 0.0f;
     }
-    // the gate bytes of cells 2l and 2l+1 (static, built with the flags)
-    t.gw[rho] = (in0 ? (graw[rho] & 0xFFu) : 0u) | (in1 ? (graw[rho] & 0xFF00u) : 0u);
-    if constexpr (reg_face_masks<R, PRESSURE>()) {
-      t.m0[rho] = face_masks(t.gw[rho]);
-      t.m1[rho] = face_masks(t.gw[rho] >> 8);
-      t.slow |= (mask_mixed(t.m0[rho]) ? 1u : 0u) << (2 * rho);
-      t.slow |= (mask_mixed(t.m1[rho]) ? 1u : 0u) << (2 * rho + 1);
-    } else {
-      t.slow |= (__any((t.gw[rho] & G_SLOW) != 0) ? 1u : 0u) << (2 * rho);
-      t.slow |= (__any((t.gw[rho] & (G_SLOW << 8)) != 0) ? 1u : 0u) << (2 * rho + 1);
-    }
+    __builtin_amdgcn_sched_barrier(0);  // row by row: mixed, they would spill
   }
 }
 
-// `sweeps` sweeps over the registers: colour 0 (even cells) first; row 0's
-// active parity in a colour-0 phase is (gy0 + rbase) & 1 and flips every
-// phase.
-template <typename T, bool PRESSURE, int R, bool ONE_SYNC>
-__device__ __attribute__((always_inline)) inline void reg_sweeps(RegTile<R>& t, RegShared& sh,
+// The face masks and quotient classes of a wavefront of kind WK_ANY, from
+// its gate bytes.  A face's two cells agree about it except at the drain
+// column, whose left face only the cell to its left names.
+template <int R>
+__device__ __attribute__((always_inline)) inline void reg_masks(RegTile<R>& t) {
+#pragma unroll
+  for (int rho = 0; rho < R; rho++) {
+    const uint32_t g0 = t.gw[rho] & 0xFFu, g1 = t.gw[rho] >> 8;
+    t.mu0[rho] = 0u - ((g0 | (lane_from_left_u(g1) >> 1)) & 1u);
+    t.mu1[rho] = 0u - ((g0 >> 1) & 1u);
+    t.mv0[rho] = 0u - ((g0 >> 2) & 1u);
+    t.mv1[rho] = 0u - ((g1 >> 2) & 1u);
+    if (rho == R - 1) {
+      t.mt0 = 0u - ((g0 >> 3) & 1u);
+      t.mt1 = 0u - ((g1 >> 3) & 1u);
+    }
+    t.cls[rho] = quotient_class(__builtin_popcount(g0 & 15u)) |
+                 quotient_class(__builtin_popcount(g1 & 15u)) << 16;
+  }
+}
+
+// Before the first phase: row 0 of the wavefront above, as loaded (a zero
+// update leaves every value's bits).
+template <int R, int NW>
+__device__ __attribute__((always_inline)) inline RowExchange reg_begin(const RegTile<R>& t,
+                                                                       RegShared<NW>& sh, int w,
+                                                                       int lane) {
+  RowExchange x;
+  x.dd = x.dtop = 0.0f;
+  if (w > 0) sh.vrow[0][w][lane] = make_float2(t.v0[0], t.v1[0]);
+  __syncthreads();
+  x.x = w < NW - 1 ? sh.vrow[0][w + 1][lane] : make_float2(0.0f, 0.0f);
+  return x;
+}
+
+// `sweeps` sweeps over the registers of a wavefront of kind KIND, after
+// reg_begin.  A wavefront takes part in a phase while some of its rows can
+// still reach the tile: rows [r0 - 1 - e, r1 + e) with e phases to come.  So
+// it sits out the last phases (all but an odd one, which does no harm).
+// Colour 0 (even cells) comes first; row 0's active parity in a colour-0
+// phase, PB, is that of its grid row, gy0 + rbase (gy0 is even).
+template <typename T, int R, int NW, int PB, int PM, int KIND>
+__device__ __attribute__((always_inline)) inline void reg_sweeps_from(RegTile<R>& t,
+                                                                      RegShared<NW>& sh,
+                                                                      RowExchange x, int lane,
+                                                                      const RegPlace& pl,
+                                                                      int sweeps,
+                                                                      const SweepParams& sq) {
+  const int idle = max(max(pl.r0 - pl.rbase - R, pl.rbase - pl.r1 + 1), 0);
+  const int pairs = max(2 * sweeps - idle + 1, 0) / 2;
+  reg_pairs<T, R, NW, PB, PM, KIND, true>(t, sh, x, lane, pl.w, pairs, sq);
+  reg_pairs<T, R, NW, PB, PM, KIND, false>(t, sh, x, lane, pl.w, sweeps - pairs, sq);
+  reg_settle<T, R, PB>(t, x);
+}
+
+template <typename T, int PM, int R, int NW, int KIND>
+__device__ __attribute__((always_inline)) inline void reg_sweeps(RegTile<R>& t, RegShared<NW>& sh,
+                                                                 const RowExchange& x,
                                                                  const StepParams& sp,
-                                                                 const RegPlace& pl, int th,
-                                                                 int sweeps) {
+                                                                 const RegPlace& pl, int sweeps) {
   const int lane = reg_lane();
-  const int w = pl.w, rbase = pl.rbase, K = pl.K;
-  const float o = sp.o;
-  const float csf = (float)sp.cs;
-  const PressureDivisor pdiv{sp.d_t, sp.pdt_recip};
-  const int nphase = 2 * sweeps;
-  float vt0 = 0.0f, vt1 = 0.0f;
-  if constexpr (ONE_SYNC) {  // row 0 of the wavefront above, as loaded
-    if (w > 0) sh.vrow[0][w][lane] = make_float2(t.v0[0], t.v1[0]);
-    __syncthreads();
-    if (w < kRegWaves - 1) {
-      const float2 x = sh.vrow[0][w + 1][lane];
-      vt0 = x.x;
-      vt1 = x.y;
-    }
-  }
-  if (((pl.gy0 + rbase) & 1) == 0) {
-    for (int s = 0; s < nphase; s += 2) {
-      reg_phase<T, R, 0, PRESSURE, ONE_SYNC>(t, sh, vt0, vt1, lane, w, rbase, s, nphase, K, th, o,
-                                             sp.density, csf, pdiv);
-      reg_phase<T, R, 1, PRESSURE, ONE_SYNC>(t, sh, vt0, vt1, lane, w, rbase, s + 1, nphase, K,
-                                             th, o, sp.density, csf, pdiv);
-    }
-  } else {
-    for (int s = 0; s < nphase; s += 2) {
-      reg_phase<T, R, 1, PRESSURE, ONE_SYNC>(t, sh, vt0, vt1, lane, w, rbase, s, nphase, K, th, o,
-                                             sp.density, csf, pdiv);
-      reg_phase<T, R, 0, PRESSURE, ONE_SYNC>(t, sh, vt0, vt1, lane, w, rbase, s + 1, nphase, K,
-                                             th, o, sp.density, csf, pdiv);
-    }
-  }
+  SweepParams sq;
+  sq.o = sp.o;
+  sq.density = sp.density;
+  sq.csf = (float)sp.cs;
+  sq.pd = PressureDivisor{sp.d_t, sp.pdt_recip};
+  sq.drain = sp.W - 1 - pl.gx0;
+  if (R % 2 == 0 || (pl.rbase & 1) == 0)
+    reg_sweeps_from<T, R, NW, 0, PM, KIND>(t, sh, x, lane, pl, sweeps, sq);
+  else
+    reg_sweeps_from<T, R, NW, 1, PM, KIND>(t, sh, x, lane, pl, sweeps, sq);
 }
 
-// Writes back the owned tile (RING: only its cells within 2K of the tile's
-// edge, which are the halos of the neighbouring tiles, and no pressure).
-template <typename T, bool PRESSURE, int R, bool RING>
+// Writes back the owned tile, and the pressure sums of its projected cells
+// (with `forces`, 0 for the others, as the forces leave them).
+template <typename T, int PM, int R>
 __device__ __attribute__((always_inline)) inline void reg_store(const RegTile<R>& t,
+                                                                const uint8_t* __restrict__ gates,
                                                                 T* __restrict__ u_out,
                                                                 T* __restrict__ v_out,
                                                                 float* __restrict__ p,
@@ -644,99 +730,290 @@ __device__ __attribute__((always_inline)) inline void reg_store(const RegTile<R>
                                                                 const RegArgs& a,
                                                                 const RegPlace& pl) {
   const int lane = reg_lane();
-  const int K = pl.K, W = sp.W, H = sp.H, P = sp.P;
+  const int W = sp.W, P = sp.P;
   const int gi = pl.gx0 + 2 * lane;
-  bool own0 = lc_in_tile(2 * lane, K, a.tw) && (unsigned)gi < (unsigned)W;
-  bool own1 = lc_in_tile(2 * lane + 1, K, a.tw) && (unsigned)(gi + 1) < (unsigned)W;
-  // RING: columns within 2K of the tile's left or right edge (pairs never
-  // straddle that bound: 2K and the tile width are even)
-  const int oc = 2 * lane - 2 * K;
-  const bool ring_col = oc < 2 * K || oc >= a.tw - 2 * K;
+  // the owned columns start and end at pairs, but for an odd W
+  const bool own0 = 2 * lane >= pl.c0 && 2 * lane < pl.c1;
+  const bool own1 = own0 && gi + 1 < W;
 #pragma unroll
   for (int rho = 0; rho < R; rho++) {
     const int r = pl.rbase + rho;
-    const int gj = pl.gy0 + r;
-    if (r < 2 * K || r >= 2 * K + a.th || gj >= H) continue;
-    bool s0 = own0, s1 = own1;
-    if constexpr (RING) {
-      const int orow = r - 2 * K;
-      const bool ring_row = orow < 2 * K || orow >= a.th - 2 * K;
-      s0 = s0 && (ring_row || ring_col);
-      s1 = s1 && (ring_row || ring_col);
+    if (r < pl.r0 || r >= pl.r1) continue;
+    const long row = (long)(pl.gy0 + r) * P;
+    const unsigned gk = (unsigned)gi;  // owned cells lie in the grid
+    store_pair(u_out + row, gk, own0, own1, own_register(t.u0[rho]), own_register(t.u1[rho]));
+    store_pair(v_out + row, gk, own0, own1, own_register(t.v0[rho]), own_register(t.v1[rho]));
+    if constexpr (PM != PM_NONE) {
+      if (own0) {
+        const uint32_t g = *reinterpret_cast<const uint16_t*>(gates + row + gk);
+        const bool upd0 = (g & G_UPD) != 0, upd1 = own1 && (g & (G_UPD << 8)) != 0;
+        if (upd0 || a.forces) p[row + gk] = upd0 ? t.s0[rho] : 0.0f;
+        if (upd1 || (own1 && a.forces)) p[row + gk + 1] = upd1 ? t.s1[rho] : 0.0f;
+      }
     }
-    const long gk = (long)gj * P + gi;
-    if constexpr (RING) {
-      coherent_store_pair(u_out, gk, s0, s1, t.u0[rho], t.u1[rho]);
-      coherent_store_pair(v_out, gk, s0, s1, t.v0[rho], t.v1[rho]);
-    } else {
-      store_pair(u_out, gk, s0, s1, t.u0[rho], t.u1[rho]);
-      store_pair(v_out, gk, s0, s1, t.v0[rho], t.v1[rho]);
-    }
-    if constexpr (PRESSURE && !RING) {
-      if (s0) p[gk] = t.s0[rho];
-      if (s1) p[gk + 1] = t.s1[rho];
-    }
-  }
-}
-
-// Reloads u and v of the halo (every register cell outside the owned tile)
-// from the neighbours' stored rings; the owned cells keep their registers.
-// Loads first (masked to the halo lanes), one wait, then cells outside the
-// grid are set to 0, as at the first load.
-template <typename T, int R>
-__device__ __attribute__((always_inline)) inline void reg_reload_halo(RegTile<R>& t,
-                                                                      const T* __restrict__ u_in,
-                                                                      const T* __restrict__ v_in,
-                                                                      const StepParams& sp,
-                                                                      const RegArgs& a,
-                                                                      const RegPlace& pl) {
-  const int lane = reg_lane();
-  const int K = pl.K, W = sp.W, H = sp.H, P = sp.P;
-  const int gi = pl.gx0 + 2 * lane;
-  const bool col0 = (unsigned)gi < (unsigned)W, col1 = (unsigned)(gi + 1) < (unsigned)W;
-  const bool halo_lane = lane < K || lane >= 64 - K;
-  const int gic = min(max(gi, 0), P - 2);
-  float nu0[R], nu1[R], nv0[R], nv1[R];
-#pragma unroll
-  for (int rho = 0; rho < R; rho++) {
-    const int r = pl.rbase + rho;
-    const bool halo_row = r < 2 * K || r >= 2 * K + a.th;
-    nu0[rho] = t.u0[rho];
-    nu1[rho] = t.u1[rho];
-    nv0[rho] = t.v0[rho];
-    nv1[rho] = t.v1[rho];
-    if (halo_row || halo_lane) {
-      const long k = (long)min(max(pl.gy0 + r, 0), H - 1) * P + gic;
-      coherent_load_pair(u_in, k, nu0[rho], nu1[rho]);
-      coherent_load_pair(v_in, k, nv0[rho], nv1[rho]);
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int rho = 0; rho < R; rho++) {
-    const int gj = pl.gy0 + pl.rbase + rho;
-    const bool row_in = (unsigned)gj < (unsigned)H;
-    const bool in0 = row_in && col0, in1 = row_in && col1;
-    t.u0[rho] = in0 ? nu0[rho] : 0.0f;
-    t.v0[rho] = in0 ? nv0[rho] : 0.0f;
-    t.u1[rho] = in1 ? nu1[rho] : 0.0f;
-    t.v1[rho] = in1 ? nv1[rho] : 0.0f;
   }
 }
 
 // One launch of the register-resident projection for tile `tile` (row-major
-// over the grid's ntx tiles per row), run by a workgroup of 64 * kRegWaves
-// threads.
-template <typename T, bool PRESSURE, int R, bool ONE_SYNC>
+// over the grid's ntx tiles per row), run by a workgroup of 64 * NW threads.
+// From the load on each kind of wavefront runs code of its own, with the same
+// barriers.
+template <typename T, int PM, int R, int NW, int KIND>
+__device__ __attribute__((always_inline)) inline void project_regs_kind(
+    RegTile<R>& t, const StepParams& sp, const uint8_t* __restrict__ gates, T* __restrict__ u_out,
+    T* __restrict__ v_out, float* __restrict__ p, const RegArgs& a, const RegPlace& pl,
+    RegShared<NW>& sh) {
+  if constexpr (KIND == WK_ANY) reg_masks<R>(t);
+  const RowExchange x = reg_begin<R, NW>(t, sh, pl.w, reg_lane());
+  reg_sweeps<T, PM, R, NW, KIND>(t, sh, x, sp, pl, a.sweeps);
+  reg_store<T, PM, R>(t, gates, u_out, v_out, p, sp, a, pl);
+}
+
+template <typename T, int PM, int R, int NW>
 __device__ __attribute__((always_inline)) inline void project_regs_tile(
     const StepParams& sp, const uint8_t* __restrict__ gates, const T* __restrict__ u_in,
     const T* __restrict__ v_in, T* __restrict__ u_out, T* __restrict__ v_out,
-    float* __restrict__ p, const RegArgs& a, int tile, RegShared& sh) {
-  const RegPlace pl = reg_place<R>(a, tile);
+    float* __restrict__ p, const RegArgs& a, int tile, RegShared<NW>& sh) {
+  const RegPlace pl = reg_place<R, NW>(a, tile, sp.W, sp.H);
   RegTile<R> t;
-  reg_load<T, PRESSURE, R>(t, sp, gates, u_in, v_in, p, a, pl);
-  reg_sweeps<T, PRESSURE, R, ONE_SYNC>(t, sh, sp, pl, a.th, a.sweeps);
-  reg_store<T, PRESSURE, R, false>(t, u_out, v_out, p, sp, a, pl);
+  reg_load<T, PM, R>(t, sp, gates, u_in, v_in, p, a, pl);
+  if (t.kind == WK_OPEN)
+    project_regs_kind<T, PM, R, NW, WK_OPEN>(t, sp, gates, u_out, v_out, p, a, pl, sh);
+  else if (t.kind == WK_WALL)
+    project_regs_kind<T, PM, R, NW, WK_WALL>(t, sp, gates, u_out, v_out, p, a, pl, sh);
+  else if (t.kind == WK_DRAIN)
+    project_regs_kind<T, PM, R, NW, WK_DRAIN>(t, sp, gates, u_out, v_out, p, a, pl, sh);
+  else if (t.kind == WK_DRAIN0)
+    project_regs_kind<T, PM, R, NW, WK_DRAIN0>(t, sp, gates, u_out, v_out, p, a, pl, sh);
+  else
+    project_regs_kind<T, PM, R, NW, WK_ANY>(t, sp, gates, u_out, v_out, p, a, pl, sh);
+}
+
+// ---- halo exchange of the resident kernel --------------------------------------
+//
+// Between stages a tile's halo comes from its neighbours through an exchange
+// buffer of three slots of 8-byte words, each a cell pair's values: in
+// binary32 one word (u0, u1) and one (v0, v1), in 16 bits one word for all
+// four.  A word is its own flag: a slot's words hold kNoWord until the owner
+// stores them and again once they have been read, so a reader polls the data
+// itself and one store and one load carry a value between two CUs (a
+// separate flag would add a wait for the stores, a barrier and a second
+// round trip).  Words are written and read with relaxed agent-scope atomics,
+// which bypass the caches that are not coherent between CUs and XCDs (a CU's
+// L1, an XCD's L2); each word is single-copy atomic, and no order between
+// words is needed.
+//
+// Ring t (the cells a tile's neighbours read before stage t) uses slot
+// (base + t) % 3; base is kept in device memory and moved on at the end of a
+// launch, so that the first rings of the next launch find clean slots.  A
+// tile clears ring t-1 once it has read all its neighbours' ring t: a
+// neighbour publishes ring t only after it has read ring t-1.  The clearing
+// stores have completed before the tile publishes ring t+1, and a neighbour
+// looks for ring t+2, the slot's next use, only after it has read ring t+1,
+// so it never takes an old word for a new one.  The last ring of a launch is
+// the one left to clear ("ring 0" of the next launch).
+//
+// A slot holds the region of every tile, a row of 64 words per region row
+// and word kind, so that a wavefront's rows lie at constant offsets from one
+// address (what bounds the exchange is instructions: the 16 wavefronts of a
+// tile issue all of it between two sweeps).  A tile stores its ring at its
+// own cells' places; a reader finds the cell that lies `d` tiles over in
+// that tile's region, tw / 2 pairs or th rows back.
+typedef unsigned long long XWord;
+constexpr XWord kNoWord = ~0ULL;  // by its low half
+constexpr int kXSlots = 3;
+
+// Words per cell pair.
+template <typename T> constexpr int xwords() { return sizeof(T) == 4 ? 2 : 1; }
+
+__device__ inline XWord xload(const XWord* a) {
+  return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void xstore(XWord* a, XWord w) {
+  __hip_atomic_store(a, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A pair's values as words.  A low half of all ones is a NaN with a full
+// payload (two in 16 bits); such a value travels with one payload bit
+// cleared.
+template <typename T>
+__device__ inline void pack_words(XWord* w, float u0, float u1, float v0, float v1) {
+  if constexpr (sizeof(T) == 4) {
+    w[0] = (XWord)__float_as_uint(u1) << 32 | min(__float_as_uint(u0), 0xFFFFFFFEu);
+    w[1] = (XWord)__float_as_uint(v1) << 32 | min(__float_as_uint(v0), 0xFFFFFFFEu);
+  } else {
+    const T e[4] = {Store<T>::st(u0), Store<T>::st(u1), Store<T>::st(v0), Store<T>::st(v1)};
+    uint32_t h[2];
+    __builtin_memcpy(h, e, 8);
+    w[0] = (XWord)h[1] << 32 | min(h[0], 0xFFFFFFFEu);
+  }
+}
+
+template <typename T>
+__device__ inline void unpack_words(const XWord* w, float& u0, float& u1, float& v0, float& v1) {
+  if constexpr (sizeof(T) == 4) {
+    u0 = __uint_as_float((uint32_t)w[0]);
+    u1 = __uint_as_float((uint32_t)(w[0] >> 32));
+    v0 = __uint_as_float((uint32_t)w[1]);
+    v1 = __uint_as_float((uint32_t)(w[1] >> 32));
+  } else {
+    T e[4];
+    __builtin_memcpy(e, w, 8);
+    u0 = Store<T>::ld(e[0]);
+    u1 = Store<T>::ld(e[1]);
+    v0 = Store<T>::ld(e[2]);
+    v1 = Store<T>::ld(e[3]);
+  }
+}
+
+// A tile's place in a slot, and what of this wavefront's rows takes part:
+// one bit per row, and the lanes of a row.  Worked out once; choosing a row's
+// lanes then takes a bit test.
+struct XPlace {
+  int tile, half;   // half: tw / 2
+  long tile_row;    // bytes from a word to that of the same cell seen from the
+                    // tile row above
+  unsigned own, ring;      // rows owned; rows of the ring, all owned lanes
+  unsigned below, above;   // halo rows owned by the tiles below and above
+  unsigned in;             // rows inside the grid
+  unsigned long long own_m, ring_m;  // owned lanes; those of the ring's strips
+  unsigned long long halo_m;         // lanes of the halo's strips
+};
+
+template <typename T, int R, int NW>
+__device__ inline XPlace x_place(const RegArgs& a, const RegPlace& pl, int tile) {
+  constexpr long kTile = (long)xwords<T>() * NW * R * 512;
+  XPlace x;
+  x.tile = tile;
+  x.half = a.tw / 2;
+  x.tile_row = a.ntx * kTile - (long)a.th * 512;
+  x.own = x.ring = x.below = x.above = x.in = 0;
+  const int K2 = 2 * pl.K;
+#pragma unroll
+  for (int rho = 0; rho < R; rho++) {
+    const int r = pl.rbase + rho;
+    const bool own = r >= pl.r0 && r < pl.r1;
+    x.own |= (own ? 1u : 0u) << rho;
+    x.ring |= (own && ((pl.below && r < pl.r0 + K2) || (pl.above && r >= pl.r1 - K2)) ? 1u : 0u)
+              << rho;
+    x.below |= (pl.below && r < pl.r0 ? 1u : 0u) << rho;
+    x.above |= (pl.above && r >= pl.r1 ? 1u : 0u) << rho;
+    x.in |= (r < pl.rows ? 1u : 0u) << rho;
+  }
+  const int lane = reg_lane(), c = 2 * lane;
+  const bool own = c >= pl.c0 && c < pl.c1;
+  x.own_m = __ballot(own);
+  x.ring_m = __ballot(own && ((pl.left && c < pl.c0 + K2) || (pl.right && c >= pl.c1 - K2)));
+  x.halo_m = __ballot((pl.left && lane < pl.K) || (pl.right && lane >= 64 - pl.K));
+  return x;
+}
+
+template <class Word>
+__device__ inline Word* x_at(Word* slot, unsigned bytes) {
+  return (Word*)((typename std::conditional<std::is_const<Word>::value, const char*, char*>::type)
+                     slot + bytes);
+}
+
+// Stores the tile's ring in `slot`: the owned cells within 2k of a side that
+// has a neighbour.  CLEAR stores kNoWord instead.
+template <typename T, int R, int NW, bool CLEAR>
+__device__ __attribute__((always_inline)) inline void ring_store(const RegTile<R>& t, XWord* slot,
+                                                                 const XPlace& x,
+                                                                 const RegPlace& pl) {
+  constexpr int NWD = xwords<T>();
+  constexpr unsigned kPlane = NW * R * 512u;  // bytes
+  const unsigned at = (unsigned)x.tile * (NWD * kPlane) + (unsigned)(pl.rbase * 64 + reg_lane()) * 8u;
+#pragma unroll
+  for (int rho = 0; rho < R; rho++) {
+    unsigned long long m = (x.ring >> rho) & 1u ? x.own_m : x.ring_m;
+    if (!((x.own >> rho) & 1u)) m = 0;
+    if (in_lanes(m)) {
+      XWord w[NWD];
+      if constexpr (!CLEAR) 
+        pack_words<T>(w, own_register(t.u0[rho]), own_register(t.u1[rho]),
+                      own_register(t.v0[rho]), own_register(t.v1[rho]));
+#pragma unroll
+      for (int i = 0; i < NWD; i++)
+        xstore(x_at(slot, at + i * kPlane) + rho * 64, CLEAR ? kNoWord : w[i]);
+    }
+  }
+}
+
+// Lanes of row rho that are halo, inside the grid.
+__device__ inline unsigned long long halo_lanes(const XPlace& x, int rho) {
+  const unsigned long long m =
+      ((x.below | x.above) >> rho) & 1u ? x.own_m | x.halo_m : x.halo_m;
+  return (x.in >> rho) & 1u ? m : 0ULL;
+}
+
+// Replaces u and v of the halo (the region's cells outside the owned ones,
+// inside the grid) by the neighbours' rings in `slot`, waiting for them.
+// Every load of a poll is issued before the first is looked at.  A wait ends
+// with the words, after spin_ticks of wall clock (the error word is set), or
+// as soon as another wait of the launch has timed out.
+template <typename T, int R, int NW>
+__device__ __attribute__((always_inline)) inline void ring_load(RegTile<R>& t, const XWord* slot,
+                                                                const XPlace& x,
+                                                                const RegPlace& pl, int* error,
+                                                                long long spin_ticks) {
+  constexpr int NWD = xwords<T>();
+  constexpr unsigned kPlane = NW * R * 512u;  // bytes
+  const int lane = reg_lane();
+  const int dx = pl.left && lane < pl.K ? -1 : pl.right && lane >= 64 - pl.K ? 1 : 0;
+  unsigned at = (unsigned)(x.tile + dx) * (NWD * kPlane) +
+                (unsigned)(pl.rbase * 64 + lane - dx * x.half) * 8u;
+  // where the tiles below and above have this wavefront's rows
+  const XWord* lo = (const XWord*)((const char*)slot - x.tile_row);
+  const XWord* hi = (const XWord*)((const char*)slot + x.tile_row);
+  const long long t0 = wall_clock64();
+  // at most six rows at a time, so that their words do not spill
+  constexpr int kRows = R <= 6 ? R : (R + 1) / 2;
+#pragma unroll
+  for (int r0 = 0; r0 < R; r0 += kRows) {
+    XWord w[kRows][NWD];
+#pragma unroll
+    for (int i = 0; i < kRows * NWD; i++) w[i / NWD][i % NWD] = 0;
+    // poll one row until it is there, then all: the others mostly are, too
+    for (int first = kRows - 1;;) {
+      uint32_t most = 0;
+      asm volatile("" : "+v"(at));  // no address per row kept across polls
+#pragma unroll
+      for (int q = 0; q < kRows; q++) {
+        const int rho = r0 + q;
+        if (q < first || rho >= R) continue;
+        const XWord* from = (x.below >> rho) & 1u ? lo : (x.above >> rho) & 1u ? hi : slot;
+        if (in_lanes(halo_lanes(x, rho)))
+#pragma unroll
+          for (int i = 0; i < NWD; i++) w[q][i] = xload(x_at(from, at + i * kPlane) + rho * 64);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kRows * NWD; i++) most = max(most, (uint32_t)w[i / NWD][i % NWD]);
+      if (!__any(most == (uint32_t)kNoWord)) {
+        if (first == 0) break;
+        first = 0;
+        continue;
+      }
+      if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
+      if (wall_clock64() - t0 > spin_ticks) {
+        __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+#pragma unroll
+    for (int q = 0; q < kRows; q++) {
+      const int rho = r0 + q;
+      if (rho >= R) continue;
+      const bool halo = in_lanes(halo_lanes(x, rho));
+      float u0, u1, v0, v1;
+      unpack_words<T>(w[q], u0, u1, v0, v1);
+      t.u0[rho] = halo ? u0 : t.u0[rho];
+      t.u1[rho] = halo ? u1 : t.u1[rho];
+      t.v0[rho] = halo ? v0 : t.v0[rho];
+      t.v1[rho] = halo ? v1 : t.v1[rho];
+    }
+  }
 }
 
 }  // namespace osy
