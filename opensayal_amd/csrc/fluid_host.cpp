@@ -92,17 +92,51 @@ BlockLayout block_layout(int W, int H, int storage) {
   return L;
 }
 
-// Starting launch shape before any autotuning: the register-resident
-// kernel with 8 rows per wavefront and 5 sweeps per launch (a 128 x 64
-// region owning 108 x 44 cells), the fastest measured at 1920 x 1080.
-ProjTuning default_tuning(int W, bool pressure) {
-  (void)W;
+// Launch shape before any autotuning: a register kernel whose region and
+// sweeps per launch k follow the grid.  While the tiles fit the CUs once, a
+// launch takes a fixed 4 to 7 us and 0.25 us (regions of 32 rows) to 0.65 us
+// (128 rows) per phase however many tiles there are, so the smallest region
+// that fits with a large k is the fastest: 50 sweeps of 256 x 144 take 60 us
+// at 32 rows and k = 7, 106 us at 64 rows and k = 5; 50 of 1280 x 720 86 us
+// at 96 rows and k = 12, 118 us at 64 rows and k = 5.  Below the k given for
+// a height the next height was faster (640 x 480: 75 us at 32 rows and k = 5
+// against 79 us at 64 and k = 10; 1001 x 563, n = 100: at k = 3 190 us against
+// 162 us).  In 16 bits and with pressure sums, where a phase is dearer, two and
+// three tiles of 32 rows to a CU still win (1001 x 563, n = 100, in bfloat16:
+// 192 us against 205 us at 64 rows; 1280 x 720 with pressure: 135 us against
+// 145 us).  Pressure sums need too many registers for more than 64 rows; two
+// such tiles run on a CU at once (1024 x 1024 with pressure: 145 us at k = 10,
+// 176 us at k = 5).  Larger grids are bound by the work and the memory of all
+// their tiles: 64 rows and k = 6, or 5 in 16 bits, where a row's rounding
+// makes the halo dearer (3840 x 2160: 369 us at k = 6, 384 us at k = 5; 498 and
+// 471 us in bfloat16).
+ProjTuning default_tuning(int W, int H, int n, bool pressure, int storage, int cus) {
+  enum { F32 = 1, HALF = 2, PRESSURE = 4 };  // binary32, 16 bits, either with sums
+  struct Height {
+    int rows, k_most, k_least, per_cu, of;
+  };
+  static constexpr Height heights[] = {
+      {4, 7, 5, 1, F32 | HALF | PRESSURE}, {4, 5, 5, 2, HALF},  {4, 5, 5, 3, PRESSURE},
+      {8, 10, 8, 1, F32 | HALF | PRESSURE}, {12, 14, 5, 1, F32 | HALF},
+      {16, 12, 6, 1, F32 | HALF},           {8, 10, 5, 2, PRESSURE}};
+  const int of = pressure ? PRESSURE : storage == OSY_STORAGE_F32 ? F32 : HALF;
   ProjTuning t;
   t.kernel = PROJ_REGS;
-  t.k = 5;
-  t.tw = 128 - 4 * t.k;
-  t.th = 8 * kRegWaves - 4 * t.k;
-  if (!t.valid(pressure)) t.kernel = PROJ_COLOUR;
+  auto shape = [&t](int rows, int k) {
+    t.k = k;
+    t.tw = 128 - 4 * k;
+    t.th = 8 * rows - 4 * k;
+  };
+  // as many sweeps in each of the launches that k makes of n
+  auto even = [n](int k) { return n > 0 ? (n + (n + k - 1) / k - 1) / ((n + k - 1) / k) : k; };
+  for (const Height& h : heights) {
+    if (!(h.of & of)) continue;
+    for (int k = h.k_most; k >= h.k_least; k--) {
+      shape(h.rows, even(k));
+      if (t.tiles(W, H) <= h.per_cu * cus) return t;
+    }
+  }
+  shape(8, even(storage == OSY_STORAGE_F32 ? 6 : 5));
   return t;
 }
 
@@ -124,7 +158,6 @@ int create_impl(const osy_config* cfg, osy_fluid** out) {
   fl->cs = (int)cfg->cell_size;
   fl->storage = cfg->storage;
   fl->elem = cfg->storage == OSY_STORAGE_F32 ? 4 : 2;
-  fl->tuning = default_tuning(fl->W, cfg->enable_pressure != 0);
   hipError_t e = hipGetDevice(&fl->device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&fl->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -142,6 +175,8 @@ int create_impl(const osy_config* cfg, osy_fluid** out) {
     delete fl;
     return set_error(OSY_E_HIP, std::string("device attribute: ") + hipGetErrorString(e));
   }
+  fl->tuning = default_tuning(fl->W, fl->H, cfg->projection_n, cfg->enable_pressure != 0,
+                              fl->storage, fl->cus);
   fl->wall_khz = khz > 0 ? khz : 100000;
   fl->spin_ticks = (long long)fl->wall_khz * 2000;  // 2 s
   fl->block_bytes = L.total();
