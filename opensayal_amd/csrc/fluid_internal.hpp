@@ -47,7 +47,7 @@ struct osy_fluid {
     hipGraphExec_t exec = nullptr;
     float d_t = 0.0f;
     int uv_out = 0, sm_out = 0;
-  } graphs[2][2];
+  } graphs[4][2];  // by buffer parity; [2..3]: kGraphSteps steps in one graph
 
   ~osy_fluid() {
     for (auto& row : graphs)
