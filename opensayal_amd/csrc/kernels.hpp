@@ -41,6 +41,7 @@ struct StepParams {
   // and the divisor 1 + 4a, both in float as the reference computes them
   int visc_on;
   float visc_a, visc_den;
+  double visc_recip;  // 1 / visc_den for 0 < |visc_den| < 2, else 0 (PressureDivisor)
   // set by the step: the first projection launch applies the velocity
   // forces to what it loads and starts the pressure sums at 0
   int forces_in_projection;

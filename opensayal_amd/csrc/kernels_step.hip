@@ -188,107 +188,175 @@ __global__ void __launch_bounds__(64 * kAdvNY)
 // ---- P2b: apply_diffusion (src/fluid.cu:167-190) as Jacobi rounds -------
 // Every interior cell (1 <= i <= W-2, 1 <= j <= H-2, solid or not) becomes
 // (u + a*(((u(i-1,j) + u(i+1,j)) + u(i,j-1)) + u(i,j+1))) / (1 + 4a) of the
-// previous round's u; borders keep theirs; v is not diffused.  A launch runs
-// up to kDiffHalo rounds on a 128 x 64 region (the owned tile plus a
-// kDiffHalo-cell halo) staged in LDS, two buffers in turn: a value at region
-// distance d from the region edge is exact for d rounds, so the owned tile
-// is exact after kDiffHalo rounds.  Eight wavefronts take the region's rows
-// in turn, each lane two columns 64 apart, so the 126 updated columns fill
-// 126 of 128 lanes.  u goes from u_in to u_out; with copy_v the launch also
-// moves v to v_out so that u and v stay in the same buffer of their pairs.
-constexpr int kDiffRX = 128, kDiffRY = 64, kDiffHalo = 6;
-static_assert(kDiffRY % 8 == 0, "eight wavefronts take the region's rows in turn");
-constexpr int kDiffTX = kDiffRX - 2 * kDiffHalo, kDiffTY = kDiffRY - 2 * kDiffHalo;
+// previous round's u; borders keep theirs; v is not diffused.
+//
+// The tiles and registers are the register projection's (projection_device.hpp):
+// NW wavefronts of R rows, lane l holds cells 2l and 2l+1 of each, and a
+// launch runs up to 2k rounds on a tile with a halo of 2k cells, since a
+// round moves a stale value one cell.  Left and right come from the lane's
+// other cell and by a lane shift, below and above from the lane's other
+// rows, and at the wavefront's first and last row through LDS, with one
+// barrier per round; the rows inside are computed first, which hides that.
+// What bounds it is the issue of vector instructions, so the quotient goes
+// through the double reciprocal of the divisor where that is exact
+// (PressureDivisor), and only wavefronts that hold border cells select.
+// 50 rounds of 1920 x 1080 take 78 us (5 launches of 15.6 us); with the region
+// in LDS they took 175 us (9 launches of 19.4 us: six reads and writes of LDS
+// and a division per cell and round).
+template <int NW>
+struct DiffShared {
+  float2 first[2][NW][64], last[2][NW][64];  // rows 0 and R-1 of each wavefront
+};
 
-template <typename T>
-__global__ void __launch_bounds__(512)
-    k_diffuse(StepParams sp, int rounds, const T* __restrict__ u_in, T* __restrict__ u_out,
-              const T* __restrict__ v_in, T* __restrict__ v_out, int copy_v, int ntx) {
-  __shared__ float buf[2][kDiffRY * kDiffRX];
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int x0 = (tile % ntx) * kDiffTX - kDiffHalo, y0 = (tile / ntx) * kDiffTY - kDiffHalo;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  // stage the region: every load of the thread (from the cell clamped into
-  // the grid, so with no branch) before its first LDS write, so a wavefront
-  // waits for HBM once rather than once per row; cells outside the grid
-  // hold 0
-  constexpr int kRowsPerWave = kDiffRY / 8;
-  float staged[kRowsPerWave][2];
+template <typename T, bool RECIP>
+__device__ inline float diffused(float x, float sum, float a, float den, double recip) {
+  const float y = x + a * sum;
+  return rnd<T>(RECIP ? (float)((double)y * recip) : y / den);
+}
+
+// One round of a wavefront's rows.  EDGE: cells outside `cols0`, `cols1`
+// (even, odd cells) and rows outside [j_lo, j_hi) keep their values.
+template <typename T, int R, bool RECIP, bool EDGE>
+__device__ __attribute__((always_inline)) inline void diffuse_rows(
+    float (&x0)[R], float (&x1)[R], const float2& below, const float2& above,
+    const StepParams& sp, unsigned long long cols0, unsigned long long cols1, int j_lo, int j_hi) {
+  float n0[R], n1[R];
 #pragma unroll
-  for (int m = 0; m < kRowsPerWave; m++) {
-    const int j = min(max(y0 + wave + 8 * m, 0), sp.H - 1);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int i = min(max(x0 + lane + 64 * h, 0), sp.W - 1);
-      staged[m][h] = ldf(u_in, (long)j * sp.P + i);
+  for (int q = 0; q < R; q++) {
+    const int rho = q + 1 < R - 1 ? q + 1 : q + 1 == R - 1 ? 0 : R - 1;  // inner rows first
+    const float b0 = rho > 0 ? x0[rho > 0 ? rho - 1 : 0] : below.x;
+    const float b1 = rho > 0 ? x1[rho > 0 ? rho - 1 : 0] : below.y;
+    const float t0 = rho + 1 < R ? x0[rho + 1 < R ? rho + 1 : rho] : above.x;
+    const float t1 = rho + 1 < R ? x1[rho + 1 < R ? rho + 1 : rho] : above.y;
+    const float s0 = ((lane_from_left(x1[rho]) + x1[rho]) + b0) + t0;
+    const float s1 = ((x0[rho] + lane_from_right(x0[rho])) + b1) + t1;
+    n0[rho] = diffused<T, RECIP>(x0[rho], s0, sp.visc_a, sp.visc_den, sp.visc_recip);
+    n1[rho] = diffused<T, RECIP>(x1[rho], s1, sp.visc_a, sp.visc_den, sp.visc_recip);
+    if constexpr (EDGE) {
+      const bool row = rho >= j_lo && rho < j_hi;
+      n0[rho] = in_lanes(row ? cols0 : 0ULL) ? n0[rho] : x0[rho];
+      n1[rho] = in_lanes(row ? cols1 : 0ULL) ? n1[rho] : x1[rho];
     }
   }
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int m = 0; m < kRowsPerWave; m++) {
-    const int r = wave + 8 * m, j = y0 + r;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int c = lane + 64 * h, i = x0 + c;
-      const bool in = (unsigned)i < (unsigned)sp.W && (unsigned)j < (unsigned)sp.H;
-      const float x = in ? staged[m][h] : 0.0f;
-      buf[0][r * kDiffRX + c] = x;
-      buf[1][r * kDiffRX + c] = x;
-    }
+  for (int rho = 0; rho < R; rho++) {
+    x0[rho] = n0[rho];
+    x1[rho] = n1[rho];
   }
-  __syncthreads();
-  const float a = sp.visc_a, den = sp.visc_den;
-  // columns 1 + lane and 65 + lane (the second only for lanes 0..61)
-  const int c0 = 1 + lane, c1 = 65 + lane;
-  const bool in0 = x0 + c0 >= 1 && x0 + c0 <= sp.W - 2;
-  const bool in1 = c1 < kDiffRX - 1 && x0 + c1 >= 1 && x0 + c1 <= sp.W - 2;
+}
+
+template <typename T, int R, int NW, bool RECIP, bool EDGE>
+__device__ __attribute__((always_inline)) inline void diffuse_rounds(
+    float (&x0)[R], float (&x1)[R], DiffShared<NW>& sh, const StepParams& sp, int w, int rounds,
+    int active, unsigned long long cols0, unsigned long long cols1, int j_lo, int j_hi) {
+  const int lane = reg_lane();
   for (int it = 0; it < rounds; it++) {
-    const float* src = buf[it & 1];
-    float* dst = buf[(it & 1) ^ 1];
-#pragma unroll
-    for (int m = 0; m < kRowsPerWave; m++) {
-      const int r = 1 + wave + 8 * m, j = y0 + r;
-      if (r >= kDiffRY - 1 || j < 1 || j > sp.H - 2) continue;
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        if (!(h ? in1 : in0)) continue;
-        const int l = r * kDiffRX + (h ? c1 : c0);
-        const float sum = ((src[l - 1] + src[l + 1]) + src[l - kDiffRX]) + src[l + kDiffRX];
-        dst[l] = rnd<T>((src[l] + a * sum) / den);
-      }
-    }
+    const int slot = it & 1;
+    sh.first[slot][w][lane] = make_float2(x0[0], x1[0]);
+    sh.last[slot][w][lane] = make_float2(x0[R - 1], x1[R - 1]);
     __syncthreads();
-  }
-  const float* res = buf[rounds & 1];
-  for (int r = kDiffHalo + wave; r < kDiffHalo + kDiffTY; r += 8) {
-    const int j = y0 + r;
-    if (j >= sp.H) break;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int c = kDiffHalo + lane + 64 * h, i = x0 + c;
-      if (c >= kDiffHalo + kDiffTX || i >= sp.W) continue;
-      const long k = (long)j * sp.P + i;
-      stf(u_out, k, res[r * kDiffRX + c]);
-      if (copy_v) v_out[k] = v_in[k];
+    // (a slot is written again two rounds on, after the barrier between)
+    if (it < active) {
+      const float2 below = sh.last[slot][max(w - 1, 0)][lane];
+      const float2 above = sh.first[slot][min(w + 1, NW - 1)][lane];
+      diffuse_rows<T, R, RECIP, EDGE>(x0, x1, below, above, sp, cols0, cols1, j_lo, j_hi);
     }
   }
 }
 
-// `sp.n` rounds in ceil(n / kDiffHalo) launches; advances *uv by the launch
-// count (v moves with u on the last launch when that count is odd).
+// u goes from u_in to u_out; with copy_v the launch also moves v to v_out so
+// that u and v stay in the same buffer of their pairs.
+template <typename T, int R, int NW, bool RECIP>
+__global__ void __launch_bounds__(64 * NW, NW / 2)
+    k_diffuse(StepParams sp, const T* __restrict__ u_in, T* __restrict__ u_out,
+              const T* __restrict__ v_in, T* __restrict__ v_out, int copy_v, RegArgs a) {
+  __shared__ DiffShared<NW> sh;
+  const RegPlace pl = reg_place<R, NW>(a, xcd_tile(blockIdx.x, gridDim.x), sp.W, sp.H);
+  const int lane = reg_lane(), W = sp.W, H = sp.H, P = sp.P;
+  const int gi = pl.gx0 + 2 * lane;
+  // every load first, from the pair clamped into the row and the row clamped
+  // into the grid
+  const unsigned gic = (unsigned)min(gi, P - 2);
+  float x0[R], x1[R];
+#pragma unroll
+  for (int rho = 0; rho < R; rho++) {
+    const long row = (long)min(pl.gy0 + pl.rbase + rho, H - 1) * P;
+    load_pair(u_in + row, gic, true, true, x0[rho], x1[rho]);
+  }
+  const bool own0 = 2 * lane >= pl.c0 && 2 * lane < pl.c1;
+  const bool own1 = own0 && gi + 1 < W;
+  if (copy_v) {
+#pragma unroll
+    for (int rho = 0; rho < R; rho++) {
+      const int r = pl.rbase + rho;
+      if (r < pl.r0 || r >= pl.r1) continue;
+      const long row = (long)(pl.gy0 + r) * P;
+      float v0, v1;
+      load_pair(v_in + row, gic, true, true, v0, v1);
+      store_pair(v_out + row, (unsigned)gi, own0, own1, v0, v1);
+    }
+  }
+  // cells that are updated: lanes, and rows [j_lo, j_hi) of the wavefront
+  const unsigned long long cols0 = __ballot(gi >= 1 && gi <= W - 2);
+  const unsigned long long cols1 = __ballot(gi + 1 <= W - 2);
+  const int y = pl.gy0 + pl.rbase;
+  const int j_lo = max(1 - y, 0), j_hi = min(H - 1 - y, R);
+  // rounds in which some row can still reach the tile's own
+  const int idle = max(max(pl.r0 - pl.rbase - R, pl.rbase - pl.r1) + 1, 0);
+  const int active = a.sweeps - idle;
+  if ((cols0 & cols1) == ~0ULL && j_lo == 0 && j_hi == R)
+    diffuse_rounds<T, R, NW, RECIP, false>(x0, x1, sh, sp, pl.w, a.sweeps, active, cols0, cols1,
+                                           j_lo, j_hi);
+  else
+    diffuse_rounds<T, R, NW, RECIP, true>(x0, x1, sh, sp, pl.w, a.sweeps, active, cols0, cols1,
+                                          j_lo, j_hi);
+#pragma unroll
+  for (int rho = 0; rho < R; rho++) {
+    const int r = pl.rbase + rho;
+    if (r < pl.r0 || r >= pl.r1) continue;
+    store_pair(u_out + (long)(pl.gy0 + r) * P, (unsigned)gi, own0, own1, x0[rho], x1[rho]);
+  }
+}
+
+// `sp.n` rounds in launches of 2k; advances *uv by the launch count (v moves
+// with u on the last launch when that count is odd).  Regions of 32 rows
+// while their tiles fit the CUs once, else of 96 (kernel's figures above).
 template <typename T>
 void enqueue_diffusion(const StepParams& sp, const FieldPtrs& f, int* uv, hipStream_t s) {
   if (sp.n <= 0) return;
-  const int ntx = (sp.W + kDiffTX - 1) / kDiffTX, nty = (sp.H + kDiffTY - 1) / kDiffTY;
-  const int launches = (sp.n + kDiffHalo - 1) / kDiffHalo;
+  ProjTuning t;
+  bool low = false;
+  auto fits = [&](int rows, int k_most, int k_least) {
+    for (t.k = k_most; t.k >= k_least; t.k--) {
+      t.tw = 128 - 4 * t.k;
+      t.th = 8 * rows - 4 * t.k;
+      if (t.tiles(sp.W, sp.H) <= sp.cus) return true;
+    }
+    return false;
+  };
+  low = fits(4, 6, 4);
+  if (!low && !fits(12, 12, 5)) {
+    t.k = 5;
+    t.tw = 128 - 4 * t.k;
+    t.th = 96 - 4 * t.k;
+  }
+  RegArgs a{};
+  a.tw = t.tw;
+  a.th = t.th;
+  a.k = t.k;
+  a.ntx = t.tiles_x(sp.W);
+  a.nty = t.tiles_y(sp.H);
+  const int launches = (sp.n + 2 * t.k - 1) / (2 * t.k);
   int cur = *uv;
   for (int q = 0; q < launches; q++) {
-    const int rounds = q + 1 < launches ? kDiffHalo : sp.n - kDiffHalo * (launches - 1);
+    a.sweeps = min(2 * t.k, sp.n - 2 * t.k * q);
     const int copy_v = (q + 1 == launches) && (launches & 1);
-    hipLaunchKernelGGL(k_diffuse<T>, dim3(ntx * nty), dim3(512), 0, s, sp, rounds,
-                       (const T*)f.u[cur], (T*)f.u[1 - cur], (const T*)f.v[cur],
-                       (T*)f.v[1 - cur], copy_v, ntx);
+    const dim3 grid(a.ntx * a.nty), block(low ? 512 : 1024);
+    auto* kernel = low ? (sp.visc_recip != 0.0 ? k_diffuse<T, 4, 8, true> : k_diffuse<T, 4, 8, false>)
+                       : (sp.visc_recip != 0.0 ? k_diffuse<T, 6, 16, true>
+                                               : k_diffuse<T, 6, 16, false>);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, sp, (const T*)f.u[cur], (T*)f.u[1 - cur],
+                       (const T*)f.v[cur], (T*)f.v[1 - cur], copy_v, a);
     cur = 1 - cur;
   }
   *uv = cur;

@@ -110,3 +110,23 @@ def test_batch_refuses_diffusing_members():
         with pytest.raises(OpenSayalError) as e:
             b.add(Fluid(make_config(64, 36, viscosity=0.001)))
         assert "viscosity" in str(e.value)
+
+
+@pytest.mark.parametrize("W,H,n", [(3, 3, 4), (128, 32, 13), (129, 33, 12), (128, 96, 25),
+                                   (701, 613, 11), (1301, 1099, 21), (2101, 1203, 11)])
+@pytest.mark.parametrize("viscosity,storage", [(0.001, 0), (6.0, 0), (-9.0, 1), (0.3, 2)])
+def test_diffusion_tiles_match_oracle(W, H, n, viscosity, storage):
+    """One tile, one cell more, both region heights and more tiles than CUs;
+    divisors below 2 (a double reciprocal), of 2.2 (a division) and negative,
+    where binary16 can overflow (IEEE 754 leaves a NaN's sign open: any NaN
+    stands for any other)."""
+    cfg = make_config(W, H, projection_n=n, viscosity=viscosity, storage=storage, wind_speed=0.5,
+                      obstacle_enable=0)
+    fl, o = pair(cfg, 23)
+    fl.update()
+    o.update()
+    for name, attr in (("vel_x", "u"), ("vel_y", "v"), ("smoke", "smoke")):
+        got, want = fl.get_field(name), np.asarray(getattr(o, attr), np.float32)
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got), nan), name
+        assert same(np.where(nan, np.float32(0), got), np.where(nan, np.float32(0), want)), name
