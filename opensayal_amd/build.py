@@ -28,6 +28,7 @@ CXX = os.environ.get("CXX", "g++")
 SOURCES = [
     "json_value.cpp",
     "config.cpp",
+    "staging.cpp",
     "fluid_host.cpp",
     "batch_host.cpp",
     "kernels_step.hip",

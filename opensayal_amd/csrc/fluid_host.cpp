@@ -294,6 +294,39 @@ int adopt_tuning(osy_fluid* fl, const ProjTuning& t) {
   return OSY_OK;
 }
 
+// bytes of device memory to host memory, complete on return.
+int copy_back(osy_fluid* fl, void* dst, const void* src, size_t bytes) {
+  StagingLease pinned(fl->device, dst);
+  if (pinned) {
+    OSY_HIP_CHECK(pinned.copy_out(dst, src, bytes, fl->stream));
+    return OSY_OK;
+  }
+  OSY_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, fl->stream));
+  OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+  return OSY_OK;
+}
+
+// Launches `make` to write W*H 4-byte values and brings them to dst: small
+// results are written to pinned memory by the kernel, larger ones to the
+// handle's device staging buffer and copied from there.
+template <class Make>
+int copy_result(osy_fluid* fl, void* dst, size_t bytes, const Make& make) {
+  if (bytes <= kStagingDirect) {
+    StagingLease pinned(fl->device, dst);
+    if (pinned) {
+      make((float*)pinned.slot());
+      const hipError_t e = hipGetLastError();
+      OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+      OSY_HIP_CHECK(e);
+      std::memcpy(dst, pinned.slot(), bytes);
+      return OSY_OK;
+    }
+  }
+  make(fl->staging);
+  OSY_HIP_CHECK(hipGetLastError());
+  return copy_back(fl, dst, fl->staging, bytes);
+}
+
 int field_elem_ok(int field) { return field >= OSY_FIELD_VEL_X && field <= OSY_FIELD_TOTAL_S; }
 
 }  // namespace
@@ -467,11 +500,10 @@ int osy_fluid_get_field(osy_fluid* fl, int32_t field, void* dst, size_t bytes) {
     return set_error(OSY_E_INVALID, "buffer must hold width*height 4-byte elements");
   if (int st = batch_wait(fl)) return st;
   StepParams sp = fl->params(fl->cfg.d_t, nullptr);
-  enqueue_export(field, fl->storage, sp, fl->f, fl->uv, fl->sm, fl->staging, fl->stream);
-  OSY_HIP_CHECK(hipGetLastError());
-  OSY_HIP_CHECK(hipMemcpyAsync(dst, fl->staging, bytes, hipMemcpyDeviceToHost, fl->stream));
-  OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
-  return fluid_check_error(fl);
+  int st = copy_result(fl, dst, bytes, [&](float* to) {
+    enqueue_export(field, fl->storage, sp, fl->f, fl->uv, fl->sm, to, fl->stream);
+  });
+  return st == OSY_OK ? fluid_check_error(fl) : st;
 }
 
 int osy_fluid_set_field(osy_fluid* fl, int32_t field, const void* src, size_t bytes) {
@@ -482,10 +514,17 @@ int osy_fluid_set_field(osy_fluid* fl, int32_t field, const void* src, size_t by
   if (bytes != (size_t)fl->W * fl->H * 4)
     return set_error(OSY_E_INVALID, "buffer must hold width*height 4-byte elements");
   if (int st = batch_wait(fl)) return st;
-  OSY_HIP_CHECK(hipMemcpyAsync(fl->staging, src, bytes, hipMemcpyHostToDevice, fl->stream));
+  StagingLease pinned(fl->device, bytes <= kStagingDirect ? src : nullptr);
+  float* from = fl->staging;
+  if (pinned)
+    from = (float*)std::memcpy(pinned.slot(), src, bytes);
+  else  // (the runtime brings larger fields over as fast)
+    OSY_HIP_CHECK(hipMemcpyAsync(fl->staging, src, bytes, hipMemcpyHostToDevice, fl->stream));
   StepParams sp = fl->params(fl->cfg.d_t, nullptr);
-  enqueue_import(field, fl->storage, sp, fl->f, fl->uv, fl->sm, fl->staging, fl->stream);
-  OSY_HIP_CHECK(hipGetLastError());
+  enqueue_import(field, fl->storage, sp, fl->f, fl->uv, fl->sm, from, fl->stream);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) (void)hipStreamSynchronize(fl->stream);  // before the slot goes back
+  OSY_HIP_CHECK(e);
   OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
   return OSY_OK;
 }
@@ -517,12 +556,11 @@ int osy_fluid_render_rgba(osy_fluid* fl, uint32_t* dst, size_t bytes) {
     enqueue_pressure_range(sp, fl->f, fl->stream);
     OSY_HIP_CHECK(hipGetLastError());
   }
-  enqueue_render(fl->storage, sp, fl->f, fl->sm, fl->cfg.enable_pressure != 0,
-                 fl->cfg.enable_smoke != 0, (uint32_t*)fl->staging, fl->stream);
-  OSY_HIP_CHECK(hipGetLastError());
-  OSY_HIP_CHECK(hipMemcpyAsync(dst, fl->staging, bytes, hipMemcpyDeviceToHost, fl->stream));
-  OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
-  return fluid_check_error(fl);
+  int st = copy_result(fl, dst, bytes, [&](float* to) {
+    enqueue_render(fl->storage, sp, fl->f, fl->sm, fl->cfg.enable_pressure != 0,
+                   fl->cfg.enable_smoke != 0, (uint32_t*)to, fl->stream);
+  });
+  return st == OSY_OK ? fluid_check_error(fl) : st;
 }
 
 int osy_fluid_traces(osy_fluid* fl, int32_t distance, int32_t length, float d_t,
@@ -539,23 +577,22 @@ int osy_fluid_traces(osy_fluid* fl, int32_t distance, int32_t length, float d_t,
                      "each buffer must hold (W/distance)*(H/distance)*length int32 entries");
   if (each == 0) return OSY_OK;
   if (int st = batch_wait(fl)) return st;
-  if (fl->trace_cap < 2 * each) {
+  const size_t room = align_up(each, 256);
+  if (fl->trace_cap < 2 * room) {
     OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
     if (fl->trace_buf) OSY_HIP_CHECK(hipFree(fl->trace_buf));
     fl->trace_buf = nullptr;
     fl->trace_cap = 0;
-    OSY_HIP_CHECK(hipMalloc(&fl->trace_buf, 2 * each));
-    fl->trace_cap = 2 * each;
+    OSY_HIP_CHECK(hipMalloc(&fl->trace_buf, 2 * room));
+    fl->trace_cap = 2 * room;
   }
   int32_t* dx = (int32_t*)fl->trace_buf;
-  int32_t* dy = dx + each / 4;
+  int32_t* dy = dx + room / 4;
   const StepParams sp = fl->params(d_t, nullptr);
   enqueue_traces(fl->storage, sp, fl->f, fl->uv, distance, length, d_t, dx, dy, fl->stream);
   OSY_HIP_CHECK(hipGetLastError());
-  OSY_HIP_CHECK(hipMemcpyAsync(traces_x, dx, each, hipMemcpyDeviceToHost, fl->stream));
-  OSY_HIP_CHECK(hipMemcpyAsync(traces_y, dy, each, hipMemcpyDeviceToHost, fl->stream));
-  OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
-  return OSY_OK;
+  if (int st = copy_back(fl, traces_x, dx, each)) return st;
+  return copy_back(fl, traces_y, dy, each);
 }
 
 int osy_fluid_divergence_norm(osy_fluid* fl, double* l2, double* linf) {

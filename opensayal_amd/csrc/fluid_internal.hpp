@@ -10,6 +10,7 @@
 
 #include "kernels.hpp"
 #include "osy_internal.hpp"
+#include "staging.hpp"
 
 #define OSY_HIP_CHECK(call)                                                              \
   do {                                                                                   \
@@ -49,6 +50,7 @@ struct osy_fluid {
     int uv_out = 0, sm_out = 0;
   } graphs[4][2];  // by buffer parity; [2..3]: kGraphSteps steps in one graph
 
+  osy_fluid() { osy::staging_retain(); }
   ~osy_fluid() {
     for (auto& row : graphs)
       for (auto& g : row)
@@ -57,6 +59,7 @@ struct osy_fluid {
     if (trace_buf) (void)hipFree(trace_buf);
     if (exchange) (void)hipFree(exchange);
     if (stream) (void)hipStreamDestroy(stream);
+    osy::staging_release();
   }
 
   // StepParams for this configuration and step size; `src` may be null.
