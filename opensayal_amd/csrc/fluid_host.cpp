@@ -236,8 +236,8 @@ int enqueue_eager(osy_fluid* fl, const osy_source* src, float d_t, hipStream_t s
 }
 
 // Steps recorded in one graph while at least as many are to run: between two
-// graphs the GPU waits 8 us (1920 x 1080) to 17 us (256 x 144, where the host
-// is not ahead), between the kernels of one it does not.
+// graphs the GPU waits for the next (20 steps of 256 x 144 take 1.73 ms with a
+// step per graph, 1.67 ms with four).
 constexpr int kGraphSteps = 4;
 
 int enqueue_graph_steps(osy_fluid* fl, int32_t steps, float d_t, hipStream_t s) {

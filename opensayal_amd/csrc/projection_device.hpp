@@ -929,7 +929,7 @@ __device__ __attribute__((always_inline)) inline void ring_store(const RegTile<R
     if (!((x.own >> rho) & 1u)) m = 0;
     if (in_lanes(m)) {
       XWord w[NWD];
-      if constexpr (!CLEAR) 
+      if constexpr (!CLEAR)
         pack_words<T>(w, own_register(t.u0[rho]), own_register(t.u1[rho]),
                       own_register(t.v0[rho]), own_register(t.v1[rho]));
 #pragma unroll
