@@ -86,7 +86,7 @@ BlockLayout block_layout(int W, int H, int storage) {
   L.f32 = align_up(cells * 4, 256);
   L.ref = align_up((size_t)W * H * 4, 256);
   L.flg = align_up(cells, 256);
-  L.red = align_up(sizeof(float) * (2 * kReduceBlocks + 2), 256);
+  L.red = align_up(sizeof(float) * (2 * kReduceBlocks + 3), 256);
   L.dred = align_up(sizeof(double) * (2 * kReduceBlocks + 2), 256);
   L.rsd = 256;  // resident projection: error word
   return L;
