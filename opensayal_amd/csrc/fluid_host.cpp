@@ -15,7 +15,6 @@
 
 #include "batch.hpp"
 #include "fluid_internal.hpp"
-#include "projection.hpp"
 
 namespace osy {
 
@@ -353,16 +352,16 @@ int fluid_clean_exchange(osy_fluid* fl, const ProjTuning& shape) {
   const size_t bytes =
       256 + 3 * 8 * t.exchange_words(fl->W, fl->H, (size_t)fl->elem);
   if (fl->exchange_bytes < bytes) {
-    OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
-    if (fl->exchange) OSY_HIP_CHECK(hipFree(fl->exchange));
-    fl->exchange = nullptr;
-    fl->exchange_bytes = 0;
-    hipError_t e = hipMalloc(&fl->exchange, bytes);
+    // the new memory first: without it the handle goes on with the old
+    void* mem = nullptr;
+    const hipError_t e = hipMalloc(&mem, bytes);
     if (e != hipSuccess) {
-      fl->exchange = nullptr;
+      (void)hipGetLastError();  // reported here, not by a later launch's check
       return set_error(OSY_E_NOMEM, "halo exchange of " + std::to_string(bytes) +
                                         " bytes: " + hipGetErrorString(e));
     }
+    if (fl->exchange) (void)hipFree(fl->exchange);  // waits for the launches that use it
+    fl->exchange = mem;
     fl->exchange_bytes = bytes;
     fl->f.rstate = (unsigned*)fl->exchange;
     fl->f.exchange = (char*)fl->exchange + 256;

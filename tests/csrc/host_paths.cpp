@@ -1,0 +1,92 @@
+// host_paths.cpp - the host side of the solver (fluid_host.cpp, batch_host.cpp,
+// staging.cpp) on a runtime in host memory (fake_hip.cpp): what happens to
+// device memory and streams where a GPU could only fault.  One scenario per
+// run, named by the first argument; prints "ok", or what went wrong.
+#include <cstdio>
+#include <cstring>
+#include <map>
+#include <string>
+
+#include "../../include/opensayal.h"
+#include "fake_hip.hpp"
+
+namespace {
+
+int g_failed = 0;
+
+void expect(bool ok, const char* what) {
+  if (ok) return;
+  std::printf("failed: %s\n", what);
+  g_failed = 1;
+}
+#define EXPECT(x) expect((x), #x)
+
+osy_config config(int W, int H, int n, bool pressure = false) {
+  osy_config c;
+  osy_config_defaults(&c);
+  char text[128];
+  std::snprintf(text, sizeof text,
+                "{\"sim\": {\"width\": %d, \"height\": %d}, \"fluid\": {\"viscosity\": 0}}", W, H);
+  osy_config_parse_string(text, &c);
+  c.projection_n = n;
+  c.enable_pressure = pressure ? 1 : 0;
+  return c;
+}
+
+osy_fluid* create(const osy_config& c) {
+  osy_fluid* fl = nullptr;
+  EXPECT(osy_fluid_create(&c, &fl) == OSY_OK);
+  return fl;
+}
+
+// A register (2) or resident (3) shape of `rows` x 8 region rows.
+osy_tuning shape(int kernel, int rows, int k) {
+  osy_tuning t;
+  t.projection_kernel = kernel;
+  t.tile_width = 128 - 4 * k;
+  t.tile_height = 8 * rows - 4 * k;
+  t.sweeps_per_launch = k;
+  return t;
+}
+
+// A larger exchange buffer cannot be had: the shape is refused, and the
+// handle goes on with what it has.
+void exchange_out_of_memory() {
+  osy_fluid* fl = create(config(250, 230, 20));
+  osy_tuning small = shape(3, 12, 5), large = shape(3, 4, 3);
+  EXPECT(osy_fluid_set_tuning(fl, &small) == OSY_OK);
+  EXPECT(osy_fluid_step(fl, 5, 0.05f) == OSY_OK);
+  fake::state().fail_malloc_from = 1;
+  EXPECT(osy_fluid_set_tuning(fl, &large) == OSY_E_NOMEM);
+  // no error is left behind for the calls that follow
+  EXPECT(osy_fluid_project(fl, 20, nullptr) == OSY_OK);
+  EXPECT(osy_fluid_step(fl, 5, 0.05f) == OSY_OK);
+  osy_tuning now;
+  EXPECT(osy_fluid_get_tuning(fl, &now) == OSY_OK);
+  EXPECT(std::memcmp(&now, &small, sizeof now) == 0);
+  fake::state().fail_malloc_from = ~size_t(0);
+  EXPECT(osy_fluid_set_tuning(fl, &large) == OSY_OK);
+  EXPECT(osy_fluid_step(fl, 5, 0.05f) == OSY_OK);
+  EXPECT(fake::state().launches.back().resident);
+  osy_fluid_destroy(fl);
+}
+
+const std::map<std::string, void (*)()> kScenarios = {
+    {"exchange_out_of_memory", exchange_out_of_memory},
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  if (argc != 2 || !kScenarios.count(argv[1])) {
+    for (const auto& s : kScenarios) std::printf("%s\n", s.first.c_str());
+    return 2;
+  }
+  kScenarios.at(argv[1])();
+  for (const std::string& v : fake::state().violations) {
+    std::printf("violation: %s\n", v.c_str());
+    g_failed = 1;
+  }
+  if (!g_failed) std::printf("ok\n");
+  return g_failed;
+}
