@@ -286,7 +286,8 @@ int enqueue_graph_steps(osy_fluid* fl, int32_t steps, float d_t, hipStream_t s) 
 // resident projection starts from a clean exchange buffer.
 int adopt_tuning(osy_fluid* fl, const ProjTuning& t) {
   if (t.kernel == PROJ_RESIDENT) {
-    if (int st = fluid_clean_exchange(fl, t)) return st;
+    if (int st = fluid_clean_exchange(fl, t, &fl->exchange)) return st;
+    fl->exchange.bind(fl->f);
     OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
   }
   fl->tuning = t;
@@ -346,12 +347,12 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t) {
   return t.tiles(fl->W, fl->H) <= resident_slots(t.reg_rows(), fl->cus);
 }
 
-int fluid_clean_exchange(osy_fluid* fl, const ProjTuning& shape) {
+int fluid_clean_exchange(const osy_fluid* fl, const ProjTuning& shape, Exchange* x) {
   ProjTuning t;
   if (!shape.resident_plan(fl->W, fl->H, fl->cus, &t)) return OSY_OK;
   const size_t bytes =
       256 + 3 * 8 * t.exchange_words(fl->W, fl->H, (size_t)fl->elem);
-  if (fl->exchange_bytes < bytes) {
+  if (x->bytes < bytes) {
     // the new memory first: without it the handle goes on with the old
     void* mem = nullptr;
     const hipError_t e = hipMalloc(&mem, bytes);
@@ -360,14 +361,12 @@ int fluid_clean_exchange(osy_fluid* fl, const ProjTuning& shape) {
       return set_error(OSY_E_NOMEM, "halo exchange of " + std::to_string(bytes) +
                                         " bytes: " + hipGetErrorString(e));
     }
-    if (fl->exchange) (void)hipFree(fl->exchange);  // waits for the launches that use it
-    fl->exchange = mem;
-    fl->exchange_bytes = bytes;
-    fl->f.rstate = (unsigned*)fl->exchange;
-    fl->f.exchange = (char*)fl->exchange + 256;
+    x->release();
+    x->mem = mem;
+    x->bytes = bytes;
   }
-  OSY_HIP_CHECK(hipMemsetAsync(fl->exchange, 0, 256, fl->stream));
-  OSY_HIP_CHECK(hipMemsetAsync(fl->f.exchange, 0xFF, fl->exchange_bytes - 256, fl->stream));
+  OSY_HIP_CHECK(hipMemsetAsync(x->mem, 0, 256, fl->stream));
+  OSY_HIP_CHECK(hipMemsetAsync((char*)x->mem + 256, 0xFF, x->bytes - 256, fl->stream));
   return OSY_OK;
 }
 
@@ -381,7 +380,7 @@ int fluid_check_error(osy_fluid* fl) {
     OSY_HIP_CHECK(hipMemcpy(fl->f.error, &zero, sizeof(int), hipMemcpyHostToDevice));
     // rings may be left half read
     if (fl->tuning.kernel == PROJ_RESIDENT)
-      if (int st = fluid_clean_exchange(fl, fl->tuning)) return st;
+      if (int st = fluid_clean_exchange(fl, fl->tuning, &fl->exchange)) return st;
     OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
     return set_error(OSY_E_STATE,
                      "projection: a neighbour wait of the resident kernel timed out; the "
@@ -785,18 +784,24 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
     if (e == hipSuccess) e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);
     best_ms = 1e30;
+    // the trials' own exchange buffer: the handle's stays as its graphs name it
+    // should the trials fail
+    Exchange trial;
+    FieldPtrs ft = fl->f;
     for (const ProjTuning& cand : tuning_candidates(pressure)) {
       if (e != hipSuccess) break;
       if (!tuning_fits(fl, cand)) continue;
-      if (cand.kernel == PROJ_RESIDENT)
-        if (fluid_clean_exchange(fl, cand) != OSY_OK) continue;  // no memory for it
+      if (cand.kernel == PROJ_RESIDENT) {
+        if (fluid_clean_exchange(fl, cand, &trial) != OSY_OK) continue;  // no memory for it
+        trial.bind(ft);
+      }
       float t_min = 1e30f;
       for (int rep = 0; rep < 3 && e == hipSuccess; rep++) {  // rep 0 warms up
         e = restore(fl->stream);
         if (e == hipSuccess) e = hipEventRecord(e0, fl->stream);
         int cur = fl->uv;
         if (e == hipSuccess) {
-          enqueue_projection_only(fl->storage, sp, fl->f, &cur, cand, fl->stream);
+          enqueue_projection_only(fl->storage, sp, ft, &cur, cand, fl->stream);
           e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipEventRecord(e1, fl->stream);
@@ -822,7 +827,11 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     (void)hipFree(snap);
-    if (e != hipSuccess) return set_error(OSY_E_HIP, std::string("autotune: ") + hipGetErrorString(e));
+    trial.release();
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by a later launch's check
+      return set_error(OSY_E_HIP, std::string("autotune: ") + hipGetErrorString(e));
+    }
     int st = drop_graphs(fl);
     if (st != OSY_OK) return st;
     st = adopt_tuning(fl, best);

@@ -23,6 +23,28 @@ using osy::FieldPtrs;
 using osy::ProjTuning;
 using osy::StepParams;
 
+namespace osy {
+
+// Device memory of a resident projection's halo exchange: a line of state
+// words, then the slots.
+struct Exchange {
+  void* mem = nullptr;
+  size_t bytes = 0;
+  ~Exchange() { release(); }
+  // (hipFree waits for the launches that use it)
+  void release() {
+    if (mem) (void)hipFree(mem);
+    mem = nullptr;
+    bytes = 0;
+  }
+  void bind(FieldPtrs& f) const {
+    f.rstate = (unsigned*)mem;
+    f.exchange = mem ? (char*)mem + 256 : nullptr;
+  }
+};
+
+}  // namespace osy
+
 struct osy_fluid {
   osy_config cfg{};
   int W = 0, H = 0, P = 0, cs = 1, storage = 0, elem = 4;
@@ -35,8 +57,7 @@ struct osy_fluid {
   float* staging = nullptr;  // W*H*4 bytes, reference-order copies
   void* trace_buf = nullptr;  // path-line output, grown on demand
   size_t trace_cap = 0;
-  void* exchange = nullptr;   // resident projection's halo exchange, made when
-  size_t exchange_bytes = 0;  // that shape is first chosen (fluid_clean_exchange)
+  osy::Exchange exchange;  // made when a resident shape is first chosen
   ProjTuning tuning;  // projection kernel shape, chosen at create
   long long spin_ticks = 0;  // bound of a resident projection's neighbour wait
   int cus = 0;               // CUs of the device
@@ -57,7 +78,6 @@ struct osy_fluid {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
     if (block) (void)hipFree(block);
     if (trace_buf) (void)hipFree(trace_buf);
-    if (exchange) (void)hipFree(exchange);
     if (stream) (void)hipStreamDestroy(stream);
     osy::staging_release();
   }
@@ -129,9 +149,9 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t);
 // autotuner tunes the projection of members that step on their own graphs.
 int fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms);
 
-// Makes the handle's halo exchange buffer large enough for projection shape
-// t and fills it with empty words on the handle's stream.
-int fluid_clean_exchange(osy_fluid* fl, const ProjTuning& t);
+// Makes a halo exchange buffer large enough for projection shape t of a handle
+// and fills it with empty words on the handle's stream.
+int fluid_clean_exchange(const osy_fluid* fl, const ProjTuning& t, Exchange* x);
 
 // Reads and clears the device error word (a resident projection whose
 // neighbour wait timed out) when a resident projection ran since the last

@@ -370,6 +370,9 @@ hipError_t hipEventDestroy(hipEvent_t e) {
   return hipSuccess;
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  long& left = fake::state().event_records_left;
+  if (left == 0) return done(hipErrorUnknown);
+  if (left > 0) left--;
   push(s, [e] { ((Event*)e)->at = g_clock; });
   return hipSuccess;
 }

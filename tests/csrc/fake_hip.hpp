@@ -31,6 +31,7 @@ struct State {
   std::vector<std::string> violations;
   std::vector<Launch> launches;  // in the order they started
   size_t fail_malloc_from = ~size_t(0);  // hipMalloc of at least this many bytes fails
+  long event_records_left = -1;  // hipEventRecord fails after as many (-1: never)
   int batch_launches = 0;
   int host_mallocs = 0, host_frees = 0;
   size_t device_bytes = 0;  // held by hipMalloc now

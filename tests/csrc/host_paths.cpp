@@ -71,8 +71,42 @@ void exchange_out_of_memory() {
   osy_fluid_destroy(fl);
 }
 
+// An autotune that fails on the way leaves the handle, its exchange buffer and
+// the graphs that name it as they were.
+void autotune_fails() {
+  osy_fluid* fl = create(config(250, 230, 20));
+  osy_tuning mine = shape(3, 12, 5);
+  EXPECT(osy_fluid_set_tuning(fl, &mine) == OSY_OK);
+  for (int parity = 0; parity < 2; parity++) EXPECT(osy_fluid_step(fl, 5, 0.05f) == OSY_OK);
+  for (long records = 1; records < 700; records += 3) {
+    fake::state().event_records_left = records;
+    const int st = osy_fluid_autotune(fl, nullptr, nullptr);
+    if (st == OSY_OK) break;  // there were enough
+    fake::state().event_records_left = -1;
+    EXPECT(osy_fluid_step(fl, 5, 0.05f) == OSY_OK);
+    osy_tuning now;
+    EXPECT(osy_fluid_get_tuning(fl, &now) == OSY_OK);
+    EXPECT(std::memcmp(&now, &mine, sizeof now) == 0);
+  }
+  osy_fluid_destroy(fl);
+  EXPECT(fake::state().device_bytes == 0);
+}
+
+// No memory for any exchange buffer: the autotuner picks among the others.
+void autotune_without_exchange() {
+  osy_fluid* fl = create(config(250, 230, 20));
+  fake::state().fail_malloc_from = 1 << 20;  // the snapshot fits
+  osy_tuning best;
+  EXPECT(osy_fluid_autotune(fl, &best, nullptr) == OSY_OK);
+  EXPECT(best.projection_kernel != 3);
+  EXPECT(osy_fluid_step(fl, 5, 0.05f) == OSY_OK);
+  osy_fluid_destroy(fl);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
+    {"autotune_fails", autotune_fails},
+    {"autotune_without_exchange", autotune_without_exchange},
 };
 
 }  // namespace

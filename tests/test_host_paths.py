@@ -15,6 +15,8 @@ ROCM = Path("/opt/rocm/include")
 
 SCENARIOS = [
     "exchange_out_of_memory",
+    "autotune_fails",
+    "autotune_without_exchange",
 ]
 
 
