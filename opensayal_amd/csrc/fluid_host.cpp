@@ -809,6 +809,18 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
         float t = 0.0f;
         if (e == hipSuccess) e = hipEventElapsedTime(&t, e0, e1);
         if (rep > 0 && t < t_min) t_min = t;
+        // a wait that timed out (another program's work held the CUs): this
+        // launch and, until its rings are clean again, those after it leave
+        // without waiting, so none of their times counts
+        int timed_out = 0;
+        if (e == hipSuccess && cand.kernel == PROJ_RESIDENT)
+          e = hipMemcpy(&timed_out, fl->f.error, sizeof(int), hipMemcpyDeviceToHost);
+        if (timed_out) {
+          const int zero = 0;
+          e = hipMemcpy(fl->f.error, &zero, sizeof(int), hipMemcpyHostToDevice);
+          t_min = 1e30f;
+          break;
+        }
       }
       if (e == hipSuccess && t_min < best_ms) {
         best_ms = t_min;
@@ -819,8 +831,7 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
     if (e == hipSuccess) e = r;
     r = hipStreamSynchronize(fl->stream);
     if (e == hipSuccess) e = r;
-    // a resident trial whose wait timed out only mistimed itself: the state
-    // was restored from the snapshot, so its error word is cleared
+    // (a trial that failed before its error word was read may have set it)
     const int zero = 0;
     r = hipMemcpy(fl->f.error, &zero, sizeof(int), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = r;

@@ -103,10 +103,35 @@ void autotune_without_exchange() {
   osy_fluid_destroy(fl);
 }
 
+// A resident trial whose wait times out leaves early from then on; its time is
+// no time of that shape, nor are the ones after it.
+void autotune_times_out() {
+  osy_tuning best;
+  osy_fluid* one = create(config(250, 230, 20));
+  fake::state().times_out = [](const osy::ProjTuning& t) { return t.k == 5; };
+  EXPECT(osy_fluid_autotune(one, &best, nullptr) == OSY_OK);
+  EXPECT(best.projection_kernel == 3 && best.sweeps_per_launch != 5);
+  EXPECT(osy_fluid_step(one, 5, 0.05f) == OSY_OK);
+  osy_fluid_destroy(one);
+  osy_fluid* all = create(config(250, 231, 20));
+  fake::state().times_out = [](const osy::ProjTuning&) { return true; };
+  EXPECT(osy_fluid_autotune(all, &best, nullptr) == OSY_OK);
+  EXPECT(best.projection_kernel != 3);
+  osy_fluid* next = create(config(250, 231, 20));
+  EXPECT(osy_fluid_autotune_cached(next) == 1);
+  EXPECT(osy_fluid_get_tuning(next, &best) == OSY_OK);
+  EXPECT(best.projection_kernel != 3);
+  EXPECT(osy_fluid_step(all, 5, 0.05f) == OSY_OK);
+  EXPECT(osy_fluid_synchronize(all) == OSY_OK);
+  osy_fluid_destroy(next);
+  osy_fluid_destroy(all);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
     {"autotune_without_exchange", autotune_without_exchange},
+    {"autotune_times_out", autotune_times_out},
 };
 
 }  // namespace

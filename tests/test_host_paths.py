@@ -17,6 +17,7 @@ SCENARIOS = [
     "exchange_out_of_memory",
     "autotune_fails",
     "autotune_without_exchange",
+    "autotune_times_out",
 ]
 
 
