@@ -543,6 +543,9 @@ int osy_batch_autotune(osy_batch* b, osy_batch_tuning* chosen, double* ms) {
   if (st == OSY_OK && e != hipSuccess) st = set_error(OSY_E_HIP, hipGetErrorString(e));
   // restore
   (void)hipStreamSynchronize(b->stream);
+  // a resident trial that timed out: what it left in its exchange buffer goes
+  // now, since the state put back has no error word to tell
+  for (osy_fluid* fl : b->members) (void)fluid_check_error(fl);
   off = 0;
   for (size_t i = 0; i < b->members.size(); i++) {
     osy_fluid* fl = b->members[i];

@@ -127,11 +127,39 @@ void autotune_times_out() {
   osy_fluid_destroy(all);
 }
 
+// A wait that times out in a batch autotuner's trial, in a member that steps
+// on its own graphs: its state is put back, and its rings are clean again.
+void batch_autotune_times_out() {
+  osy_fluid* own = create(config(250, 230, 20));
+  osy_fluid* shared = create(config(64, 36, 20));
+  osy_batch* b = nullptr;
+  EXPECT(osy_batch_create(0, &b) == OSY_OK);
+  EXPECT(osy_batch_set_per_grid_cells(b, 250 * 230) == OSY_OK);
+  EXPECT(osy_batch_add(b, own) == OSY_OK);
+  EXPECT(osy_batch_add(b, shared) == OSY_OK);
+  fake::state().times_out = [](const osy::ProjTuning&) {
+    return fake::state().batch_launches == 100;
+  };
+  EXPECT(osy_batch_autotune(b, nullptr, nullptr) == OSY_OK);
+  EXPECT(fake::state().batch_launches > 100);
+  fake::state().times_out = nullptr;
+  osy_tuning t;
+  EXPECT(osy_fluid_get_tuning(own, &t) == OSY_OK && t.projection_kernel == 3);
+  fake::state().violations.clear();  // those of the trials, whose results are dropped
+  EXPECT(osy_batch_step(b, 4) == OSY_OK);
+  float p[250 * 230];
+  EXPECT(osy_fluid_get_field(own, OSY_FIELD_VEL_X, p, sizeof p) == OSY_OK);
+  osy_batch_destroy(b);
+  osy_fluid_destroy(own);
+  osy_fluid_destroy(shared);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
     {"autotune_without_exchange", autotune_without_exchange},
     {"autotune_times_out", autotune_times_out},
+    {"batch_autotune_times_out", batch_autotune_times_out},
 };
 
 }  // namespace

@@ -18,6 +18,7 @@ SCENARIOS = [
     "autotune_fails",
     "autotune_without_exchange",
     "autotune_times_out",
+    "batch_autotune_times_out",
 ]
 
 
