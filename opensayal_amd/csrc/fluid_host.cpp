@@ -226,8 +226,27 @@ int create_impl(const osy_config* cfg, osy_fluid** out) {
   return OSY_OK;
 }
 
+void clean_exchange(Exchange* x, hipStream_t s) {
+  if (x->mem) enqueue_clean_exchange(x->mem, x->bytes, s);
+  x->dirty = false;
+}
+
+// Before projections of the handle's shape are put on stream s.
+int before_projection(osy_fluid* fl, hipStream_t s) {
+  if (fl->tuning.kernel != PROJ_RESIDENT) return OSY_OK;
+  fl->resident_pending = true;
+  if (!fl->exchange.dirty) return OSY_OK;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  OSY_HIP_CHECK(hipStreamIsCapturing(s, &capture));
+  clean_exchange(&fl->exchange, s);
+  // (a captured cleaning runs with its graph, not now)
+  fl->exchange.dirty = capture != hipStreamCaptureStatusNone;
+  OSY_HIP_CHECK(hipGetLastError());
+  return OSY_OK;
+}
+
 int enqueue_eager(osy_fluid* fl, const osy_source* src, float d_t, hipStream_t s) {
-  if (fl->tuning.kernel == PROJ_RESIDENT) fl->resident_pending = true;
+  if (int st = before_projection(fl, s)) return st;
   StepParams sp = fl->params(d_t, src);
   enqueue_step(fl->storage, sp, fl->f, &fl->uv, &fl->sm, fl->tuning, s);
   OSY_HIP_CHECK(hipGetLastError());
@@ -240,7 +259,8 @@ int enqueue_eager(osy_fluid* fl, const osy_source* src, float d_t, hipStream_t s
 constexpr int kGraphSteps = 4;
 
 int enqueue_graph_steps(osy_fluid* fl, int32_t steps, float d_t, hipStream_t s) {
-  if (steps > 0 && fl->tuning.kernel == PROJ_RESIDENT) fl->resident_pending = true;
+  if (steps > 0)
+    if (int st = before_projection(fl, s)) return st;
   for (int32_t k = 0, count; k < steps; k += count) {
     count = steps - k >= kGraphSteps ? kGraphSteps : 1;
     osy_fluid::Graph& g = fl->graphs[fl->uv + (count > 1 ? 2 : 0)][fl->sm];
@@ -281,14 +301,21 @@ int enqueue_graph_steps(osy_fluid* fl, int32_t steps, float d_t, hipStream_t s) 
   return OSY_OK;
 }
 
-// Makes `t` the handle's projection shape (its graphs are gone and its
-// stream is idle).  The rings of another shape lie elsewhere, so the
-// resident projection starts from a clean exchange buffer.
+// Makes `t` the handle's projection shape (its graphs are gone and its own
+// stream is idle; launches may still run on a stream of the caller's).  The
+// rings of another shape lie elsewhere, so the resident projection starts from a
+// clean exchange buffer.
 int adopt_tuning(osy_fluid* fl, const ProjTuning& t) {
   if (t.kernel == PROJ_RESIDENT) {
-    if (int st = fluid_clean_exchange(fl, t, &fl->exchange)) return st;
-    fl->exchange.bind(fl->f);
-    OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+    Exchange& x = fl->exchange;
+    const void* had = x.mem;
+    if (int st = fluid_reserve_exchange(fl, t, &x)) return st;
+    x.bind(fl->f);
+    if (x.mem != had) {  // no launch knows it yet
+      clean_exchange(&x, fl->stream);
+      OSY_HIP_CHECK(hipGetLastError());
+      OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+    }
   }
   fl->tuning = t;
   return OSY_OK;
@@ -347,7 +374,7 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t) {
   return t.tiles(fl->W, fl->H) <= resident_slots(t.reg_rows(), fl->cus);
 }
 
-int fluid_clean_exchange(const osy_fluid* fl, const ProjTuning& shape, Exchange* x) {
+int fluid_reserve_exchange(const osy_fluid* fl, const ProjTuning& shape, Exchange* x) {
   ProjTuning t;
   if (!shape.resident_plan(fl->W, fl->H, fl->cus, &t)) return OSY_OK;
   const size_t bytes =
@@ -365,8 +392,7 @@ int fluid_clean_exchange(const osy_fluid* fl, const ProjTuning& shape, Exchange*
     x->mem = mem;
     x->bytes = bytes;
   }
-  OSY_HIP_CHECK(hipMemsetAsync(x->mem, 0, 256, fl->stream));
-  OSY_HIP_CHECK(hipMemsetAsync((char*)x->mem + 256, 0xFF, x->bytes - 256, fl->stream));
+  x->dirty = true;
   return OSY_OK;
 }
 
@@ -378,10 +404,7 @@ int fluid_check_error(osy_fluid* fl) {
   if (err) {
     const int zero = 0;
     OSY_HIP_CHECK(hipMemcpy(fl->f.error, &zero, sizeof(int), hipMemcpyHostToDevice));
-    // rings may be left half read
-    if (fl->tuning.kernel == PROJ_RESIDENT)
-      if (int st = fluid_clean_exchange(fl, fl->tuning, &fl->exchange)) return st;
-    OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+    fl->exchange.dirty = true;  // rings may be left half read
     return set_error(OSY_E_STATE,
                      "projection: a neighbour wait of the resident kernel timed out; the "
                      "fields are invalid");
@@ -485,7 +508,7 @@ int osy_fluid_project(osy_fluid* fl, int32_t sweeps, void* hip_stream) {
   hipStream_t s = hip_stream ? (hipStream_t)hip_stream : fl->stream;
   StepParams sp = fl->params(fl->cfg.d_t, nullptr);
   sp.n = sweeps;
-  if (fl->tuning.kernel == PROJ_RESIDENT) fl->resident_pending = true;
+  if (int st = before_projection(fl, s)) return st;
   enqueue_projection_only(fl->storage, sp, fl->f, &fl->uv, fl->tuning, s);
   OSY_HIP_CHECK(hipGetLastError());
   return OSY_OK;
@@ -792,8 +815,9 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
       if (e != hipSuccess) break;
       if (!tuning_fits(fl, cand)) continue;
       if (cand.kernel == PROJ_RESIDENT) {
-        if (fluid_clean_exchange(fl, cand, &trial) != OSY_OK) continue;  // no memory for it
+        if (fluid_reserve_exchange(fl, cand, &trial) != OSY_OK) continue;  // no memory for it
         trial.bind(ft);
+        clean_exchange(&trial, fl->stream);
       }
       float t_min = 1e30f;
       for (int rep = 0; rep < 3 && e == hipSuccess; rep++) {  // rep 0 warms up

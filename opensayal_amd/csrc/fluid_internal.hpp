@@ -30,6 +30,9 @@ namespace osy {
 struct Exchange {
   void* mem = nullptr;
   size_t bytes = 0;
+  // another shape or a timed-out wait left words in it: it is cleaned on the
+  // stream of the next launch, behind whatever still uses it there
+  bool dirty = false;
   ~Exchange() { release(); }
   // (hipFree waits for the launches that use it)
   void release() {
@@ -149,9 +152,9 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t);
 // autotuner tunes the projection of members that step on their own graphs.
 int fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms);
 
-// Makes a halo exchange buffer large enough for projection shape t of a handle
-// and fills it with empty words on the handle's stream.
-int fluid_clean_exchange(const osy_fluid* fl, const ProjTuning& t, Exchange* x);
+// Makes a halo exchange buffer large enough for projection shape t of a handle;
+// it is dirty then.
+int fluid_reserve_exchange(const osy_fluid* fl, const ProjTuning& t, Exchange* x);
 
 // Reads and clears the device error word (a resident projection whose
 // neighbour wait timed out) when a resident projection ran since the last

@@ -214,6 +214,11 @@ void enqueue_render(int storage, const StepParams& sp, const FieldPtrs& f, int s
 void enqueue_traces(int storage, const StepParams& sp, const FieldPtrs& f, int uv, int distance,
                     int length, float d_t, int32_t* tx, int32_t* ty, hipStream_t s);
 
+// Empties a resident projection's halo exchange buffer (`bytes` a multiple of
+// 16): 256 bytes of state words, 0, and slots of words that hold nothing.  A
+// kernel rather than a fill of the runtime's, so that it can be captured.
+void enqueue_clean_exchange(void* mem, size_t bytes, hipStream_t s);
+
 // Plain device-to-device copy of `bytes` (a multiple of 16) with 16-byte
 // loads and stores, for calibrating hardware byte counters.
 void enqueue_copy(void* dst, const void* src, size_t bytes, hipStream_t s);

@@ -600,7 +600,20 @@ __global__ void __launch_bounds__(256) k_copy(uint4* __restrict__ dst,
   for (size_t k = (size_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (size_t)gridDim.x * 256)
     dst[k] = src[k];
 }
+__global__ void __launch_bounds__(256) k_clean_exchange(uint4* __restrict__ mem, size_t n) {
+  for (size_t k = (size_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (size_t)gridDim.x * 256) {
+    const uint32_t w = k < 16 ? 0u : ~0u;
+    mem[k] = make_uint4(w, w, w, w);
+  }
+}
 }  // namespace
+
+void enqueue_clean_exchange(void* mem, size_t bytes, hipStream_t s) {
+  const size_t n = bytes / 16;
+  size_t blocks = (n + 255) / 256;
+  if (blocks > 8192) blocks = 8192;
+  hipLaunchKernelGGL(k_clean_exchange, dim3((unsigned)blocks), dim3(256), 0, s, (uint4*)mem, n);
+}
 
 void enqueue_copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
   const size_t n = bytes / 16;

@@ -154,12 +154,46 @@ void batch_autotune_times_out() {
   osy_fluid_destroy(shared);
 }
 
+// The exchange buffer is cleaned in the order of the stream that uses it: not
+// while a launch that the caller put on a stream of their own is running.
+void cleaned_in_stream_order() {
+  osy_fluid* fl = create(config(250, 230, 20));
+  osy_tuning first = shape(3, 12, 5), second = shape(3, 12, 4);
+  void* s = nullptr;
+  EXPECT(osy_stream_create(&s) == OSY_OK);
+  EXPECT(osy_fluid_set_tuning(fl, &second) == OSY_OK);
+  EXPECT(osy_fluid_set_tuning(fl, &first) == OSY_OK);
+  EXPECT(osy_fluid_step_async(fl, 2, 0.05f, s) == OSY_OK);
+  while (fake::state().launches.empty()) fake::run((hipStream_t)s, 1);
+  // the first step's launch is running
+  EXPECT(fake::state().launches.size() == 1);
+  EXPECT(osy_fluid_set_tuning(fl, &second) == OSY_OK);
+  EXPECT(osy_fluid_step_async(fl, 3, 0.05f, s) == OSY_OK);
+  EXPECT(osy_stream_synchronize(s) == OSY_OK);
+  EXPECT(fake::state().launches.size() == 5);
+
+  fake::state().times_out = [](const osy::ProjTuning&) {
+    return fake::state().launches.size() == 6;
+  };
+  EXPECT(osy_fluid_step_async(fl, 2, 0.05f, s) == OSY_OK);
+  while (fake::state().launches.size() < 7) fake::run((hipStream_t)s, 1);
+  // the sixth has timed out, the seventh is running
+  EXPECT(osy_fluid_synchronize(fl) == OSY_E_STATE);
+  EXPECT(osy_fluid_step_async(fl, 2, 0.05f, s) == OSY_OK);
+  EXPECT(osy_stream_synchronize(s) == OSY_OK);
+  EXPECT(fake::state().launches.size() == 9);
+  EXPECT(osy_fluid_synchronize(fl) == OSY_OK);
+  osy_fluid_destroy(fl);
+  EXPECT(osy_stream_destroy(s) == OSY_OK);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
     {"autotune_without_exchange", autotune_without_exchange},
     {"autotune_times_out", autotune_times_out},
     {"batch_autotune_times_out", batch_autotune_times_out},
+    {"cleaned_in_stream_order", cleaned_in_stream_order},
 };
 
 }  // namespace

@@ -19,6 +19,7 @@ SCENARIOS = [
     "autotune_without_exchange",
     "autotune_times_out",
     "batch_autotune_times_out",
+    "cleaned_in_stream_order",
 ]
 
 
