@@ -4,6 +4,7 @@
 // step sequence replayed from captured HIP graphs.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -235,12 +236,14 @@ void clean_exchange(Exchange* x, hipStream_t s) {
 int before_projection(osy_fluid* fl, hipStream_t s) {
   if (fl->tuning.kernel != PROJ_RESIDENT) return OSY_OK;
   fl->resident_pending = true;
-  if (!fl->exchange.dirty) return OSY_OK;
+  Exchange& x = fl->exchange;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  OSY_HIP_CHECK(hipStreamIsCapturing(s, &capture));
-  clean_exchange(&fl->exchange, s);
-  // (a captured cleaning runs with its graph, not now)
-  fl->exchange.dirty = capture != hipStreamCaptureStatusNone;
+  if (s != fl->stream) OSY_HIP_CHECK(hipStreamIsCapturing(s, &capture));
+  const bool captured = capture != hipStreamCaptureStatusNone;
+  if (captured) x.captured = true;
+  if (!x.dirty) return OSY_OK;
+  clean_exchange(&x, s);
+  x.dirty = captured;  // a captured cleaning runs with its graph, not now
   OSY_HIP_CHECK(hipGetLastError());
   return OSY_OK;
 }
@@ -306,16 +309,31 @@ int enqueue_graph_steps(osy_fluid* fl, int32_t steps, float d_t, hipStream_t s) 
 // rings of another shape lie elsewhere, so the resident projection starts from a
 // clean exchange buffer.
 int adopt_tuning(osy_fluid* fl, const ProjTuning& t) {
-  if (t.kernel == PROJ_RESIDENT) {
-    Exchange& x = fl->exchange;
-    const void* had = x.mem;
-    if (int st = fluid_reserve_exchange(fl, t, &x)) return st;
-    x.bind(fl->f);
-    if (x.mem != had) {  // no launch knows it yet
-      clean_exchange(&x, fl->stream);
-      OSY_HIP_CHECK(hipGetLastError());
-      OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+  ProjTuning run;
+  Exchange& x = fl->exchange;
+  if (t.kernel == PROJ_RESIDENT && t.resident_plan(fl->W, fl->H, fl->cus, &run) &&
+      !x.serves(run)) {
+    auto kept = std::find_if(fl->captured.begin(), fl->captured.end(),
+                             [&](const Exchange& c) { return c.serves(run); });
+    if (kept != fl->captured.end()) {
+      x.swap(*kept);
+      if (!kept->captured) fl->captured.erase(kept);
+    } else {
+      Exchange fresh;
+      Exchange& to = x.captured ? fresh : x;
+      const void* had = to.mem;
+      if (int st = fluid_reserve_exchange(fl, run, &to)) return st;
+      if (to.mem != had) {  // no launch knows it yet
+        clean_exchange(&to, fl->stream);
+        OSY_HIP_CHECK(hipGetLastError());
+        OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+      }
+      if (x.captured) {
+        x.swap(fresh);
+        fl->captured.push_back(std::move(fresh));
+      }
     }
+    x.bind(fl->f);
   }
   fl->tuning = t;
   return OSY_OK;
@@ -374,11 +392,8 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t) {
   return t.tiles(fl->W, fl->H) <= resident_slots(t.reg_rows(), fl->cus);
 }
 
-int fluid_reserve_exchange(const osy_fluid* fl, const ProjTuning& shape, Exchange* x) {
-  ProjTuning t;
-  if (!shape.resident_plan(fl->W, fl->H, fl->cus, &t)) return OSY_OK;
-  const size_t bytes =
-      256 + 3 * 8 * t.exchange_words(fl->W, fl->H, (size_t)fl->elem);
+int fluid_reserve_exchange(const osy_fluid* fl, const ProjTuning& run, Exchange* x) {
+  const size_t bytes = 256 + 3 * 8 * run.exchange_words(fl->W, fl->H, (size_t)fl->elem);
   if (x->bytes < bytes) {
     // the new memory first: without it the handle goes on with the old
     void* mem = nullptr;
@@ -392,12 +407,15 @@ int fluid_reserve_exchange(const osy_fluid* fl, const ProjTuning& shape, Exchang
     x->mem = mem;
     x->bytes = bytes;
   }
+  x->k = run.k;
+  x->th = run.th;
   x->dirty = true;
   return OSY_OK;
 }
 
 int fluid_check_error(osy_fluid* fl) {
-  if (!fl->resident_pending) return OSY_OK;
+  const bool graphs = fl->exchange.captured || !fl->captured.empty();
+  if (!fl->resident_pending && !graphs) return OSY_OK;
   fl->resident_pending = false;
   int err = 0;
   OSY_HIP_CHECK(hipMemcpy(&err, fl->f.error, sizeof(int), hipMemcpyDeviceToHost));
@@ -405,6 +423,13 @@ int fluid_check_error(osy_fluid* fl) {
     const int zero = 0;
     OSY_HIP_CHECK(hipMemcpy(fl->f.error, &zero, sizeof(int), hipMemcpyHostToDevice));
     fl->exchange.dirty = true;  // rings may be left half read
+    if (graphs) {  // the caller's do not look whether theirs is dirty
+      OSY_HIP_CHECK(hipDeviceSynchronize());
+      clean_exchange(&fl->exchange, fl->stream);
+      for (Exchange& x : fl->captured) clean_exchange(&x, fl->stream);
+      OSY_HIP_CHECK(hipGetLastError());
+      OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+    }
     return set_error(OSY_E_STATE,
                      "projection: a neighbour wait of the resident kernel timed out; the "
                      "fields are invalid");
@@ -814,8 +839,9 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
     for (const ProjTuning& cand : tuning_candidates(pressure)) {
       if (e != hipSuccess) break;
       if (!tuning_fits(fl, cand)) continue;
-      if (cand.kernel == PROJ_RESIDENT) {
-        if (fluid_reserve_exchange(fl, cand, &trial) != OSY_OK) continue;  // no memory for it
+      ProjTuning run;
+      if (cand.kernel == PROJ_RESIDENT && cand.resident_plan(fl->W, fl->H, fl->cus, &run)) {
+        if (fluid_reserve_exchange(fl, run, &trial) != OSY_OK) continue;  // no memory for it
         trial.bind(ft);
         clean_exchange(&trial, fl->stream);
       }

@@ -7,6 +7,8 @@
 
 #include <cmath>
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "kernels.hpp"
 #include "osy_internal.hpp"
@@ -30,16 +32,36 @@ namespace osy {
 struct Exchange {
   void* mem = nullptr;
   size_t bytes = 0;
+  int k = 0, th = 0;  // the shape it serves (ProjTuning::resident_plan)
   // another shape or a timed-out wait left words in it: it is cleaned on the
   // stream of the next launch, behind whatever still uses it there
   bool dirty = false;
+  // a graph that the caller captured names it: it stays, for its shape, until
+  // the handle goes
+  bool captured = false;
+
+  Exchange() = default;
+  Exchange(Exchange&& o) noexcept { swap(o); }
+  Exchange& operator=(Exchange&& o) noexcept {
+    swap(o);
+    return *this;
+  }
   ~Exchange() { release(); }
+  void swap(Exchange& o) noexcept {
+    std::swap(mem, o.mem);
+    std::swap(bytes, o.bytes);
+    std::swap(k, o.k);
+    std::swap(th, o.th);
+    std::swap(dirty, o.dirty);
+    std::swap(captured, o.captured);
+  }
   // (hipFree waits for the launches that use it)
   void release() {
     if (mem) (void)hipFree(mem);
     mem = nullptr;
     bytes = 0;
   }
+  bool serves(const ProjTuning& run) const { return mem && run.k == k && run.th == th; }
   void bind(FieldPtrs& f) const {
     f.rstate = (unsigned*)mem;
     f.exchange = mem ? (char*)mem + 256 : nullptr;
@@ -61,6 +83,7 @@ struct osy_fluid {
   void* trace_buf = nullptr;  // path-line output, grown on demand
   size_t trace_cap = 0;
   osy::Exchange exchange;  // made when a resident shape is first chosen
+  std::vector<osy::Exchange> captured;  // other shapes' that graphs name
   ProjTuning tuning;  // projection kernel shape, chosen at create
   long long spin_ticks = 0;  // bound of a resident projection's neighbour wait
   int cus = 0;               // CUs of the device
@@ -152,9 +175,9 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t);
 // autotuner tunes the projection of members that step on their own graphs.
 int fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms);
 
-// Makes a halo exchange buffer large enough for projection shape t of a handle;
-// it is dirty then.
-int fluid_reserve_exchange(const osy_fluid* fl, const ProjTuning& t, Exchange* x);
+// Makes a halo exchange buffer large enough for resident plan `run` of a
+// handle; it is dirty then.
+int fluid_reserve_exchange(const osy_fluid* fl, const ProjTuning& run, Exchange* x);
 
 // Reads and clears the device error word (a resident projection whose
 // neighbour wait timed out) when a resident projection ran since the last

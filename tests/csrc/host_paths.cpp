@@ -187,6 +187,54 @@ void cleaned_in_stream_order() {
   EXPECT(osy_stream_destroy(s) == OSY_OK);
 }
 
+// A projection that the caller captured goes on working with its own exchange
+// buffer, whatever shapes the handle takes after that.
+void captured_projection() {
+  osy_fluid* fl = create(config(250, 230, 20));
+  const osy_tuning first = shape(3, 12, 5), larger = shape(3, 4, 3), smaller = shape(3, 12, 4),
+                   launches = shape(2, 8, 5);
+  void* s = nullptr;
+  EXPECT(osy_stream_create(&s) == OSY_OK);
+  EXPECT(osy_fluid_set_tuning(fl, &first) == OSY_OK);
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  EXPECT(hipStreamBeginCapture((hipStream_t)s, hipStreamCaptureModeThreadLocal) == hipSuccess);
+  for (int i = 0; i < 2; i++) EXPECT(osy_fluid_project(fl, 20, s) == OSY_OK);
+  EXPECT(hipStreamEndCapture((hipStream_t)s, &graph) == hipSuccess);
+  EXPECT(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess);
+  size_t held = 0;
+  for (int round = 0; round < 3; round++) {
+    for (const osy_tuning* t : {&larger, &smaller, &launches, &first}) {
+      EXPECT(osy_fluid_set_tuning(fl, t) == OSY_OK);
+      EXPECT(osy_fluid_step_async(fl, 2, 0.05f, s) == OSY_OK);
+      EXPECT(hipGraphLaunch(exec, (hipStream_t)s) == hipSuccess);
+      EXPECT(osy_fluid_step_async(fl, 2, 0.05f, s) == OSY_OK);
+      EXPECT(osy_stream_synchronize(s) == OSY_OK);
+      EXPECT(osy_fluid_synchronize(fl) == OSY_OK);
+    }
+    if (round == 1) held = fake::state().device_bytes;
+    if (round == 2) EXPECT(fake::state().device_bytes == held);
+  }
+  // one of its replays times out while the handle has another shape
+  EXPECT(osy_fluid_set_tuning(fl, &smaller) == OSY_OK);
+  EXPECT(osy_fluid_step_async(fl, 2, 0.05f, s) == OSY_OK);
+  EXPECT(osy_stream_synchronize(s) == OSY_OK);
+  EXPECT(osy_fluid_synchronize(fl) == OSY_OK);
+  fake::state().times_out = [](const osy::ProjTuning& t) { return t.k == 5; };
+  EXPECT(hipGraphLaunch(exec, (hipStream_t)s) == hipSuccess);
+  EXPECT(osy_stream_synchronize(s) == OSY_OK);
+  fake::state().times_out = nullptr;
+  EXPECT(osy_fluid_synchronize(fl) == OSY_E_STATE);
+  EXPECT(hipGraphLaunch(exec, (hipStream_t)s) == hipSuccess);
+  EXPECT(osy_stream_synchronize(s) == OSY_OK);
+  EXPECT(osy_fluid_synchronize(fl) == OSY_OK);
+  hipGraphExecDestroy(exec);
+  hipGraphDestroy(graph);
+  osy_fluid_destroy(fl);
+  EXPECT(osy_stream_destroy(s) == OSY_OK);
+  EXPECT(fake::state().device_bytes == 0);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
@@ -194,6 +242,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"autotune_times_out", autotune_times_out},
     {"batch_autotune_times_out", batch_autotune_times_out},
     {"cleaned_in_stream_order", cleaned_in_stream_order},
+    {"captured_projection", captured_projection},
 };
 
 }  // namespace

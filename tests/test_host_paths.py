@@ -20,6 +20,7 @@ SCENARIOS = [
     "autotune_times_out",
     "batch_autotune_times_out",
     "cleaned_in_stream_order",
+    "captured_projection",
 ]
 
 
