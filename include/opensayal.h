@@ -128,7 +128,8 @@ typedef struct osy_fluid_info {
                                 3: register tiles resident for all sweeps,
                                    one launch                              */
   int32_t sweeps_per_launch; /* sweeps one projection launch runs          */
-  size_t device_bytes;  /* device memory held by this handle               */
+  size_t device_bytes;  /* device memory held by this handle: its fields, and
+                           the halo exchange of a resident projection       */
 } osy_fluid_info;
 
 /* Launch shape of the projection, this implementation's own knob (the
@@ -316,7 +317,8 @@ int osy_fluid_autotune(osy_fluid* fluid, osy_tuning* chosen, double* ms);
 int osy_fluid_autotune_cached(osy_fluid* fluid);
 
 /* Device bytes osy_fluid_create would allocate for `cfg` (for admission
- * under a memory budget before creating). */
+ * under a memory budget before creating).  Choosing a resident projection
+ * (kernel 3) adds its halo exchange, which osy_fluid_get_info counts. */
 int osy_fluid_device_bytes(const osy_config* cfg, uint64_t* bytes);
 
 /* ---- batches (no counterpart in the reference, which steps one Fluid) ----
@@ -329,7 +331,10 @@ int osy_fluid_device_bytes(const osy_config* cfg, uint64_t* bytes);
  * divergence_norm first wait for the batch's queued steps.  Each member
  * steps with its own configuration's time.d_t. */
 
-/* `budget_bytes` bounds the sum of the members' device bytes (0 = none).
+/* `budget_bytes` bounds the sum of the members' device bytes (0 = none).  The
+ * halo exchange of a member's resident projection counts: one that does not
+ * fit is given back when the member is added, and its projection then runs
+ * as a launch per stage, with the same results.
  * The batch starts with the shape rows 12, sweeps_per_tile 10, occupancy 2. */
 int osy_batch_create(uint64_t budget_bytes, osy_batch** out);
 /* Members leave the batch (they stay valid).  NULL is accepted. */

@@ -16,7 +16,7 @@
 using namespace osy;
 
 struct osy_batch {
-  uint64_t budget = 0, used = 0;
+  uint64_t budget = 0;
   hipStream_t stream = nullptr;
   hipStream_t last = nullptr;  // stream of the last enqueued steps
   std::vector<osy_fluid*> members;
@@ -47,6 +47,12 @@ struct osy_batch {
   bool timing = false;    // stamp every work item (osy_batch_set_timing)
   bool stamped = false;   // a step ran since the tables were built with stamps
 
+  // device bytes of the members, which the budget bounds
+  uint64_t used() const {
+    uint64_t bytes = 0;
+    for (const osy_fluid* fl : members) bytes += fluid_device_bytes(fl);
+    return bytes;
+  }
   ~osy_batch() { release(); if (stream) (void)hipStreamDestroy(stream); }
   void release() {
     if (exec) (void)hipGraphExecDestroy(exec);
@@ -365,7 +371,6 @@ void batch_forget(osy_fluid* fl) {
   if (!b) return;
   (void)sync_batch(b);
   b->members.erase(std::remove(b->members.begin(), b->members.end(), fl), b->members.end());
-  b->used -= fl->block_bytes;
   fl->batch = nullptr;
   b->release();
 }
@@ -409,15 +414,19 @@ int osy_batch_add(osy_batch* b, osy_fluid* fl) {
   if (fl->cfg.viscosity != 0.0f)
     return set_error(OSY_E_UNSUPPORTED,
                      "a batch does not run the diffusion pass: members need fluid.viscosity 0");
-  if (b->budget && b->used + fl->block_bytes > b->budget)
-    return set_error(OSY_E_BUDGET, "the handle's " + std::to_string(fl->block_bytes) +
+  const uint64_t left = b->budget ? b->budget - std::min(b->budget, b->used()) : ~uint64_t(0);
+  // (without an exchange buffer, if that is what makes it fit)
+  const uint64_t least =
+      fluid_device_bytes(fl) - (fl->exchange.captured ? 0 : fl->exchange.bytes);
+  if (least > left)
+    return set_error(OSY_E_BUDGET, "the handle's " + std::to_string(least) +
                                        " device bytes exceed the batch budget (" +
-                                       std::to_string(b->budget - b->used) + " bytes left)");
+                                       std::to_string(left) + " bytes left)");
   int st = sync_batch(b);
   if (st != OSY_OK) return st;
   OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+  if (fluid_device_bytes(fl) > left) fluid_drop_exchange(fl);
   b->members.push_back(fl);
-  b->used += fl->block_bytes;
   fl->batch = b;
   b->release();
   return OSY_OK;
@@ -486,7 +495,9 @@ int osy_batch_autotune(osy_batch* b, osy_batch_tuning* chosen, double* ms) {
   // batch's stream, so a resident projection is safe there)
   for (osy_fluid* fl : b->members)
     if (b->per_grid_cells > 0 && (int64_t)fl->W * fl->H >= b->per_grid_cells) {
-      st = fluid_autotune(fl, nullptr, nullptr);
+      const uint64_t others = b->used() - fl->exchange.bytes;
+      st = fluid_autotune(fl, nullptr, nullptr,
+                          b->budget ? b->budget - std::min(b->budget, others) : ~uint64_t(0));
       if (st != OSY_OK) return st;
     }
   // save every member's device state and buffer parity
@@ -641,7 +652,7 @@ int osy_batch_get_info(const osy_batch* b, osy_batch_info* info) {
   std::memset(info, 0, sizeof(*info));
   info->count = (int32_t)b->members.size();
   info->budget_bytes = b->budget;
-  info->used_bytes = b->used;
+  info->used_bytes = b->used();
   for (const osy_fluid* fl : b->members) info->cells += (int64_t)fl->W * fl->H;
   info->groups = (int32_t)b->groups.size();
   for (const osy_batch::Group& g : b->groups) info->work_items += g.args.nitems;

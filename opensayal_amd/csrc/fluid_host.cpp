@@ -227,6 +227,20 @@ int create_impl(const osy_config* cfg, osy_fluid** out) {
   return OSY_OK;
 }
 
+int drop_graphs(osy_fluid* fl) {
+  for (auto& row : fl->graphs)
+    for (auto& g : row)
+      if (g.exec) {
+        OSY_HIP_CHECK(hipGraphExecDestroy(g.exec));
+        g.exec = nullptr;
+      }
+  return OSY_OK;
+}
+
+size_t exchange_bytes(const osy_fluid* fl, const ProjTuning& run) {
+  return 256 + 3 * 8 * run.exchange_words(fl->W, fl->H, (size_t)fl->elem);
+}
+
 void clean_exchange(Exchange* x, hipStream_t s) {
   if (x->mem) enqueue_clean_exchange(x->mem, x->bytes, s);
   x->dirty = false;
@@ -335,6 +349,7 @@ int adopt_tuning(osy_fluid* fl, const ProjTuning& t) {
     }
     x.bind(fl->f);
   }
+  if (t.kernel != PROJ_RESIDENT) fluid_drop_exchange(fl);
   fl->tuning = t;
   return OSY_OK;
 }
@@ -392,8 +407,24 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t) {
   return t.tiles(fl->W, fl->H) <= resident_slots(t.reg_rows(), fl->cus);
 }
 
+uint64_t fluid_device_bytes(const osy_fluid* fl) {
+  uint64_t bytes = fl->block_bytes + fl->exchange.bytes;
+  for (const Exchange& x : fl->captured) bytes += x.bytes;
+  return bytes;
+}
+
+void fluid_drop_exchange(osy_fluid* fl) {
+  (void)drop_graphs(fl);  // they name it
+  if (fl->exchange.captured) {
+    fl->captured.push_back(std::move(fl->exchange));
+    fl->exchange = Exchange();
+  }
+  fl->exchange.release();
+  fl->exchange.bind(fl->f);
+}
+
 int fluid_reserve_exchange(const osy_fluid* fl, const ProjTuning& run, Exchange* x) {
-  const size_t bytes = 256 + 3 * 8 * run.exchange_words(fl->W, fl->H, (size_t)fl->elem);
+  const size_t bytes = exchange_bytes(fl, run);
   if (x->bytes < bytes) {
     // the new memory first: without it the handle goes on with the old
     void* mem = nullptr;
@@ -685,12 +716,7 @@ int osy_fluid_set_tuning(osy_fluid* fl, const osy_tuning* t) {
                          "12 or 16 rows (resident: both tile sides >= 2k)");
   }
   OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
-  for (auto& row : fl->graphs)
-    for (auto& g : row)
-      if (g.exec) {
-        OSY_HIP_CHECK(hipGraphExecDestroy(g.exec));
-        g.exec = nullptr;
-      }
+  if (int st = drop_graphs(fl)) return st;
   return adopt_tuning(fl, pt);
 }
 
@@ -764,16 +790,6 @@ std::vector<ProjTuning> tuning_candidates(bool pressure) {
   return out;
 }
 
-int drop_graphs(osy_fluid* fl) {
-  for (auto& row : fl->graphs)
-    for (auto& g : row)
-      if (g.exec) {
-        OSY_HIP_CHECK(hipGraphExecDestroy(g.exec));
-        g.exec = nullptr;
-      }
-  return OSY_OK;
-}
-
 osy_tuning to_abi(const ProjTuning& t) {
   osy_tuning o;
   o.projection_kernel = t.kernel;
@@ -795,7 +811,7 @@ int osy_fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
 
 }  // extern "C"
 
-int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
+int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms, uint64_t exchange_limit) {
   const bool pressure = fl->cfg.enable_pressure != 0;
   StepParams sp = fl->params(fl->cfg.d_t, nullptr);
   sp.forces_in_projection = 0;
@@ -841,6 +857,7 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms) {
       if (!tuning_fits(fl, cand)) continue;
       ProjTuning run;
       if (cand.kernel == PROJ_RESIDENT && cand.resident_plan(fl->W, fl->H, fl->cus, &run)) {
+        if (exchange_bytes(fl, run) > exchange_limit) continue;
         if (fluid_reserve_exchange(fl, run, &trial) != OSY_OK) continue;  // no memory for it
         trial.bind(ft);
         clean_exchange(&trial, fl->stream);
@@ -934,7 +951,7 @@ int osy_fluid_get_info(const osy_fluid* fl, osy_fluid_info* info) {
   info->storage = fl->storage;
   info->projection_kernel = fl->tuning.kernel;
   info->sweeps_per_launch = fl->tuning.kernel == PROJ_COLOUR ? 1 : fl->tuning.k;
-  info->device_bytes = fl->block_bytes;
+  info->device_bytes = fluid_device_bytes(fl);
   return OSY_OK;
 }
 

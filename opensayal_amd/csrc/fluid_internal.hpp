@@ -173,7 +173,18 @@ bool tuning_fits(const osy_fluid* fl, const ProjTuning& t);
 
 // osy_fluid_autotune without the batch-membership check: the batch
 // autotuner tunes the projection of members that step on their own graphs.
-int fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms);
+// Resident shapes whose exchange buffer takes more than `exchange_limit`
+// bytes are left out.
+int fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms,
+                   uint64_t exchange_limit = ~uint64_t(0));
+
+// Device memory that the handle holds: its fields and its exchange buffers.
+uint64_t fluid_device_bytes(const osy_fluid* fl);
+
+// Gives the exchange buffer back, unless a captured graph names it.  A resident
+// shape then runs as a launch per stage, with the same results, until a
+// resident shape is chosen again.
+void fluid_drop_exchange(osy_fluid* fl);
 
 // Makes a halo exchange buffer large enough for resident plan `run` of a
 // handle; it is dirty then.

@@ -235,6 +235,68 @@ void captured_projection() {
   EXPECT(fake::state().device_bytes == 0);
 }
 
+uint64_t device_bytes(osy_fluid* fl) {
+  osy_fluid_info info;
+  EXPECT(osy_fluid_get_info(fl, &info) == OSY_OK);
+  return info.device_bytes;
+}
+
+// The exchange buffer is part of the device memory a handle says it holds, and
+// goes when another kernel is chosen.
+void exchange_is_counted() {
+  osy_fluid* fl = create(config(250, 230, 20));
+  const uint64_t plain = device_bytes(fl);
+  EXPECT(plain == fake::state().device_bytes);
+  const osy_tuning resident = shape(3, 12, 5), launches = shape(2, 8, 5);
+  EXPECT(osy_fluid_set_tuning(fl, &resident) == OSY_OK);
+  EXPECT(device_bytes(fl) > plain);
+  EXPECT(device_bytes(fl) == fake::state().device_bytes);
+  EXPECT(osy_fluid_step(fl, 4, 0.05f) == OSY_OK);
+  EXPECT(osy_fluid_set_tuning(fl, &launches) == OSY_OK);
+  EXPECT(device_bytes(fl) == plain);
+  EXPECT(fake::state().device_bytes == plain);
+  EXPECT(osy_fluid_step(fl, 4, 0.05f) == OSY_OK);
+  osy_fluid_destroy(fl);
+}
+
+// A batch's budget bounds its members' exchange buffers too: what does not
+// fit is given back, and the autotuner does not pick what would not.
+void exchange_in_a_budget() {
+  const osy_config c = config(250, 230, 20);
+  uint64_t plain = 0;
+  EXPECT(osy_fluid_device_bytes(&c, &plain) == OSY_OK);
+  const osy_tuning resident = shape(3, 12, 5);
+  for (const uint64_t budget : {2 * plain + 100000, uint64_t(1) << 32}) {
+    const bool fits = budget > 3 * plain;
+    osy_fluid *one = create(c), *two = create(c);
+    EXPECT(osy_fluid_set_tuning(one, &resident) == OSY_OK);
+    for (int parity = 0; parity < 2; parity++) EXPECT(osy_fluid_step(one, 5, 0.05f) == OSY_OK);
+    osy_batch* b = nullptr;
+    osy_batch_info info;
+    EXPECT(osy_batch_create(budget, &b) == OSY_OK);
+    EXPECT(osy_batch_set_per_grid_cells(b, 1) == OSY_OK);
+    EXPECT(osy_batch_add(b, one) == OSY_OK);
+    EXPECT(osy_batch_add(b, two) == OSY_OK);
+    EXPECT(osy_batch_step(b, 2) == OSY_OK);
+    EXPECT(!fake::state().launches.back().resident);  // member two
+    EXPECT((fake::state().launches.end() - 2)->resident == fits);
+    EXPECT(osy_batch_get_info(b, &info) == OSY_OK);
+    EXPECT(info.used_bytes == device_bytes(one) + device_bytes(two));
+    EXPECT(info.used_bytes <= budget);
+    EXPECT(osy_batch_autotune(b, nullptr, nullptr) == OSY_OK);
+    EXPECT(osy_batch_get_info(b, &info) == OSY_OK);
+    EXPECT(info.used_bytes == device_bytes(one) + device_bytes(two));
+    EXPECT(info.used_bytes <= budget);
+    EXPECT((info.used_bytes > 2 * plain) == fits);
+    EXPECT(osy_batch_step(b, 2) == OSY_OK);
+    osy_fluid* three = create(c);
+    EXPECT(osy_batch_add(b, three) == (fits ? OSY_OK : OSY_E_BUDGET));
+    osy_batch_destroy(b);
+    for (osy_fluid* fl : {one, two, three}) osy_fluid_destroy(fl);
+  }
+  EXPECT(fake::state().device_bytes == 0);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
@@ -243,6 +305,8 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"batch_autotune_times_out", batch_autotune_times_out},
     {"cleaned_in_stream_order", cleaned_in_stream_order},
     {"captured_projection", captured_projection},
+    {"exchange_is_counted", exchange_is_counted},
+    {"exchange_in_a_budget", exchange_in_a_budget},
 };
 
 }  // namespace

@@ -21,6 +21,8 @@ SCENARIOS = [
     "batch_autotune_times_out",
     "cleaned_in_stream_order",
     "captured_projection",
+    "exchange_is_counted",
+    "exchange_in_a_budget",
 ]
 
 
