@@ -126,7 +126,9 @@ typedef struct osy_fluid_info {
                                 1: LDS-tiled, several sweeps per launch;
                                 2: register tiles, several sweeps per launch;
                                 3: register tiles resident for all sweeps,
-                                   one launch                              */
+                                   one launch.  What runs: 2 when a resident
+                                   shape was chosen that runs as a launch
+                                   per stage                               */
   int32_t sweeps_per_launch; /* sweeps one projection launch runs          */
   size_t device_bytes;  /* device memory held by this handle: its fields, and
                            the halo exchange of a resident projection       */
@@ -140,7 +142,11 @@ typedef struct osy_tuning {
                                 2: register tiles; 3: register tiles
                                 resident for all sweeps (one launch; every
                                 tile's workgroup must fit on the device at
-                                once, and both tile sides be >= 2 x k)     */
+                                once, and both tile sides be >= 2 x k).
+                                Regions of 64 rows and more are run as ones
+                                of 96; where those do not fit, and with
+                                pressure sums for d_t = 0 or |d_t| >= 2, as
+                                a launch per stage of kernel 2            */
   int32_t tile_width;        /* tiled: cells a workgroup owns along i (even) */
   int32_t tile_height;       /* tiled: cells a workgroup owns along j       */
   int32_t sweeps_per_launch; /* tiled: sweeps per launch (halo = 2x this);

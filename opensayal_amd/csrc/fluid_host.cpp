@@ -855,8 +855,10 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms, uint64_t 
     for (const ProjTuning& cand : tuning_candidates(pressure)) {
       if (e != hipSuccess) break;
       if (!tuning_fits(fl, cand)) continue;
-      ProjTuning run;
-      if (cand.kernel == PROJ_RESIDENT && cand.resident_plan(fl->W, fl->H, fl->cus, &run)) {
+      if (cand.kernel == PROJ_RESIDENT) {
+        ProjTuning run;
+        // (else it is the register candidate over again)
+        if (!cand.resident_plan(fl->W, fl->H, fl->cus, &run)) continue;
         if (exchange_bytes(fl, run) > exchange_limit) continue;
         if (fluid_reserve_exchange(fl, run, &trial) != OSY_OK) continue;  // no memory for it
         trial.bind(ft);
@@ -949,7 +951,11 @@ int osy_fluid_get_info(const osy_fluid* fl, osy_fluid_info* info) {
   info->projection_n = fl->cfg.projection_n;
   info->pitch = fl->P;
   info->storage = fl->storage;
-  info->projection_kernel = fl->tuning.kernel;
+  ProjTuning run;
+  const bool per_stage =
+      fl->tuning.kernel == PROJ_RESIDENT &&
+      !(fl->exchange.mem && fl->tuning.resident_plan(fl->W, fl->H, fl->cus, &run));
+  info->projection_kernel = per_stage ? PROJ_REGS : fl->tuning.kernel;
   info->sweeps_per_launch = fl->tuning.kernel == PROJ_COLOUR ? 1 : fl->tuning.k;
   info->device_bytes = fluid_device_bytes(fl);
   return OSY_OK;

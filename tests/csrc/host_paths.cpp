@@ -297,6 +297,33 @@ void exchange_in_a_budget() {
   EXPECT(fake::state().device_bytes == 0);
 }
 
+// A resident shape that runs as a launch per stage says so.
+void resident_says_what_runs() {
+  osy_fluid* fl = create(config(2400, 1400, 20));
+  // 500 tiles of 64 rows, which the call takes; 320 of 96, which do not fit
+  const osy_tuning asked = shape(3, 8, 2), fits = shape(3, 12, 5);
+  osy_fluid_info info;
+  osy_tuning now;
+  EXPECT(osy_fluid_set_tuning(fl, &asked) == OSY_OK);
+  EXPECT(osy_fluid_project(fl, 20, nullptr) == OSY_OK);
+  EXPECT(osy_fluid_synchronize(fl) == OSY_OK);
+  EXPECT(!fake::state().launches.back().resident);
+  EXPECT(osy_fluid_get_info(fl, &info) == OSY_OK);
+  EXPECT(info.projection_kernel == 2 && info.sweeps_per_launch == 2);
+  EXPECT(osy_fluid_get_tuning(fl, &now) == OSY_OK);
+  EXPECT(std::memcmp(&now, &asked, sizeof now) == 0);
+  EXPECT(osy_fluid_set_tuning(fl, &fits) == OSY_E_INVALID);  // 414 tiles
+  osy_fluid_destroy(fl);
+  fl = create(config(1920, 1080, 20));
+  EXPECT(osy_fluid_set_tuning(fl, &fits) == OSY_OK);
+  EXPECT(osy_fluid_project(fl, 20, nullptr) == OSY_OK);
+  EXPECT(osy_fluid_synchronize(fl) == OSY_OK);
+  EXPECT(fake::state().launches.back().resident);
+  EXPECT(osy_fluid_get_info(fl, &info) == OSY_OK);
+  EXPECT(info.projection_kernel == 3 && info.sweeps_per_launch == 5);
+  osy_fluid_destroy(fl);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
@@ -307,6 +334,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"captured_projection", captured_projection},
     {"exchange_is_counted", exchange_is_counted},
     {"exchange_in_a_budget", exchange_in_a_budget},
+    {"resident_says_what_runs", resident_says_what_runs},
 };
 
 }  // namespace

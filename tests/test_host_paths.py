@@ -23,6 +23,7 @@ SCENARIOS = [
     "captured_projection",
     "exchange_is_counted",
     "exchange_in_a_budget",
+    "resident_says_what_runs",
 ]
 
 
