@@ -13,9 +13,16 @@
 namespace osy {
 namespace {
 
-std::mutex g_mu;
-Staging* g_idle[kStagingKept];
-int g_idle_count = 0;
+// The buffers of a device: `made` exist or are being made, `idle` of them lie
+// here.
+struct Pool {
+  Staging* idle[kStagingKept];
+  int idle_count, made;
+};
+
+constexpr int kMaxDevices = 64;
+std::mutex g_mu;  // never held while one is made or freed
+Pool g_pools[kMaxDevices];
 long g_handles = 0;
 
 void destroy(Staging* st) {
@@ -66,32 +73,52 @@ void staging_retain() {
 }
 
 void staging_release() {
-  std::lock_guard<std::mutex> lock(g_mu);
-  if (--g_handles > 0) return;
-  while (g_idle_count > 0) destroy(g_idle[--g_idle_count]);
+  for (Pool& pool : g_pools) {
+    Staging* out[kStagingKept];
+    int n = 0;
+    {
+      std::lock_guard<std::mutex> lock(g_mu);
+      if (&pool == g_pools) g_handles--;
+      if (g_handles > 0) return;
+      n = pool.idle_count;
+      std::copy(pool.idle, pool.idle + n, out);
+      pool.idle_count = 0;
+      pool.made -= n;
+    }
+    for (int i = 0; i < n; i++) destroy(out[i]);
+  }
 }
 
 StagingLease::StagingLease(int device, const void* host) {
-  if (!host || !pageable(host)) return;
+  if (!host || device < 0 || device >= kMaxDevices || !pageable(host)) return;
+  Pool& pool = g_pools[device];
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    for (int i = g_idle_count - 1; i >= 0; i--)
-      if (g_idle[i]->device == device) {
-        st_ = g_idle[i];
-        g_idle[i] = g_idle[--g_idle_count];
-        return;
-      }
+    if (pool.idle_count > 0) {
+      st_ = pool.idle[--pool.idle_count];
+      return;
+    }
+    if (pool.made == kStagingKept) return;  // all are out: the runtime's copy
+    pool.made++;
   }
   st_ = create(device);
+  if (st_) return;
+  std::lock_guard<std::mutex> lock(g_mu);
+  pool.made--;
 }
 
 StagingLease::~StagingLease() {
   if (!st_) return;
-  std::lock_guard<std::mutex> lock(g_mu);
-  if (g_handles > 0 && g_idle_count < kStagingKept)
-    g_idle[g_idle_count++] = st_;
-  else
-    destroy(st_);
+  Pool& pool = g_pools[st_->device];
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (g_handles > 0) {
+      pool.idle[pool.idle_count++] = st_;
+      return;
+    }
+    pool.made--;
+  }
+  destroy(st_);
 }
 
 hipError_t StagingLease::copy_out(void* dst, const void* src, size_t bytes, hipStream_t s) {

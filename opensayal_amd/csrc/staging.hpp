@@ -30,8 +30,9 @@ struct Staging {
 };
 
 // Buffers are taken for the length of a call, so calls on several threads and
-// streams never share one.  At most kStagingKept lie idle, and none once the
-// last handle is gone.
+// streams never share one.  A device has at most kStagingKept of them, which
+// are kept between calls; a call that finds them all taken goes without.  None
+// is left once the last handle is gone.
 constexpr int kStagingKept = 4;
 void staging_retain();   // a handle is made
 void staging_release();  // and destroyed

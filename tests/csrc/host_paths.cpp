@@ -2,12 +2,17 @@
 // staging.cpp) on a runtime in host memory (fake_hip.cpp): what happens to
 // device memory and streams where a GPU could only fault.  One scenario per
 // run, named by the first argument; prints "ok", or what went wrong.
+#include <chrono>
 #include <cstdio>
 #include <cstring>
+#include <future>
 #include <map>
+#include <memory>
 #include <string>
+#include <vector>
 
 #include "../../include/opensayal.h"
+#include "../../opensayal_amd/csrc/staging.hpp"
 #include "fake_hip.hpp"
 
 namespace {
@@ -324,6 +329,35 @@ void resident_says_what_runs() {
   osy_fluid_destroy(fl);
 }
 
+// Pinned buffers are made a few times per device and kept, however many callers
+// there are, and nobody waits while one is freed.
+void staging_is_bounded() {
+  using osy::StagingLease;
+  char host[16];
+  osy::staging_retain();
+  for (int round = 0; round < 3; round++) {
+    std::vector<std::unique_ptr<StagingLease>> at_once;
+    for (int i = 0; i < 7; i++) at_once.emplace_back(new StagingLease(0, host));
+    int have = 0;
+    for (auto& lease : at_once) have += *lease ? 1 : 0;
+    EXPECT(have == osy::kStagingKept);
+  }
+  EXPECT(fake::state().host_mallocs == osy::kStagingKept);
+  for (int round = 0; round < 3; round++)
+    for (int device = 1; device < 8; device++) EXPECT((bool)StagingLease(device, host));
+  EXPECT(fake::state().host_mallocs == osy::kStagingKept + 7);
+  EXPECT(fake::state().host_frees == 0);
+  std::vector<std::future<void>> others;
+  fake::state().on_host_free = [&] {
+    if (!others.empty()) return;
+    others.push_back(std::async(std::launch::async, [&host] { StagingLease lease(9, host); }));
+    EXPECT(others.back().wait_for(std::chrono::seconds(2)) == std::future_status::ready);
+  };
+  osy::staging_release();
+  others.clear();
+  EXPECT(fake::state().host_frees == fake::state().host_mallocs);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
@@ -335,6 +369,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_is_counted", exchange_is_counted},
     {"exchange_in_a_budget", exchange_in_a_budget},
     {"resident_says_what_runs", resident_says_what_runs},
+    {"staging_is_bounded", staging_is_bounded},
 };
 
 }  // namespace
