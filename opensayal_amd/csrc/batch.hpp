@@ -85,6 +85,15 @@ inline bool batch_occupancy_supported(int rows, int occupancy) {
   return (occupancy == 1 && rows == 8) || occupancy == 2;
 }
 
+// Whether that kernel has the division that pressure sums take for d_t = 0 or
+// |d_t| >= 2 (other members beside it still take the reciprocal).  24 members of
+// 128 to 384 wide with n = 50 take 309 us a step dividing at rows 12, 349 at
+// rows 8, and 2822 on graphs of their own, one after the other.  The division
+// costs the others nothing at rows 12 (265 us, 286 without it) and 1% at rows 8
+// uncapped (323 against 319), but 5% at rows 8 capped (516 against 490), where
+// registers are short; so a launch with dividing members is uncapped there.
+constexpr bool batch_divides(int rows, int occupancy) { return rows == 12 || occupancy == 1; }
+
 // Occupancy-derived workgroup count for the batch kernel of this storage /
 // pressure / rows combination.
 hipError_t batch_grid_size(int storage, bool pressure, int rows, int occupancy, int* grid);

@@ -81,7 +81,9 @@ __device__ inline bool wait_tiles(const unsigned long long* tdone, const unsigne
   return true;
 }
 
-template <typename T, bool PRESSURE, int R, int NW>
+// Pressure sums go through the double reciprocal of d_t, or divide where there
+// is none (pdt_recip).  DIVIDE false: the sums never divide.
+template <typename T, bool PRESSURE, bool DIVIDE, int R, int NW>
 __device__ __attribute__((always_inline)) inline void run_item(const BatchStage& st, const BatchSim& sim, int tile,
                                 unsigned epoch_bit, int tw, int th, int k, BatchShared<NW>& sh) {
   const StepParams& sp = sim.sp;
@@ -100,9 +102,17 @@ __device__ __attribute__((always_inline)) inline void run_item(const BatchStage&
     a.sweeps = st.sweeps;
     a.forces = st.forces;
     const int in = uv ^ (st.q & 1);
-    project_regs_tile<T, PRESSURE ? PM_RECIP : PM_NONE, R, NW>(sp, sim.gates, (const T*)sim.u[in],
-                                                 (const T*)sim.v[in], (T*)sim.u[in ^ 1],
-                                                 (T*)sim.v[in ^ 1], sim.p, a, tile, sh.reg);
+    const T *u = (const T*)sim.u[in], *v = (const T*)sim.v[in];
+    T *u_out = (T*)sim.u[in ^ 1], *v_out = (T*)sim.v[in ^ 1];
+    if constexpr (!PRESSURE)
+      project_regs_tile<T, PM_NONE, R, NW>(sp, sim.gates, u, v, u_out, v_out, sim.p, a, tile,
+                                           sh.reg);
+    else if (!DIVIDE || sp.pdt_recip != 0.0)
+      project_regs_tile<T, PM_RECIP, R, NW>(sp, sim.gates, u, v, u_out, v_out, sim.p, a, tile,
+                                            sh.reg);
+    else
+      project_regs_tile<T, PM_DIVIDE, R, NW>(sp, sim.gates, u, v, u_out, v_out, sim.p, a, tile,
+                                             sh.reg);
     return;
   }
   const int bx = tile % st.ntx, by = tile / st.ntx;
@@ -182,8 +192,8 @@ __global__ void __launch_bounds__(64 * NW, OCC2 ? 4 : 1) k_batch_step(BatchArgs 
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_ok)) {
       const int simi = __builtin_amdgcn_readfirstlane(st.sim);
-      run_item<T, PRESSURE, R, NW>(st, A.sims[simi], tile, (unsigned)(epoch & 1ULL), A.tw, A.th, A.k,
-                               sh);
+      run_item<T, PRESSURE, batch_divides(NW * R / 8, OCC2 ? 2 : 1), R, NW>(
+          st, A.sims[simi], tile, (unsigned)(epoch & 1ULL), A.tw, A.th, A.k, sh);
     }
     // every wavefront's stores have reached the L2 before the barrier; thread
     // 0's release then writes the L2 back once for the whole workgroup

@@ -358,6 +358,25 @@ void staging_is_bounded() {
   EXPECT(fake::state().host_frees == fake::state().host_mallocs);
 }
 
+// Members whose pressure sums divide (d_t = 0 or |d_t| >= 2) step in the
+// batch's launch like the others.
+void batch_division() {
+  osy_batch* b = nullptr;
+  EXPECT(osy_batch_create(0, &b) == OSY_OK);
+  std::vector<osy_fluid*> members;
+  for (const float d_t : {0.05f, 0.0f, 2.0f, -3.5f}) {
+    osy_config c = config(64, 36, 20, true);
+    c.d_t = d_t;
+    members.push_back(create(c));
+    EXPECT(osy_batch_add(b, members.back()) == OSY_OK);
+  }
+  EXPECT(osy_batch_step(b, 3) == OSY_OK);
+  EXPECT(fake::state().batch_launches == 3);
+  EXPECT(fake::state().launches.empty());
+  osy_batch_destroy(b);
+  for (osy_fluid* fl : members) osy_fluid_destroy(fl);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
@@ -370,6 +389,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_in_a_budget", exchange_in_a_budget},
     {"resident_says_what_runs", resident_says_what_runs},
     {"staging_is_bounded", staging_is_bounded},
+    {"batch_division", batch_division},
 };
 
 }  // namespace

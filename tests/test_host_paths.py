@@ -25,6 +25,7 @@ SCENARIOS = [
     "exchange_in_a_budget",
     "resident_says_what_runs",
     "staging_is_bounded",
+    "batch_division",
 ]
 
 
