@@ -85,6 +85,7 @@ struct osy_fluid {
   osy::Exchange exchange;  // made when a resident shape is first chosen
   std::vector<osy::Exchange> captured;  // other shapes' that graphs name
   ProjTuning tuning;  // projection kernel shape, chosen at create
+  bool tuned = false;  // or set, or autotuned, since
   long long spin_ticks = 0;  // bound of a resident projection's neighbour wait
   int cus = 0;               // CUs of the device
   int wall_khz = 100000;     // the device's wall-clock rate

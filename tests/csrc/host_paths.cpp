@@ -377,6 +377,26 @@ void batch_division() {
   for (osy_fluid* fl : members) osy_fluid_destroy(fl);
 }
 
+// The starting shape follows the sweeps a call asks for, not only those the
+// handle was made with; a chosen shape stays.
+void project_shape_follows_sweeps() {
+  osy_fluid *one = create(config(1920, 1080, 1)), *fifty = create(config(1920, 1080, 50));
+  EXPECT(osy_fluid_project(one, 50, nullptr) == OSY_OK);
+  EXPECT(osy_fluid_project(fifty, 50, nullptr) == OSY_OK);
+  EXPECT(osy_fluid_synchronize(one) == OSY_OK);
+  EXPECT(osy_fluid_synchronize(fifty) == OSY_OK);
+  const auto& did = fake::state().launches;
+  EXPECT(did.size() == 2 && did[0].tuning.k == did[1].tuning.k &&
+         did[0].tuning.th == did[1].tuning.th);
+  const osy_tuning chosen = shape(2, 8, 2);
+  EXPECT(osy_fluid_set_tuning(one, &chosen) == OSY_OK);
+  EXPECT(osy_fluid_project(one, 50, nullptr) == OSY_OK);
+  EXPECT(osy_fluid_synchronize(one) == OSY_OK);
+  EXPECT(did.back().tuning.k == 2);
+  osy_fluid_destroy(one);
+  osy_fluid_destroy(fifty);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
@@ -390,6 +410,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"resident_says_what_runs", resident_says_what_runs},
     {"staging_is_bounded", staging_is_bounded},
     {"batch_division", batch_division},
+    {"project_shape_follows_sweeps", project_shape_follows_sweeps},
 };
 
 }  // namespace

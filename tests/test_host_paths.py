@@ -26,6 +26,7 @@ SCENARIOS = [
     "resident_says_what_runs",
     "staging_is_bounded",
     "batch_division",
+    "project_shape_follows_sweeps",
 ]
 
 
