@@ -237,6 +237,14 @@ int drop_graphs(osy_fluid* fl) {
   return OSY_OK;
 }
 
+// Whether projections of shape t run as one launch (`run`) at the handle's d_t:
+// the resident kernel leaves out pressure sums that divide.
+bool one_launch(const osy_fluid* fl, const ProjTuning& t, ProjTuning* run) {
+  const bool divides =
+      fl->cfg.enable_pressure != 0 && fl->params(fl->cfg.d_t, nullptr).pdt_recip == 0.0;
+  return t.kernel == PROJ_RESIDENT && !divides && t.resident_plan(fl->W, fl->H, fl->cus, run);
+}
+
 size_t exchange_bytes(const osy_fluid* fl, const ProjTuning& run) {
   return 256 + 3 * 8 * run.exchange_words(fl->W, fl->H, (size_t)fl->elem);
 }
@@ -864,7 +872,7 @@ int osy::fluid_autotune(osy_fluid* fl, osy_tuning* chosen, double* ms, uint64_t 
       if (cand.kernel == PROJ_RESIDENT) {
         ProjTuning run;
         // (else it is the register candidate over again)
-        if (!cand.resident_plan(fl->W, fl->H, fl->cus, &run)) continue;
+        if (!one_launch(fl, cand, &run)) continue;
         if (exchange_bytes(fl, run) > exchange_limit) continue;
         if (fluid_reserve_exchange(fl, run, &trial) != OSY_OK) continue;  // no memory for it
         trial.bind(ft);
@@ -958,9 +966,8 @@ int osy_fluid_get_info(const osy_fluid* fl, osy_fluid_info* info) {
   info->pitch = fl->P;
   info->storage = fl->storage;
   ProjTuning run;
-  const bool per_stage =
-      fl->tuning.kernel == PROJ_RESIDENT &&
-      !(fl->exchange.mem && fl->tuning.resident_plan(fl->W, fl->H, fl->cus, &run));
+  const bool per_stage = fl->tuning.kernel == PROJ_RESIDENT &&
+                         !(fl->exchange.mem && one_launch(fl, fl->tuning, &run));
   info->projection_kernel = per_stage ? PROJ_REGS : fl->tuning.kernel;
   info->sweeps_per_launch = fl->tuning.kernel == PROJ_COLOUR ? 1 : fl->tuning.k;
   info->device_bytes = fluid_device_bytes(fl);
