@@ -129,7 +129,7 @@ typedef struct osy_fluid_info {
                                    one launch.  What runs: 2 when a resident
                                    shape was chosen that runs as a launch
                                    per stage                               */
-  int32_t sweeps_per_launch; /* sweeps one projection launch runs          */
+  int32_t sweeps_per_launch; /* sweeps one projection launch of a step runs */
   size_t device_bytes;  /* device memory held by this handle: its fields, and
                            the halo exchange of a resident projection       */
 } osy_fluid_info;
@@ -233,6 +233,10 @@ int osy_fluid_synchronize(osy_fluid* fluid);
  * handle's stream) without waiting.  For timing and testing the dominant
  * phase by itself. */
 int osy_fluid_project(osy_fluid* fluid, int32_t sweeps, void* hip_stream);
+/* Projection kernel launches that call makes (until a shape is set or
+ * autotuned, its shape follows `sweeps`, not only the configuration's n). */
+int osy_fluid_project_launches(const osy_fluid* fluid, int32_t sweeps,
+                               int32_t* launches);
 
 /* Copy a field to / from host memory in the reference's indx order.
  * `bytes` must equal W*H*4.  IS_SOLID and TOTAL_S are read-only. */

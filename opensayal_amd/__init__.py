@@ -195,12 +195,9 @@ class Fluid:
 
     def launches_per_call(self, sweeps: int) -> int:
         """Projection kernel launches one ``project(sweeps)`` call makes."""
-        if self.projection_kernel == 0:
-            return 2 * sweeps
-        if self.projection_kernel == 3:
-            return 1 if sweeps > 0 else 0
-        k = self.sweeps_per_launch
-        return -(-sweeps // k)
+        launches = ctypes.c_int32()
+        check(lib().osy_fluid_project_launches(self._h, sweeps, ctypes.byref(launches)))
+        return launches.value
 
     @classmethod
     def from_json(cls, path: str) -> "Fluid":

@@ -123,6 +123,8 @@ PROTOTYPES = {
     "osy_fluid_step_async": (ctypes.c_int, [ctypes.c_void_p, _i32, _f32, ctypes.c_void_p]),
     "osy_fluid_synchronize": (ctypes.c_int, [ctypes.c_void_p]),
     "osy_fluid_project": (ctypes.c_int, [ctypes.c_void_p, _i32, ctypes.c_void_p]),
+    "osy_fluid_project_launches": (ctypes.c_int, [ctypes.c_void_p, _i32,
+                                                  ctypes.POINTER(_i32)]),
     "osy_fluid_get_field": (ctypes.c_int, [ctypes.c_void_p, _i32, ctypes.c_void_p, ctypes.c_size_t]),
     "osy_fluid_set_field": (ctypes.c_int, [ctypes.c_void_p, _i32, ctypes.c_void_p, ctypes.c_size_t]),
     "osy_fluid_pressure_range": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(_f32), ctypes.POINTER(_f32)]),

@@ -245,6 +245,15 @@ bool one_launch(const osy_fluid* fl, const ProjTuning& t, ProjTuning* run) {
   return t.kernel == PROJ_RESIDENT && !divides && t.resident_plan(fl->W, fl->H, fl->cus, run);
 }
 
+// The shape in which osy_fluid_project runs `sweeps`: the chosen one, or the
+// starting shape for these sweeps (50 sweeps of 1920 x 1080 in the shape of a
+// handle with n = 1 take 468 us, a sweep per launch, 138 us in their own).
+ProjTuning project_shape(const osy_fluid* fl, int sweeps) {
+  return fl->tuned ? fl->tuning
+                   : default_tuning(fl->W, fl->H, sweeps, fl->cfg.enable_pressure != 0,
+                                    fl->storage, fl->cus);
+}
+
 size_t exchange_bytes(const osy_fluid* fl, const ProjTuning& run) {
   return 256 + 3 * 8 * run.exchange_words(fl->W, fl->H, (size_t)fl->elem);
 }
@@ -574,13 +583,22 @@ int osy_fluid_project(osy_fluid* fl, int32_t sweeps, void* hip_stream) {
   StepParams sp = fl->params(fl->cfg.d_t, nullptr);
   sp.n = sweeps;
   if (int st = before_projection(fl, s)) return st;
-  // the starting shape for these sweeps: 50 sweeps of 1920 x 1080 in the shape of
-  // a handle with n = 1 take 468 us (a sweep per launch), 138 us in their own
-  const ProjTuning t = fl->tuned ? fl->tuning
-                                 : default_tuning(fl->W, fl->H, sweeps, sp.pressure_on != 0,
-                                                  fl->storage, fl->cus);
-  enqueue_projection_only(fl->storage, sp, fl->f, &fl->uv, t, s);
+  enqueue_projection_only(fl->storage, sp, fl->f, &fl->uv, project_shape(fl, sweeps), s);
   OSY_HIP_CHECK(hipGetLastError());
+  return OSY_OK;
+}
+
+int osy_fluid_project_launches(const osy_fluid* fl, int32_t sweeps, int32_t* launches) {
+  if (!fl || !launches) return set_error(OSY_E_INVALID, "null argument");
+  if (sweeps < 0) return set_error(OSY_E_INVALID, "sweeps must be >= 0");
+  const ProjTuning t = project_shape(fl, sweeps);
+  ProjTuning run;
+  if (t.kernel == PROJ_COLOUR)
+    *launches = 2 * sweeps;
+  else if (fl->exchange.mem && one_launch(fl, t, &run))
+    *launches = sweeps > 0 ? 1 : 0;
+  else
+    *launches = (int32_t)(((int64_t)sweeps + t.k - 1) / t.k);
   return OSY_OK;
 }
 

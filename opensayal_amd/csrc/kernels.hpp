@@ -130,11 +130,6 @@ struct ProjTuning {
     return kernel == PROJ_TILED && k >= 1 && k <= 64 && tw >= 2 && th >= 1 && tw % 2 == 0 &&
            pw() <= 64 * kTileWaves && lds_bytes(pressure) <= kLdsLimit;
   }
-  // projection launches for `sweeps` sweeps
-  int launches(int sweeps) const {
-    if (kernel == PROJ_RESIDENT) return sweeps > 0 ? 1 : 0;
-    return kernel == PROJ_COLOUR ? 2 * sweeps : (sweeps + k - 1) / k;
-  }
   // register kernels: tiles over a W x H grid (the first and last of a row
   // or column own 2k cells more, RegPlace)
   int tiles_x(int W) const { return W <= 4 * k + tw ? 1 : (W - 4 * k + tw - 1) / tw; }

@@ -425,6 +425,34 @@ void project_shape_follows_sweeps() {
   osy_fluid_destroy(fifty);
 }
 
+// The launches a projection is said to make are those it makes: starting and
+// chosen shapes, one launch or one per stage.
+void launches_are_counted() {
+  const osy_tuning starting = shape(-1, 0, 0);
+  for (const osy_tuning& t : {starting, shape(2, 8, 2), shape(3, 12, 5), shape(3, 8, 4)}) {
+    for (const float d_t : {0.05f, 2.0f}) {
+      osy_config c = config(640, 480, 1, t.sweeps_per_launch != 5);  // (sums: up to 64 rows)
+      c.d_t = d_t;
+      osy_fluid* fl = create(c);
+      if (t.projection_kernel >= 0) EXPECT(osy_fluid_set_tuning(fl, &t) == OSY_OK);
+      for (const int sweeps : {0, 1, 7, 50}) {
+        int32_t said = -1;
+        EXPECT(osy_fluid_project_launches(fl, sweeps, &said) == OSY_OK);
+        EXPECT(osy_fluid_project(fl, sweeps, nullptr) == OSY_OK);
+        EXPECT(osy_fluid_synchronize(fl) == OSY_OK);
+        if (sweeps == 0) {
+          EXPECT(said == 0);
+          continue;
+        }
+        const fake::Launch& did = fake::state().launches.back();
+        const int k = did.tuning.k;
+        EXPECT(did.sweeps == sweeps && said == (did.resident ? 1 : (sweeps + k - 1) / k));
+      }
+      osy_fluid_destroy(fl);
+    }
+  }
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_out_of_memory", exchange_out_of_memory},
     {"autotune_fails", autotune_fails},
@@ -440,6 +468,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"staging_is_bounded", staging_is_bounded},
     {"batch_division", batch_division},
     {"project_shape_follows_sweeps", project_shape_follows_sweeps},
+    {"launches_are_counted", launches_are_counted},
 };
 
 }  // namespace

@@ -28,6 +28,7 @@ SCENARIOS = [
     "staging_is_bounded",
     "batch_division",
     "project_shape_follows_sweeps",
+    "launches_are_counted",
 ]
 
 
