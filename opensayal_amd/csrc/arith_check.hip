@@ -12,6 +12,7 @@
 
 #include "fluid_device.hpp"
 #include "fluid_internal.hpp"
+#include "projection_device.hpp"
 
 #pragma clang fp contract(off)
 
@@ -79,7 +80,7 @@ __global__ void __launch_bounds__(kCheckThreads)
       // the pressure sums' quotient x / d_t as a double multiply by the
       // double nearest 1 / d_t, for the step sizes 0.05 and 1/60
       const float b = mode == 5 ? 0.05f : 1.0f / 60.0f;
-      const float q1 = (float)((double)x * (1.0 / (double)b));
+      const float q1 = recip_quotient(x, 1.0 / (double)b);
       bad = __float_as_uint(q1) != __float_as_uint(div_ieee(x, b));
     } else if (mode == 3 || mode == 4) {
       // rnd2 (one packed conversion) against rnd (one scalar conversion per

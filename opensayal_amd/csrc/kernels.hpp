@@ -41,12 +41,12 @@ struct StepParams {
   // and the divisor 1 + 4a, both in float as the reference computes them
   int visc_on;
   float visc_a, visc_den;
-  double visc_recip;  // 1 / visc_den for 0 < |visc_den| < 2, else 0 (PressureDivisor)
+  double visc_recip;  // 1 / visc_den for 0 < |visc_den| < 2, else 0 (recip_quotient)
   // set by the step: the first projection launch applies the velocity
   // forces to what it loads and starts the pressure sums at 0
   int forces_in_projection;
   // 1.0 / (double)d_t when 0 < |d_t| < 2, else 0: the pressure sums'
-  // division by d_t as a double multiply (PressureDivisor)
+  // division by d_t as a double multiply (recip_quotient)
   double pdt_recip;
   // bound of one neighbour wait of the resident projection (wall-clock ticks)
   long long spin_ticks;

@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(64 * kAdvNY)
 // barrier per round; the rows inside are computed first, which hides that.
 // What bounds it is the issue of vector instructions, so the quotient goes
 // through the double reciprocal of the divisor where that is exact
-// (PressureDivisor), and only wavefronts that hold border cells select.
+// (recip_quotient), and only wavefronts that hold border cells select.
 // 50 rounds of 1920 x 1080 take 78 us (5 launches of 15.6 us); with the region
 // in LDS they took 175 us (9 launches of 19.4 us: six reads and writes of LDS
 // and a division per cell and round).
@@ -254,7 +254,7 @@ struct DiffShared {
 template <typename T, bool RECIP>
 __device__ inline float diffused(float x, float sum, float a, float den, double recip) {
   const float y = x + a * sum;
-  return rnd<T>(RECIP ? (float)((double)y * recip) : y / den);
+  return rnd<T>(RECIP ? recip_quotient(y, recip) : y / den);
 }
 
 // One round of a wavefront's rows.  EDGE: cells outside `cols0`, `cols1`

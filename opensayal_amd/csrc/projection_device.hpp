@@ -101,9 +101,6 @@ __device__ inline float lane_from_right(float x) {  // lane l gets lane l+1's x 
 __device__ inline float lane_from_left(float x) {  // lane l gets lane l-1's x (0 for lane 0)
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
 }
-__device__ inline uint32_t lane_from_right_u(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x130, 0xf, 0xf, true);
-}
 __device__ inline uint32_t lane_from_left_u(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x138, 0xf, 0xf, true);
 }
@@ -185,18 +182,15 @@ struct PressureDivisor {
   double recip;
 };
 
-// update_pressure_at (src/fluid.cu:221-227): ((d * density) * cell_size) / d_t.
-// With recip set the quotient is (float)(x * recip) in double, which is the
-// IEEE float quotient x / d_t for every binary32 x: the double is within
-// 2^-52 of x / d_t; a quotient of two binary32 numbers lies at least 2^-49
-// of itself from every binary32 rounding midpoint in the normal range, and
-// in the subnormal range it can only equal a midpoint if the divisor's
-// lowest set bit weighs 2 or more, which |d_t| < 2 excludes.  (Exhaustive
-// device check for d_t = 0.05 and 1/60: osy_arith_check, modes 5 and 6.)
-__device__ inline float pressure_term(float d, float density, float csf,
-                                      const PressureDivisor& pd) {
-  const float x = (d * density) * csf;
-  return pd.recip != 0.0 ? (float)((double)x * pd.recip) : x / pd.d_t;
+// x / b for 0 < |b| < 2 with recip the double nearest 1 / b: the IEEE float
+// quotient for every binary32 x.  The double is within 2^-52 of x / b; a
+// quotient of two binary32 numbers lies at least 2^-49 of itself from every
+// binary32 rounding midpoint in the normal range, and in the subnormal range
+// it can only equal a midpoint if the divisor's lowest set bit weighs 2 or
+// more, which |b| < 2 excludes.  (Exhaustive device check for b = 0.05 and
+// 1/60: osy_arith_check, modes 5 and 6.)
+__device__ inline float recip_quotient(float x, double recip) {
+  return (float)((double)x * recip);
 }
 
 // How a kernel adds the pressure sums: not at all; through the double
@@ -211,10 +205,11 @@ struct SweepParams {
               // region (128 or more) in all but the last tiles of a row
 };
 
+// update_pressure_at (src/fluid.cu:221-227): p + ((d * density) * cell_size) / d_t.
 template <int PM>
 __device__ inline float pressure_add(float p, float d, const SweepParams& q) {
-  if constexpr (PM == PM_UNIT) return p + (float)((double)d * q.pd.recip);
-  if constexpr (PM == PM_RECIP) return p + (float)((double)((d * q.density) * q.csf) * q.pd.recip);
+  if constexpr (PM == PM_UNIT) return p + recip_quotient(d, q.pd.recip);
+  if constexpr (PM == PM_RECIP) return p + recip_quotient((d * q.density) * q.csf, q.pd.recip);
   if constexpr (PM == PM_DIVIDE) return p + ((d * q.density) * q.csf) / q.pd.d_t;
   return p;
 }
@@ -269,7 +264,8 @@ __device__ inline bool in_lanes(unsigned long long m) {
 
 // div / s with y = 1 / s rounded: third_quotient's correction, which for
 // s = 1, 2, 4 adds the (exact) remainder of a quotient that is already
-// rounded, so nothing.  With s = y = 0 it gives div * 0.
+// rounded, so nothing.  With s = y = 0 it gives div * 0.  (Every s and binary32
+// div against IEEE division: tests/test_any_quotient.py.)
 __device__ inline float any_quotient(float div, float y, float s) {
   const float q0 = div * y;
   const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, s, div), y, q0);
