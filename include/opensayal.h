@@ -144,9 +144,8 @@ typedef struct osy_tuning {
                                 tile's workgroup must fit on the device at
                                 once, and both tile sides be >= 2 x k).
                                 Regions of 64 rows and more are run as ones
-                                of 96; where those do not fit, and with
-                                pressure sums for d_t = 0 or |d_t| >= 2, as
-                                a launch per stage of kernel 2            */
+                                of 96; where those do not fit, as a launch
+                                per stage of kernel 2                      */
   int32_t tile_width;        /* tiled: cells a workgroup owns along i (even) */
   int32_t tile_height;       /* tiled: cells a workgroup owns along j       */
   int32_t sweeps_per_launch; /* tiled: sweeps per launch (halo = 2x this);

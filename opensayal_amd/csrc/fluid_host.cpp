@@ -237,12 +237,9 @@ int drop_graphs(osy_fluid* fl) {
   return OSY_OK;
 }
 
-// Whether projections of shape t run as one launch (`run`) at the handle's d_t:
-// the resident kernel leaves out pressure sums that divide.
+// Whether projections of shape t run as one launch (`run`).
 bool one_launch(const osy_fluid* fl, const ProjTuning& t, ProjTuning* run) {
-  const bool divides =
-      fl->cfg.enable_pressure != 0 && fl->params(fl->cfg.d_t, nullptr).pdt_recip == 0.0;
-  return t.kernel == PROJ_RESIDENT && !divides && t.resident_plan(fl->W, fl->H, fl->cus, run);
+  return t.kernel == PROJ_RESIDENT && t.resident_plan(fl->W, fl->H, fl->cus, run);
 }
 
 // The shape in which osy_fluid_project runs `sweeps`: the chosen one, or the
@@ -342,8 +339,7 @@ int enqueue_graph_steps(osy_fluid* fl, int32_t steps, float d_t, hipStream_t s) 
 int adopt_tuning(osy_fluid* fl, const ProjTuning& t) {
   ProjTuning run;
   Exchange& x = fl->exchange;
-  if (t.kernel == PROJ_RESIDENT && t.resident_plan(fl->W, fl->H, fl->cus, &run) &&
-      !x.serves(run)) {
+  if (one_launch(fl, t, &run) && !x.serves(run)) {
     auto kept = std::find_if(fl->captured.begin(), fl->captured.end(),
                              [&](const Exchange& c) { return c.serves(run); });
     if (kept != fl->captured.end()) {

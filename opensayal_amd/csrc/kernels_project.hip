@@ -472,8 +472,6 @@ template <typename T>
 void enqueue_projection(const StepParams& sp, const GridView& g, const FieldPtrs& f, int* cur,
                         const ProjTuning& t, hipStream_t s) {
   if ((t.kernel == PROJ_RESIDENT || t.kernel == PROJ_REGS) && t.valid(sp.pressure_on)) {
-    // (pressure sums that need a division, d_t = 0 or |d_t| >= 2, always run
-    // a launch per stage)
     ProjTuning run;
     const bool resident = t.kernel == PROJ_RESIDENT && f.exchange &&
                           t.resident_plan(sp.W, sp.H, sp.cus, &run);
@@ -481,7 +479,8 @@ void enqueue_projection(const StepParams& sp, const GridView& g, const FieldPtrs
       resident ? launch_resident<T, PM_NONE>(sp, f, cur, run, s)
                : launch_regs<T, PM_NONE>(sp, f, cur, t, s);
     } else if (sp.pdt_recip == 0.0) {
-      launch_regs<T, PM_DIVIDE>(sp, f, cur, t, s);
+      resident ? launch_resident<T, PM_DIVIDE>(sp, f, cur, run, s)
+               : launch_regs<T, PM_DIVIDE>(sp, f, cur, t, s);
     } else if (sp.density == 1.0f && sp.cs == 1) {
       resident ? launch_resident<T, PM_UNIT>(sp, f, cur, run, s)
                : launch_regs<T, PM_UNIT>(sp, f, cur, t, s);

@@ -95,8 +95,7 @@ void project(const StepParams& sp, const FieldPtrs& f, const ProjTuning& t, size
   if (sp.n <= 0) return;
   ProjTuning run;
   const bool resident = t.kernel == PROJ_RESIDENT && f.exchange &&
-                        t.resident_plan(sp.W, sp.H, sp.cus, &run) &&
-                        !(sp.pressure_on && sp.pdt_recip == 0.0);
+                        t.resident_plan(sp.W, sp.H, sp.cus, &run);
   auto& st = fake::state();
   if (!resident) {
     push(s, [=, &st] {

@@ -329,30 +329,21 @@ void resident_says_what_runs() {
   osy_fluid_destroy(fl);
 }
 
-// So does one whose pressure sums divide (d_t = 0 or |d_t| >= 2), and the
-// autotuner does not take it for a resident one.
-void dividing_says_what_runs() {
+// One whose pressure sums divide (d_t = 0 or |d_t| >= 2) is resident like the
+// others.
+void dividing_is_resident() {
   for (const float d_t : {0.05f, 0.0f, 2.0f, -3.5f}) {
-    const bool divides = d_t != 0.05f;
     osy_config c = config(250, 230, 20, true);
     c.d_t = d_t;
     osy_fluid* fl = create(c);
     const osy_tuning asked = shape(3, 8, 5);
     osy_fluid_info info;
-    osy_tuning best;
     EXPECT(osy_fluid_set_tuning(fl, &asked) == OSY_OK);
     EXPECT(osy_fluid_project(fl, 20, nullptr) == OSY_OK);
     EXPECT(osy_fluid_synchronize(fl) == OSY_OK);
-    EXPECT(fake::state().launches.back().resident == !divides);
+    EXPECT(fake::state().launches.back().resident);
     EXPECT(osy_fluid_get_info(fl, &info) == OSY_OK);
-    EXPECT(info.projection_kernel == (divides ? 2 : 3));
-    fake::state().times_out = [&](const osy::ProjTuning&) {
-      EXPECT(!divides);  // no resident trial
-      return false;
-    };
-    EXPECT(osy_fluid_autotune(fl, &best, nullptr) == OSY_OK);
-    EXPECT(!divides || best.projection_kernel != 3);
-    fake::state().times_out = nullptr;
+    EXPECT(info.projection_kernel == 3);
     osy_fluid_destroy(fl);
   }
 }
@@ -464,7 +455,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"exchange_is_counted", exchange_is_counted},
     {"exchange_in_a_budget", exchange_in_a_budget},
     {"resident_says_what_runs", resident_says_what_runs},
-    {"dividing_says_what_runs", dividing_says_what_runs},
+    {"dividing_is_resident", dividing_is_resident},
     {"staging_is_bounded", staging_is_bounded},
     {"batch_division", batch_division},
     {"project_shape_follows_sweeps", project_shape_follows_sweeps},

@@ -24,7 +24,7 @@ SCENARIOS = [
     "exchange_is_counted",
     "exchange_in_a_budget",
     "resident_says_what_runs",
-    "dividing_says_what_runs",
+    "dividing_is_resident",
     "staging_is_bounded",
     "batch_division",
     "project_shape_follows_sweeps",
