@@ -157,7 +157,8 @@ typedef struct osy_fluid osy_fluid;
 /* Projection launch shape of a batch: register-tile rows per wavefront (8 or
  * 12; the tile is (128 - 4k) x (8 * rows - 4k) cells with a 2k-cell halo),
  * sweeps per tile k, and occupancy: 1 = the compiler's register allocation
- * (rows 8 only), 2 = registers capped for two workgroups per CU; 0 means 1. */
+ * (rows 8 only), 2 = registers capped for two workgroups per CU (but for rows
+ * 8 with pressure sums, where the cap only costs time); 0 means 1. */
 typedef struct osy_batch_tuning {
   int32_t rows;
   int32_t sweeps_per_tile;

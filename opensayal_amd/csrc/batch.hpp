@@ -79,20 +79,20 @@ struct BatchArgs {
 
 // Register-tile rows per wavefront supported by the batch kernel, and its
 // occupancy variants: 1 = registers as the compiler allocates them, 2 = capped
-// for two workgroups per CU (rows 8 both ways, rows 12 only capped).
+// for two workgroups per CU (rows 8 both ways, rows 12 only capped; batch_capped).
 inline bool batch_rows_supported(int rows) { return rows == 8 || rows == 12; }
 inline bool batch_occupancy_supported(int rows, int occupancy) {
   return (occupancy == 1 && rows == 8) || occupancy == 2;
 }
 
-// Whether that kernel has the division that pressure sums take for d_t = 0 or
-// |d_t| >= 2 (other members beside it still take the reciprocal).  24 members of
-// 128 to 384 wide with n = 50 take 309 us a step dividing at rows 12, 349 at
-// rows 8, and 2822 on graphs of their own, one after the other.  The division
-// costs the others nothing at rows 12 (265 us, 286 without it) and 1% at rows 8
-// uncapped (323 against 319), but 5% at rows 8 capped (516 against 490), where
-// registers are short; so a launch with dividing members is uncapped there.
-constexpr bool batch_divides(int rows, int occupancy) { return rows == 12 || occupancy == 1; }
+// Whether occupancy 2 caps the registers of that kernel.  Not at 8 rows with
+// pressure sums, where the cap spills 60 to 80 values per tile and both
+// occupancies are the same kernel: with 24 members of 128 to 384 wide, n = 50,
+// k = 6, a step took 463 us capped and takes 311 (60 of 64 to 256 wide: 477 and
+// 357; 8 of 640x360: 583 and 448).
+constexpr bool batch_capped(bool pressure, int rows, bool occupancy2) {
+  return occupancy2 && !(pressure && rows == 8);
+}
 
 // Occupancy-derived workgroup count for the batch kernel of this storage /
 // pressure / rows combination.

@@ -32,7 +32,6 @@ struct osy_batch {
   struct Group {
     int storage = 0;
     bool pressure = false;
-    int occupancy = 1;  // the batch's, or 1 where only that kernel divides
     BatchArgs args{};
     std::vector<int> member;  // indices into members
     std::vector<int> flip_uv, flip_sm;
@@ -141,13 +140,9 @@ int rebuild(osy_batch* b) {
       b->groups.emplace_back();
       b->groups.back().storage = fl->storage;
       b->groups.back().pressure = pressure;
-      b->groups.back().occupancy = b->occupancy;
       it = b->groups.end() - 1;
     }
     it->member.push_back((int)m);
-    if (pressure && fl->params(fl->cfg.d_t, nullptr).pdt_recip == 0.0 &&
-        !batch_divides(rows, b->occupancy))
-      it->occupancy = 1;
   }
 
   struct Tables {
@@ -299,7 +294,7 @@ int rebuild(osy_batch* b) {
     a.tw = tw;
     a.th = th;
     a.k = k;
-    OSY_HIP_CHECK(batch_grid_size(g.storage, g.pressure, rows, g.occupancy, &a.grid));
+    OSY_HIP_CHECK(batch_grid_size(g.storage, g.pressure, rows, b->occupancy, &a.grid));
   }
   OSY_HIP_CHECK(hipStreamSynchronize(b->stream));
 
@@ -311,7 +306,7 @@ int rebuild(osy_batch* b) {
   hipGraph_t graph = nullptr;
   OSY_HIP_CHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   for (const osy_batch::Group& g : b->groups)
-    enqueue_batch_step(g.storage, g.pressure, rows, g.occupancy, g.args, b->stream);
+    enqueue_batch_step(g.storage, g.pressure, rows, b->occupancy, g.args, b->stream);
   hipError_t le = hipGetLastError();
   hipError_t ce = hipStreamEndCapture(b->stream, &graph);
   if (le != hipSuccess || ce != hipSuccess) {

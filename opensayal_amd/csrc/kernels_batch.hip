@@ -82,8 +82,10 @@ __device__ inline bool wait_tiles(const unsigned long long* tdone, const unsigne
 }
 
 // Pressure sums go through the double reciprocal of d_t, or divide where there
-// is none (pdt_recip).  DIVIDE false: the sums never divide.
-template <typename T, bool PRESSURE, bool DIVIDE, int R, int NW>
+// is none (pdt_recip): chosen by member, which costs the others nothing at rows
+// 12 and 1% at rows 8 (24 members of 128 to 384 wide with n = 50 take 309 us a
+// step dividing at rows 12, 349 at rows 8, 2822 on graphs of their own).
+template <typename T, bool PRESSURE, int R, int NW>
 __device__ __attribute__((always_inline)) inline void run_item(const BatchStage& st, const BatchSim& sim, int tile,
                                 unsigned epoch_bit, int tw, int th, int k, BatchShared<NW>& sh) {
   const StepParams& sp = sim.sp;
@@ -107,7 +109,7 @@ __device__ __attribute__((always_inline)) inline void run_item(const BatchStage&
     if constexpr (!PRESSURE)
       project_regs_tile<T, PM_NONE, R, NW>(sp, sim.gates, u, v, u_out, v_out, sim.p, a, tile,
                                            sh.reg);
-    else if (!DIVIDE || sp.pdt_recip != 0.0)
+    else if (sp.pdt_recip != 0.0)
       project_regs_tile<T, PM_RECIP, R, NW>(sp, sim.gates, u, v, u_out, v_out, sim.p, a, tile,
                                             sh.reg);
     else
@@ -152,9 +154,11 @@ __device__ __attribute__((always_inline)) inline void run_item(const BatchStage&
 // loop that thread 0 leaves, which deadlocks the other threads.)
 // A region of 8 wavefronts of 8 rows (rows 8) or 16 of 6 (rows 12).  OCC2:
 // registers capped at 128, for sixteen wavefronts per CU (two workgroups of
-// eight, or one of sixteen); the batch autotuner decides whether that pays.
+// eight, or one of sixteen), where batch_capped says so; the batch autotuner
+// decides whether that pays.
 template <typename T, bool PRESSURE, int R, int NW, bool OCC2>
-__global__ void __launch_bounds__(64 * NW, OCC2 ? 4 : 1) k_batch_step(BatchArgs A) {
+__global__ void __launch_bounds__(64 * NW, batch_capped(PRESSURE, NW * R / 8, OCC2) ? 4 : 1)
+    k_batch_step(BatchArgs A) {
   __shared__ BatchShared<NW> sh;
   __shared__ unsigned long long s_claim;
   __shared__ int s_ok;
@@ -192,8 +196,8 @@ __global__ void __launch_bounds__(64 * NW, OCC2 ? 4 : 1) k_batch_step(BatchArgs 
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_ok)) {
       const int simi = __builtin_amdgcn_readfirstlane(st.sim);
-      run_item<T, PRESSURE, batch_divides(NW * R / 8, OCC2 ? 2 : 1), R, NW>(
-          st, A.sims[simi], tile, (unsigned)(epoch & 1ULL), A.tw, A.th, A.k, sh);
+      run_item<T, PRESSURE, R, NW>(st, A.sims[simi], tile, (unsigned)(epoch & 1ULL), A.tw, A.th, A.k,
+                               sh);
     }
     // every wavefront's stores have reached the L2 before the barrier; thread
     // 0's release then writes the L2 back once for the whole workgroup
