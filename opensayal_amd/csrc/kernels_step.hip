@@ -171,7 +171,10 @@ __global__ void __launch_bounds__(kMinmaxThreads)
         (unsigned long long)__float_as_uint(hi) << 32 | __float_as_uint(lo);
     __hip_atomic_store(&part[blockIdx.x], both, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // the word has reached the other XCDs before the count; an ordering atomic
-    // would also write back and drop the whole L2
+    // would also write back and drop the whole L2.  (The fences on both sides
+    // keep the compiler from moving either atomic past the wait, which is what
+    // orders them on gfx950: tests/test_reduction_order.py.)
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
