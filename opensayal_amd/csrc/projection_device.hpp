@@ -402,12 +402,10 @@ struct RegShared {
 };
 
 // What a wavefront has read of its neighbours' rows after a phase and not
-// yet used: the update from below of its row 0, row 0 of the wavefront above,
-// and its own update of that row.
+// yet used: the update from below of its row 0, and row 0 of the wavefront above.
 struct RowExchange {
   float dd;
   float2 x;
-  float dtop;
 };
 
 // The update from below reaches row 0.  PB is the parity of row 0's active
@@ -444,11 +442,7 @@ __device__ __attribute__((always_inline)) inline void reg_rows(RegTile<R>& t, co
   reg_rows_from<T, R, PB, PM, KIND, 1, R - 2>(t, 0.0f, 0.0f, dtop, sq, lane);
   reg_settle<T, R, PB>(t, x);
   reg_row<T, R, PB, PM, KIND>(t, 0, 0.0f, 0.0f, dtop, sq, lane);
-  // row 0 of the wavefront above as that wavefront has it once it settles
-  constexpr bool odd = ((PB + R) & 1) != 0;
-  const float vt0 = odd ? x.x.x : rnd<T>(x.x.x - x.dtop);
-  const float vt1 = odd ? rnd<T>(x.x.y - x.dtop) : x.x.y;
-  reg_row<T, R, ((PB + R - 1) & 1), PM, KIND>(t, R - 1, vt0, vt1, dtop, sq, lane);
+  reg_row<T, R, ((PB + R - 1) & 1), PM, KIND>(t, R - 1, x.x.x, x.x.y, dtop, sq, lane);
 }
 
 // One colour phase.  PB is the parity of the active cell in row 0 of this
@@ -460,9 +454,9 @@ __device__ __attribute__((always_inline)) inline void reg_rows(RegTile<R>& t, co
 // computing (this phase's own updates, before the one from below) beside
 // dtop, the update its last row makes to the row above; after the barrier it
 // reads both its neighbours'.  In the next phase it applies the update from
-// below to its row 0, and the wavefront below applies the same update, with
-// the same rounding, to the copy it has read, which is then the row as the
-// wavefront above holds it.  The slots alternate between phases, so none is
+// below to its row 0.  The row above as it has been read lacks that update too,
+// but only in the cells that its own last row does not touch in that phase: those
+// of the other parity.  The slots alternate between phases, so none is
 // rewritten before every reader of its previous contents has passed the next
 // barrier.  reg_begin publishes and reads the rows as loaded.
 template <typename T, int R, int NW, int PB, int SLOT, int PM, int KIND, bool ACTIVE>
@@ -479,7 +473,6 @@ __device__ __attribute__((always_inline)) inline void reg_phase(RegTile<R>& t, R
   __syncthreads();
   x.dd = w > 0 ? sh.dsend[SLOT][w - 1][lane] : 0.0f;
   x.x = w < NW - 1 ? sh.vrow[SLOT][w + 1][lane] : make_float2(0.0f, 0.0f);
-  x.dtop = dtop;
 }
 
 // `pairs` pairs of phases.  A loop of its own for each kind keeps the rows in
@@ -669,7 +662,7 @@ __device__ __attribute__((always_inline)) inline RowExchange reg_begin(const Reg
                                                                        RegShared<NW>& sh, int w,
                                                                        int lane) {
   RowExchange x;
-  x.dd = x.dtop = 0.0f;
+  x.dd = 0.0f;
   if (w > 0) sh.vrow[0][w][lane] = make_float2(t.v0[0], t.v1[0]);
   __syncthreads();
   x.x = w < NW - 1 ? sh.vrow[0][w + 1][lane] : make_float2(0.0f, 0.0f);
