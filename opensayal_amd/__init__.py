@@ -384,6 +384,7 @@ class Batch:
     def add(self, fluid: Fluid) -> None:
         check(lib().osy_batch_add(self._h, fluid._h))
         self.members.append(fluid)
+        fluid._refresh_info()  # the budget may have taken its halo exchange
 
     def remove(self, fluid: Fluid) -> None:
         check(lib().osy_batch_remove(self._h, fluid._h))
@@ -414,6 +415,9 @@ class Batch:
         t = OsyBatchTuning()
         ms = ctypes.c_double()
         check(lib().osy_batch_autotune(self._h, ctypes.byref(t), ctypes.byref(ms)))
+        for fluid in self.members:  # those on their own graphs were tuned
+            if fluid._h:  # (not closed since)
+                fluid._refresh_info()
         return {"rows": t.rows, "sweeps_per_tile": t.sweeps_per_tile,
                 "occupancy": t.occupancy}, ms.value
 
