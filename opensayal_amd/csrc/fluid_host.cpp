@@ -104,7 +104,7 @@ BlockLayout block_layout(int W, int H, int storage) {
 // 162 us).  In 16 bits and with pressure sums, where a phase is dearer, two and
 // three tiles of 32 rows to a CU still win (1001 x 563, n = 100, in bfloat16:
 // 192 us against 205 us at 64 rows; 1280 x 720 with pressure: 135 us against
-// 145 us).  Pressure sums need too many registers for more than 64 rows; two
+// 145 us).  With pressure sums the kernels are built up to 64 rows only; two
 // such tiles run on a CU at once (1024 x 1024 with pressure: 145 us at k = 10,
 // 176 us at k = 5).  Larger grids are bound by the work and the memory of all
 // their tiles: 64 rows and k = 6, or 5 in 16 bits, where a row's rounding

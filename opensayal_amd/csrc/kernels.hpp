@@ -120,7 +120,8 @@ struct ProjTuning {
   bool valid(bool pressure) const {
     if (kernel == PROJ_COLOUR) return true;
     if (kernel == PROJ_REGS || kernel == PROJ_RESIDENT) {
-      // pressure sums need 2 more VGPRs per row: 16 rows spill
+      // with pressure sums (2 more VGPRs per row) only up to 64 rows are built; a
+      // resident shape of 64 runs as one of 96 (resident_plan)
       const bool regs = k >= 1 && k <= 28 && tw == 128 - 4 * k && th >= 1 &&
                         (th + 4 * k) % kRegWaves == 0 && reg_rows_supported(reg_rows()) &&
                         !(pressure && reg_rows() > 8);
@@ -160,9 +161,9 @@ constexpr int kReduceBlocks = 512;
 
 // Tiles that a resident shape may be asked to have: as many as workgroups of
 // its register kernel fit the device, from the launch bounds (which the
-// compiler meets): 8 wavefronts within 80 VGPRs at 4 rows (6 per SIMD: 3
-// workgroups per CU) and 128 at 8 and 10 rows (4: 2 workgroups); 16
-// wavefronts above (1).  LDS (12 KiB per 8 wavefronts) and the wavefront
+// compiler meets, by spilling where it has to): 8 wavefronts within 80 VGPRs at
+// 4 rows (6 per SIMD: 3 workgroups per CU) and 128 at 8 and 10 rows (4: 2
+// workgroups); 16 wavefronts above (1).  LDS (12 KiB per 8 wavefronts) and the wavefront
 // slots allow more.  (The runtime's occupancy query was not used: it has
 // returned 0 for a kernel that fits, depending on what ran before.)
 inline int resident_slots(int rows, int cus) { return (rows == 4 ? 3 : rows <= 10 ? 2 : 1) * cus; }

@@ -5,10 +5,15 @@
 // phase is a set of independent cell updates and any schedule that finishes
 // one phase before the next starts reproduces the reference bit for bit.
 //
-// Two kernels:
+// Four kernels.  A handle starts with k_project_regs (default_tuning); the
+// autotuner times all four, and any of them can be set.
+//  * k_project_regs: k sweeps per launch on a 128-cell wide region held in
+//    registers (projection_device.hpp).
+//  * k_project_resident: the same regions kept in registers for all n sweeps of
+//    one launch, with halos exchanged between the tiles every k sweeps.
 //  * k_project_colour: one launch per colour phase, in place (2n launches);
-//    the plain restatement, kept for tiny grids.
-//  * k_project_tiled: temporal blocking.  A workgroup loads its tile plus a
+//    the plain restatement.
+//  * k_project_tiled: temporal blocking in LDS.  A workgroup loads its tile plus a
 //    halo of u, v and cell flags into LDS, runs up to k sweeps there, and
 //    writes the tile to the other half of a ping-pong pair.  A colour phase
 //    changes only faces of the cells it updates, so a value can be wrong
@@ -247,7 +252,11 @@ __global__ void __launch_bounds__(kTileThreads)
 
 // Eight wavefronts hold 4, 8 or 10 rows each, sixteen hold taller regions
 // (reg_waves): so a CU always has four wavefronts per SIMD to hide latency
-// with (six at 4 rows), within 128 VGPRs (80 at 4 rows).
+// with (six at 4 rows), within 128 VGPRs (80 at 4 rows).  The compiler keeps to
+// that by spilling: 8 rows without sums 6 to 8 values, 10 rows 39, with sums
+// 8 rows 56 to 81 and 4 rows 13 to 17, nearly all of them at the load, the
+// classification and the store, none in the phases of binary32; the resident
+// kernels with sums 11 to 41, around the exchange of a stage as well.
 template <int R, int NW> constexpr int reg_waves_per_simd() { return R == 4 && NW == 8 ? 6 : 4; }
 
 template <typename T, int PM, int R, int NW>
