@@ -369,8 +369,7 @@ int adopt_tuning(osy_fluid* fl, const ProjTuning& t) {
 }
 
 // bytes of device memory to host memory, complete on return.
-int copy_back(osy_fluid* fl, void* dst, const void* src, size_t bytes) {
-  StagingLease pinned(fl->device, dst);
+int copy_back(osy_fluid* fl, StagingLease& pinned, void* dst, const void* src, size_t bytes) {
   if (pinned) {
     OSY_HIP_CHECK(pinned.copy_out(dst, src, bytes, fl->stream));
     return OSY_OK;
@@ -385,20 +384,18 @@ int copy_back(osy_fluid* fl, void* dst, const void* src, size_t bytes) {
 // handle's device staging buffer and copied from there.
 template <class Make>
 int copy_result(osy_fluid* fl, void* dst, size_t bytes, const Make& make) {
-  if (bytes <= kStagingDirect) {
-    StagingLease pinned(fl->device, dst);
-    if (pinned) {
-      make((float*)pinned.slot());
-      const hipError_t e = hipGetLastError();
-      OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
-      OSY_HIP_CHECK(e);
-      std::memcpy(dst, pinned.slot(), bytes);
-      return OSY_OK;
-    }
+  StagingLease pinned(fl->device, dst);
+  if (pinned.direct(bytes)) {
+    make((float*)pinned.slot());
+    const hipError_t e = hipGetLastError();
+    OSY_HIP_CHECK(hipStreamSynchronize(fl->stream));
+    OSY_HIP_CHECK(e);
+    std::memcpy(dst, pinned.slot(), bytes);
+    return OSY_OK;
   }
   make(fl->staging);
   OSY_HIP_CHECK(hipGetLastError());
-  return copy_back(fl, dst, fl->staging, bytes);
+  return copy_back(fl, pinned, dst, fl->staging, bytes);
 }
 
 int field_elem_ok(int field) { return field >= OSY_FIELD_VEL_X && field <= OSY_FIELD_TOTAL_S; }
@@ -621,7 +618,7 @@ int osy_fluid_set_field(osy_fluid* fl, int32_t field, const void* src, size_t by
   if (int st = batch_wait(fl)) return st;
   StagingLease pinned(fl->device, bytes <= kStagingDirect ? src : nullptr);
   float* from = fl->staging;
-  if (pinned)
+  if (pinned.direct(bytes))
     from = (float*)std::memcpy(pinned.slot(), src, bytes);
   else  // (the runtime brings larger fields over as fast)
     OSY_HIP_CHECK(hipMemcpyAsync(fl->staging, src, bytes, hipMemcpyHostToDevice, fl->stream));
@@ -696,8 +693,12 @@ int osy_fluid_traces(osy_fluid* fl, int32_t distance, int32_t length, float d_t,
   const StepParams sp = fl->params(d_t, nullptr);
   enqueue_traces(fl->storage, sp, fl->f, fl->uv, distance, length, d_t, dx, dy, fl->stream);
   OSY_HIP_CHECK(hipGetLastError());
-  if (int st = copy_back(fl, traces_x, dx, each)) return st;
-  return copy_back(fl, traces_y, dy, each);
+  {
+    StagingLease pinned(fl->device, traces_x);
+    if (int st = copy_back(fl, pinned, traces_x, dx, each)) return st;
+  }
+  StagingLease pinned(fl->device, traces_y);
+  return copy_back(fl, pinned, traces_y, dy, each);
 }
 
 int osy_fluid_divergence_norm(osy_fluid* fl, double* l2, double* linf) {

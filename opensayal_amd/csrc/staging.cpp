@@ -94,6 +94,7 @@ StagingLease::StagingLease(int device, const void* host) {
   Pool& pool = g_pools[device];
   {
     std::lock_guard<std::mutex> lock(g_mu);
+    alone_ = pool.made == pool.idle_count;
     if (pool.idle_count > 0) {
       st_ = pool.idle[--pool.idle_count];
       return;

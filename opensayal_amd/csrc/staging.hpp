@@ -18,8 +18,14 @@
 
 namespace osy {
 
-// up to here the layout kernels read and write a slot themselves
+// up to here the layout kernels read and write a slot themselves; between
+// kStagingShared and this only for a call that has the link to itself, since
+// kernels of several threads share it worse than copies do (4 threads, fields
+// of 1 MB in and out: 1550 us direct, 1290 through copies; one thread: 56 us in
+// and 58 out, 62 and 59).  Below kStagingShared the runtime's copies are so much
+// slower (0.52 MB in: 36 us, 236) that several threads lose nothing either.
 constexpr size_t kStagingDirect = 1u << 20;
+constexpr size_t kStagingShared = 1u << 19;
 constexpr size_t kStagingSlot = 1u << 20;
 constexpr int kStagingSlots = 4;
 
@@ -46,6 +52,10 @@ class StagingLease {
   StagingLease(const StagingLease&) = delete;
   StagingLease& operator=(const StagingLease&) = delete;
   explicit operator bool() const { return st_ != nullptr; }
+  // whether the layout kernels are to use the slot themselves
+  bool direct(size_t bytes) const {
+    return st_ && bytes <= (alone_ ? kStagingDirect : kStagingShared);
+  }
   char* slot(size_t i = 0) const { return st_->host + i % kStagingSlots * kStagingSlot; }
   // dst <- src (device), after what `s` holds; dst is complete on return.
   // On an error nothing is in flight.
@@ -53,6 +63,7 @@ class StagingLease {
 
  private:
   Staging* st_ = nullptr;
+  bool alone_ = false;  // no other call had a buffer of the device when this took it
 };
 
 }  // namespace osy

@@ -377,6 +377,23 @@ void staging_is_bounded() {
   EXPECT(fake::state().host_frees == fake::state().host_mallocs);
 }
 
+// The layout kernels use a slot for larger fields only in a call that has the
+// device's link to itself.
+void staging_shares_the_link() {
+  using osy::StagingLease;
+  char host[16];
+  osy::staging_retain();
+  for (int round = 0; round < 3; round++) {
+    StagingLease first(0, host);
+    EXPECT(first.direct(osy::kStagingDirect) && !first.direct(osy::kStagingDirect + 1));
+    StagingLease second(0, host), elsewhere(1, host);
+    EXPECT(second.direct(osy::kStagingShared) && !second.direct(osy::kStagingShared + 1));
+    EXPECT(elsewhere.direct(osy::kStagingDirect));
+  }
+  EXPECT(!StagingLease(0, nullptr).direct(4));  // no buffer
+  osy::staging_release();
+}
+
 // Members whose pressure sums divide (d_t = 0 or |d_t| >= 2) step in the
 // batch's launch like the others.
 void batch_division() {
@@ -457,6 +474,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"resident_says_what_runs", resident_says_what_runs},
     {"dividing_is_resident", dividing_is_resident},
     {"staging_is_bounded", staging_is_bounded},
+    {"staging_shares_the_link", staging_shares_the_link},
     {"batch_division", batch_division},
     {"project_shape_follows_sweeps", project_shape_follows_sweeps},
     {"launches_are_counted", launches_are_counted},

@@ -26,6 +26,7 @@ SCENARIOS = [
     "resident_says_what_runs",
     "dividing_is_resident",
     "staging_is_bounded",
+    "staging_shares_the_link",
     "batch_division",
     "project_shape_follows_sweeps",
     "launches_are_counted",
